@@ -844,7 +844,8 @@ template <bool PHS, class PRM, class COL, class CAN, class WRK, class PHA>
 __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, const PRM &P,
                              const double *__restrict__ pft, const COL &col, const CAN &S,
                              int i0, const int32_t *__restrict__ filter, double dtime, ErrWord *err, bool first,
-                             int budget, const WRK &W, const PHA &H, const SoilTerms *soil, double *rr_lane)
+                             int budget, const WRK &W, const PHA &H, const SoilTerms *soil, double *rr_lane,
+                             double *phs_lane)
 {
     const int p = filter ? filter[i0] : V.begp + i0;
     const long pp = V.p1(p);
@@ -1165,7 +1166,7 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
         if constexpr (PHS) {
             // sun and shade together; btran and the transpiration come from the hydraulics
             btran = photosynthesis_phs(V, sw, P, K, T, H, S, p, c, ivt, nrad, noon, forc_pbot, thm, svpts, eah, o2,
-                                       co2, rb, qsatl, qaf, sun, sha, sh, bad);
+                                       co2, rb, qsatl, qaf, sun, sha, sh, bad, phs_lane);
             S.btran[pp] = btran;
             qflx_tran_veg = S.qflx_tran_veg[pp];
         } else {
@@ -1578,11 +1579,12 @@ k_canopy_round(typename std::conditional<PHS, RoundArgsPhs, RoundArgs>::type arg
                              A->sw.light_inhibit, A->sw.itmax};
             if constexpr (PHS) {
                 const KARG RoundArgsPhs *B = (const KARG RoundArgsPhs *)A;
+                __shared__ double phs_soil[phs::SOIL_LDS * phs::SOIL_STRIDE];
                 cont = canopy_patch<true>(V, sw, A->P, A->pft, A->col, A->S, i0, A->filter, A->dtime, A->err,
-                                          first, A->budget, A->W, B->phs, soil, rr_lane);
+                                          first, A->budget, A->W, B->phs, soil, rr_lane, phs_soil + lane);
             } else {
                 cont = canopy_patch<false>(V, sw, A->P, A->pft, A->col, A->S, i0, A->filter, A->dtime, A->err,
-                                           first, A->budget, A->W, *A, soil, rr_lane);
+                                           first, A->budget, A->W, *A, soil, rr_lane, nullptr);
             }
         }
         const unsigned long long mask = __ballot(cont);

@@ -6,10 +6,13 @@
 //
 // The reference calls this once per iteration for the whole filter; here a
 // lane runs its patch's share, statement by statement in the reference's
-// order.  The solve's helpers are out-of-line functions (ci_func_phs has
-// five call sites in hybrid_phs / brent_phs and carries calcstress's Newton
-// iteration): one copy of each body.  The root-soil conductances of the
-// routine's first loop (:3062-3114) come from the conductance kernel run
+// order.  Everything is inlined, so the solve's state stays in registers (as
+// out-of-line functions its helpers passed it through scratch memory, 2 KB per
+// lane): the search for the two ci is one loop with one evaluation of
+// ci_func_PHS, and calcstress, which updates the stress factors between searches
+// and serves the night branch, has one site in the loop around it.  The soil
+// below the patch is in LDS (phs::stage_soil).  The root-soil conductances of
+// the routine's first loop (:3062-3114) come from the conductance kernel run
 // before the iteration, over the same inputs.
 #pragma once
 
@@ -38,7 +41,7 @@ struct PhsSolve {
     double pd[4], tran;
 };
 
-__device__ __noinline__ void phs_calcstress(PhsSolve &s, double *x, double &bsun, double &bsha, double gs_sun,
+__device__ __forceinline__ void phs_calcstress(PhsSolve &s, double *x, double &bsun, double &bsha, double gs_sun,
                                             double gs_sha)
 {
     double tran = 0.0;
@@ -52,13 +55,11 @@ __device__ __noinline__ void phs_calcstress(PhsSolve &s, double *x, double &bsun
     }
 }
 
-// ci_func_PHS (:4227-4486)
-__device__ __noinline__ void ci_func_phs(PhsSolve &s, double *x, double cisun, double cisha, double &fsun,
-                                         double &fsha, double &bsun, double &bsha, bool bflag, double gs0sun,
-                                         double gs0sha, double &gs_sun, double &gs_sha)
+// ci_func_PHS (:4227-4486) after its calcstress call
+__device__ __forceinline__ void ci_func_phs(PhsSolve &s, double cisun, double cisha, double &fsun, double &fsha,
+                                            double bsun, double bsha, double &gs_sun, double &gs_sha)
 {
     double r1, r2;
-    if (bflag) phs_calcstress(s, x, bsun, bsha, gs0sun, gs0sha);
     const double ci[2] = {cisun, cisha};
     const double b[2] = {bsun, bsha};
     if (s.c3) {
@@ -128,183 +129,187 @@ __device__ __noinline__ void ci_func_phs(PhsSolve &s, double *x, double cisun, d
     }
 }
 
-// brent_PHS (:4068-4223): both phases' brackets shrink together; tol is the
-// sunlit tolerance for both
-__device__ __noinline__ void brent_phs(PhsSolve &s, double &xsun, double x1sun, double x2sun, double f1sun,
-                                       double f2sun, double &xsha, double x1sha, double x2sha, double f1sha,
-                                       double f2sha, double tol, double &gs_sun, double &gs_sha, double &bsun,
-                                       double &bsha)
+// hybrid_PHS (:3815-4064) and its brent_PHS (:4068-4223): the outer loop updates
+// bsun / bsha through calcstress, the inner one is the secant / Brent search for
+// both ci (both phases' brackets shrink together; tolsun is the tolerance of
+// both).  The inner loop evaluates ci_func_PHS at the point the previous pass
+// chose, then the stage the lane is in (the two starting points, a secant step,
+// the evaluation at the best point, the Brent iteration) takes the result and
+// chooses the next point or ends the search: each lane makes the reference's
+// sequence of evaluations, and the lanes of a wave share them and, between
+// searches, calcstress.
+// night: calcstress at the minimum conductance gsmin instead (:3500-3548),
+// without a search.  vegwp (4) inout; returns soilflux clipped at 0.
+__device__ __forceinline__ double hybrid_phs(PhsSolve &s, bool night, double gsmin, double ci0, double *vegwp,
+                                             double &bsun, double &bsha, double &gs_sun, double &gs_sha)
 {
-    const int itmax = 20;
-    const double eps = 1.e-4;
-    double a[2] = {x1sun, x1sha}, b[2] = {x2sun, x2sha}, fa[2] = {f1sun, f1sha}, fb[2] = {f2sun, f2sha};
-    double c[2], fc[2], d[2] = {0.0, 0.0}, e[2] = {0.0, 0.0}, tol1[2], xm[2];
-    double dummy[4] = {0.0, 0.0, 0.0, 0.0};   // calcstress is not called from here (bflag false)
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-        if ((fa[k] > 0.0 && fb[k] > 0.0) || (fa[k] < 0.0 && fb[k] < 0.0)) {
-            s.bad = true;
-            xsun = b[PHS_SUN];
-            xsha = b[PHS_SHA];
-            return;
-        }
-    c[0] = b[0];
-    c[1] = b[1];
-    fc[0] = fb[0];
-    fc[1] = fb[1];
-    int iter = 0;
-    for (;;) {
-        if (iter == itmax) break;
-        iter = iter + 1;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if ((fb[k] > 0.0 && fc[k] > 0.0) || (fb[k] < 0.0 && fc[k] < 0.0)) {
-                c[k] = a[k];
-                fc[k] = fa[k];
-                d[k] = b[k] - a[k];
-                e[k] = d[k];
-            }
-            if (fabs(fc[k]) < fabs(fb[k])) {
-                a[k] = b[k];
-                b[k] = c[k];
-                c[k] = a[k];
-                fa[k] = fb[k];
-                fb[k] = fc[k];
-                fc[k] = fa[k];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) tol1[k] = 2.0 * eps * fabs(b[k]) + 0.5 * tol;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) xm[k] = 0.5 * (c[k] - b[k]);
-        if ((fabs(xm[PHS_SUN]) <= tol1[PHS_SUN] || fb[PHS_SUN] == 0.0) &&
-            (fabs(xm[PHS_SHA]) <= tol1[PHS_SHA] || fb[PHS_SHA] == 0.0)) {
-            xsun = b[PHS_SUN];
-            xsha = b[PHS_SHA];
-            return;
-        }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if (fabs(e[k]) >= tol1[k] && fabs(fa[k]) > fabs(fb[k])) {
-                const double ss = fb[k] / fa[k];
-                double p, q;
-                if (a[k] == c[k]) {
-                    p = 2.0 * xm[k] * ss;
-                    q = 1.0 - ss;
-                } else {
-                    q = fa[k] / fc[k];
-                    const double r = fb[k] / fc[k];
-                    p = ss * (2.0 * xm[k] * q * (q - r) - (b[k] - a[k]) * (r - 1.0));
-                    q = (q - 1.0) * (r - 1.0) * (ss - 1.0);
-                }
-                if (p > 0.0) q = -q;
-                p = fabs(p);
-                if (2.0 * p < fmin90(3.0 * xm[k] * q - fabs(tol1[k] * q), fabs(e[k] * q))) {
-                    e[k] = d[k];
-                    d[k] = p / q;
-                } else {
-                    d[k] = xm[k];
-                    e[k] = d[k];
-                }
-            } else {
-                d[k] = xm[k];
-                e[k] = d[k];
-            }
-            a[k] = b[k];
-            fa[k] = fb[k];
-            if (fabs(d[k]) > tol1[k]) b[k] = b[k] + d[k];
-            else b[k] = b[k] + copysign(fabs(tol1[k]), xm[k]);
-        }
-        const double gs0sun = gs_sun, gs0sha = gs_sha;
-        ci_func_phs(s, dummy, b[PHS_SUN], b[PHS_SHA], fb[PHS_SUN], fb[PHS_SHA], bsun, bsha, false, gs0sun, gs0sha,
-                    gs_sun, gs_sha);
-        if (fb[PHS_SUN] == 0.0 && fb[PHS_SHA] == 0.0) break;
-    }
-    xsun = b[PHS_SUN];
-    xsha = b[PHS_SHA];
-}
-
-// hybrid_PHS (:3815-4064): the outer loop updates bsun / bsha through
-// calcstress, the inner one is the secant / Brent search for both ci.
-// vegwp (4) inout; returns soilflux clipped at 0.
-__device__ __noinline__ double hybrid_phs(PhsSolve &s, double &x0sun, double &x0sha, double *vegwp, double &bsun,
-                                          double &bsha, double &gs_sun, double &gs_sha)
-{
-    const double toldb = 1.e-2, eps = 1.e-2, eps1 = 1.e-4;
-    const int itmax = 3;
+    const double toldb = 1.e-2, eps = 1.e-2, eps1 = 1.e-4, epsb = 1.e-4;
+    const int itmax = 3, itmaxb = 20;
+    enum { F_X0, F_X1, SECANT, BEST, BRENT };
     double x[4];
-    double x1sun = x0sun, x1sha = x0sha, f0sun = 0.0, f0sha = 0.0, f1sun = 0.0, f1sha = 0.0;
-    double minf = 0.0, minxsun = 0.0, minxsha = 0.0;
-    bool bflag = false;
-    double b0sun = -1.0, b0sha = -1.0, gs0sun = 0.0, gs0sha = 0.0;
-    bsun = 1.0;
-    bsha = 1.0;
+    double x0[2], x1[2] = {ci0, ci0}, f0[2] = {0.0, 0.0}, f1[2] = {0.0, 0.0};
+    double minf = 0.0, minx[2] = {0.0, 0.0}, tol[2];
+    double b0sun = -1.0, b0sha = -1.0, gs0sun = night ? gsmin : 0.0, gs0sha = night ? gsmin : 0.0;
+    bool bflag = night;
+    if (!night) {
+        bsun = 1.0;
+        bsha = 1.0;
+    }
     int iter1 = 0;
     for (;;) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) x[k] = vegwp[k];
         iter1 = iter1 + 1;
-        int iter2 = 0;
-        x0sun = fmax90(0.1, x1sun);
-        x1sun = 0.99 * x1sun;
-        x0sha = fmax90(0.1, x1sha);
-        x1sha = 0.99 * x1sha;
-        const double tolsun = fabs(x1sun) * eps;
-        const double tolsha = fabs(x1sha) * eps;
-        ci_func_phs(s, x, x0sun, x0sha, f0sun, f0sha, bsun, bsha, bflag, gs0sun, gs0sha, gs_sun, gs_sha);
+        if (bflag) phs_calcstress(s, x, bsun, bsha, gs0sun, gs0sha);
+        if (night) break;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            x0[k] = fmax90(0.1, x1[k]);
+            x1[k] = 0.99 * x1[k];
+            tol[k] = fabs(x1[k]) * eps;
+        }
         const double dbsun = b0sun - bsun;
         const double dbsha = b0sha - bsha;
         b0sun = bsun;
         b0sha = bsha;
-        bflag = false;
-        ci_func_phs(s, x, x1sun, x1sha, f1sun, f1sha, bsun, bsha, bflag, gs0sun, gs0sha, gs_sun, gs_sha);
+        int stage = F_X0, iter2 = 0, biter = 0;
+        double xe[2] = {x0[0], x0[1]}, f[2] = {f0[0], f0[1]}, dx[2] = {0.0, 0.0};
+        double a[2], b[2], c[2], fa[2], fb[2], fc[2], d[2], e[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) a[k] = b[k] = c[k] = fa[k] = fb[k] = fc[k] = d[k] = e[k] = 0.0;
         for (;;) {
-            if (fabs(f0sun) < eps1 && fabs(f0sha) < eps1) {
-                x1sun = x0sun;
-                x1sha = x0sha;
+            ci_func_phs(s, xe[PHS_SUN], xe[PHS_SHA], f[PHS_SUN], f[PHS_SHA], bsun, bsha, gs_sun, gs_sha);
+            bool brent = false;
+            if (stage == F_X0) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    f0[k] = f[k];
+                    xe[k] = x1[k];
+                }
+                stage = F_X1;
+                continue;
+            }
+            if (stage == BRENT) {
+                fb[0] = f[0];
+                fb[1] = f[1];
+                if (fb[PHS_SUN] == 0.0 && fb[PHS_SHA] == 0.0) break;
+                brent = true;
+            } else {
+                f1[0] = f[0];
+                f1[1] = f[1];
+                if (stage == BEST) break;
+                if (stage == SECANT) {
+                    if (fabs(dx[PHS_SUN]) < tol[PHS_SUN] && fabs(dx[PHS_SHA]) < tol[PHS_SHA]) break;
+                    const double fsum = fabs(f1[PHS_SUN] + f1[PHS_SHA]);
+                    if (iter2 == 1 || fsum < minf) {
+                        minf = fsum;
+                        minx[0] = x1[0];
+                        minx[1] = x1[1];
+                    }
+                    if (fabs(f1[PHS_SUN]) < eps1 && fabs(f1[PHS_SHA]) < eps1) break;
+                    if (f1[PHS_SUN] * f0[PHS_SUN] < 0.0 && f1[PHS_SHA] * f0[PHS_SHA] < 0.0) {
+                        // brent_PHS(x0, x1, f0, f1): the bracket, both signs opposite
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            a[k] = x0[k];
+                            b[k] = x1[k];
+                            fa[k] = f0[k];
+                            fb[k] = f1[k];
+                            c[k] = b[k];
+                            fc[k] = fb[k];
+                        }
+                        biter = 0;
+                        brent = true;
+                    } else if (iter2 > itmax) {
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            x1[k] = minx[k];
+                            xe[k] = x1[k];
+                        }
+                        stage = BEST;
+                        continue;
+                    }
+                }
+                if (!brent) {
+                    if (fabs(f0[PHS_SUN]) < eps1 && fabs(f0[PHS_SHA]) < eps1) {
+                        x1[0] = x0[0];
+                        x1[1] = x0[1];
+                        break;
+                    }
+                    if (fabs(f1[PHS_SUN]) < eps1 && fabs(f1[PHS_SHA]) < eps1) break;
+                    iter2 = iter2 + 1;
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        if ((f1[k] - f0[k]) == 0.0) dx[k] = 0.5 * (x1[k] + x0[k]) - x1[k];
+                        else dx[k] = -f1[k] * (x1[k] - x0[k]) / (f1[k] - f0[k]);
+                        x0[k] = x1[k];
+                        x1[k] = x1[k] + dx[k];
+                        xe[k] = x1[k];
+                    }
+                    stage = SECANT;
+                    continue;
+                }
+            }
+            // one Brent iteration up to its evaluation of ci_func_PHS
+            if (biter == itmaxb) break;
+            biter = biter + 1;
+            double tol1[2], xm[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                if ((fb[k] > 0.0 && fc[k] > 0.0) || (fb[k] < 0.0 && fc[k] < 0.0)) {
+                    c[k] = a[k];
+                    fc[k] = fa[k];
+                    d[k] = b[k] - a[k];
+                    e[k] = d[k];
+                }
+                if (fabs(fc[k]) < fabs(fb[k])) {
+                    a[k] = b[k];
+                    b[k] = c[k];
+                    c[k] = a[k];
+                    fa[k] = fb[k];
+                    fb[k] = fc[k];
+                    fc[k] = fa[k];
+                }
+                tol1[k] = 2.0 * epsb * fabs(b[k]) + 0.5 * tol[PHS_SUN];
+                xm[k] = 0.5 * (c[k] - b[k]);
+            }
+            if ((fabs(xm[PHS_SUN]) <= tol1[PHS_SUN] || fb[PHS_SUN] == 0.0) &&
+                (fabs(xm[PHS_SHA]) <= tol1[PHS_SHA] || fb[PHS_SHA] == 0.0))
                 break;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                if (fabs(e[k]) >= tol1[k] && fabs(fa[k]) > fabs(fb[k])) {
+                    const double ss = fb[k] / fa[k];
+                    double p, q;
+                    if (a[k] == c[k]) {
+                        p = 2.0 * xm[k] * ss;
+                        q = 1.0 - ss;
+                    } else {
+                        q = fa[k] / fc[k];
+                        const double r = fb[k] / fc[k];
+                        p = ss * (2.0 * xm[k] * q * (q - r) - (b[k] - a[k]) * (r - 1.0));
+                        q = (q - 1.0) * (r - 1.0) * (ss - 1.0);
+                    }
+                    if (p > 0.0) q = -q;
+                    p = fabs(p);
+                    if (2.0 * p < fmin90(3.0 * xm[k] * q - fabs(tol1[k] * q), fabs(e[k] * q))) {
+                        e[k] = d[k];
+                        d[k] = p / q;
+                    } else {
+                        d[k] = xm[k];
+                        e[k] = d[k];
+                    }
+                } else {
+                    d[k] = xm[k];
+                    e[k] = d[k];
+                }
+                a[k] = b[k];
+                fa[k] = fb[k];
+                if (fabs(d[k]) > tol1[k]) b[k] = b[k] + d[k];
+                else b[k] = b[k] + copysign(fabs(tol1[k]), xm[k]);
+                xe[k] = b[k];
             }
-            if (fabs(f1sun) < eps1 && fabs(f1sha) < eps1) break;
-            iter2 = iter2 + 1;
-            double dxsun, dxsha;
-            if ((f1sun - f0sun) == 0.0) dxsun = 0.5 * (x1sun + x0sun) - x1sun;
-            else dxsun = -f1sun * (x1sun - x0sun) / (f1sun - f0sun);
-            if ((f1sha - f0sha) == 0.0) dxsha = 0.5 * (x1sha + x0sha) - x1sha;
-            else dxsha = -f1sha * (x1sha - x0sha) / (f1sha - f0sha);
-            x0sun = x1sun;
-            x1sun = x1sun + dxsun;
-            x0sha = x1sha;
-            x1sha = x1sha + dxsha;
-            ci_func_phs(s, x, x1sun, x1sha, f1sun, f1sha, bsun, bsha, bflag, gs0sun, gs0sha, gs_sun, gs_sha);
-            if (fabs(dxsun) < tolsun && fabs(dxsha) < tolsha) {
-                x0sun = x1sun;
-                x0sha = x1sha;
-                break;
-            }
-            if (iter2 == 1) {
-                minf = fabs(f1sun + f1sha);
-                minxsun = x1sun;
-                minxsha = x1sha;
-            } else if (fabs(f1sun + f1sha) < minf) {
-                minf = fabs(f1sun + f1sha);
-                minxsun = x1sun;
-                minxsha = x1sha;
-            }
-            if (fabs(f1sun) < eps1 && fabs(f1sha) < eps1) break;
-            if (f1sun * f0sun < 0.0 && f1sha * f0sha < 0.0) {
-                double xsun, xsha;
-                brent_phs(s, xsun, x0sun, x1sun, f0sun, f1sun, xsha, x0sha, x1sha, f0sha, f1sha, tolsun, gs_sun,
-                          gs_sha, bsun, bsha);
-                x0sun = xsun;
-                x0sha = xsha;
-                break;
-            }
-            if (iter2 > itmax) {
-                x1sun = minxsun;
-                x1sha = minxsha;
-                ci_func_phs(s, x, x1sun, x1sha, f1sun, f1sha, bsun, bsha, bflag, gs0sun, gs0sha, gs_sun, gs_sha);
-                break;
-            }
+            stage = BRENT;
         }
         if (bsun > 0.01) gs0sun = gs_sun / bsun;
         if (bsha > 0.01) gs0sha = gs_sha / bsha;
@@ -312,9 +317,8 @@ __device__ __noinline__ double hybrid_phs(PhsSolve &s, double &x0sun, double &x0
         if (fabs(dbsun) < toldb && fabs(dbsha) < toldb) break;
         if (iter1 > itmax) break;
     }
-    x0sun = x1sun;
-    x0sha = x1sha;
-    double soilflux = phs::getvegwp(s.leaf, x, gs_sun, gs_sha, s.qsatl, s.qaf);
+    double soilflux = 0.0;
+    if (!night) soilflux = phs::getvegwp(s.leaf, x, gs_sun, gs_sha, s.qsatl, s.qaf);
 #pragma unroll
     for (int k = 0; k < 4; ++k) vegwp[k] = x[k];
     if (soilflux < 0.0) soilflux = 0.0;
@@ -327,12 +331,12 @@ __device__ __noinline__ double hybrid_phs(PhsSolve &s, double &x0sun, double &x0
 // arrays, vegwp, the noon conductances, vpd_can and qflx_tran_veg where the
 // reference does, and returns btran.  qsatl and qaf are the iteration's.
 template <class PRM, class CAN, class PHA>
-__device__ __noinline__ double photosynthesis_phs(const CView &V, const CSwitch &sw, const PRM &P, const PsnConst &K,
+__device__ __forceinline__ double photosynthesis_phs(const CView &V, const CSwitch &sw, const PRM &P, const PsnConst &K,
                                                   const TFac &T, const PHA &A, const CAN &S, int p, int c,
                                                   int ivt, int nrad, bool noon, double forc_pbot, double tgcm,
                                                   double esat_tv, double eair, double oair, double cair, double rb,
                                                   double qsatl, double qaf, Phase &sun, Phase &sha, Shared &sh,
-                                                  bool &bad)
+                                                  bool &bad, double *soil_lane)
 {
     const auto &H = A.H;
     const long pp = V.p1(p), cc = V.c1(c), ldp = V.ldp;
@@ -418,12 +422,8 @@ __device__ __noinline__ double photosynthesis_phs(const CView &V, const CSwitch 
             s.leaf.psi50[k] = A.table[(phs::T_PSI50 + k) * CTSM_MAX_PFT + ivt];
             s.leaf.ck[k] = A.table[(phs::T_CK + k) * CTSM_MAX_PFT + ivt];
         }
-        s.leaf.k = A.Q.k_soil_root + V.soip(p, 1);
-        s.leaf.smp = A.Q.smp_l + V.soi(c, 1);
-        s.leaf.z = A.Q.z + V.sno(c, 1);
-        s.leaf.sk = ldp;
-        s.leaf.ss = V.ldc;
-        s.leaf.n = A.nlevsoi;
+        phs::stage_soil(s.leaf, A.Q.k_soil_root + V.soip(p, 1), ldp, A.Q.smp_l + V.soi(c, 1), A.Q.z + V.sno(c, 1),
+                        V.ldc, A.nlevsoi, soil_lane);
         s.qsatl = qsatl;
         s.qaf = qaf;
         s.morning = H.local_morning[pp] != 0;
@@ -435,26 +435,9 @@ __device__ __noinline__ double photosynthesis_phs(const CView &V, const CSwitch 
         double vegwp[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) vegwp[k] = H.vegwp[pp + k * ldp];
-        if (par_z[PHS_SUN] <= 0.0) {
-            // night: the stress factors at the minimum conductance (:3500-3548)
-            vegwp[0] = 1.0;
-            phs_calcstress(s, vegwp, bb[PHS_SUN], bb[PHS_SHA], gsmin, gsmin);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                H.ac_phs[pp + k * ldp] = 0.0;
-                H.aj_phs[pp + k * ldp] = 0.0;
-                H.ap_phs[pp + k * ldp] = 0.0;
-                H.ag_phs[pp + k * ldp] = 0.0;
-                const double an = (!crop || !modify) ? 0.0 - bb[k] * lmr_z[k] : 0.0 - lmr_z[k];
-                (k == PHS_SUN ? H.an_sun : H.an_sha)[pp] = an;
-                ph[k]->psn_z = 0.0;
-                ph[k]->rs_z = fmin90(rsmax0, 1.0 / (fmax90(bb[k] * gsmin, 1.0)) * cf);
-                ph[k]->ci_z = 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < 2; ++k) ph[k]->gs_ph = cf / ph[k]->rs_z;
-        } else {
-            // day (:3550-3697)
+        const bool night = par_z[PHS_SUN] <= 0.0;
+        double ci0 = 0.0, gs[2] = {0.0, 0.0};
+        if (!night) {       // day (:3550-3697)
             const double ceair = fmin90(eair, esat_tv);
             double rh_can;
             if (!medlyn) {
@@ -470,9 +453,7 @@ __device__ __noinline__ double photosynthesis_phs(const CView &V, const CSwitch 
                 if (!quadratic(P.theta_psii, -(qabs + jmax_z[k]), qabs * jmax_z[k], r1, r2)) bad = true;
                 s.je[k] = fmin90(r1, r2);
             }
-            double ci[2];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) ci[k] = K.c3 ? 0.7 * cair : 0.4 * cair;
+            ci0 = K.c3 ? 0.7 * cair : 0.4 * cair;
             s.c3 = K.c3;
             s.medlyn = medlyn;
             s.forc_pbot = forc_pbot;
@@ -504,9 +485,29 @@ __device__ __noinline__ double photosynthesis_phs(const CView &V, const CSwitch 
             }
             s.an[PHS_SUN] = H.an_sun[pp];
             s.an[PHS_SHA] = H.an_sha[pp];
-            double gs[2] = {S.gs_mol_sun[pp], S.gs_mol_sha[pp]};
-            const double soilflux = hybrid_phs(s, ci[PHS_SUN], ci[PHS_SHA], vegwp, bb[PHS_SUN], bb[PHS_SHA],
-                                               gs[PHS_SUN], gs[PHS_SHA]);
+            gs[PHS_SUN] = S.gs_mol_sun[pp];
+            gs[PHS_SHA] = S.gs_mol_sha[pp];
+        } else {
+            vegwp[0] = 1.0;     // marks night to calcstress
+        }
+        const double soilflux = hybrid_phs(s, night, gsmin, ci0, vegwp, bb[PHS_SUN], bb[PHS_SHA], gs[PHS_SUN],
+                                           gs[PHS_SHA]);
+        if (night) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                H.ac_phs[pp + k * ldp] = 0.0;
+                H.aj_phs[pp + k * ldp] = 0.0;
+                H.ap_phs[pp + k * ldp] = 0.0;
+                H.ag_phs[pp + k * ldp] = 0.0;
+                const double an = (!crop || !modify) ? 0.0 - bb[k] * lmr_z[k] : 0.0 - lmr_z[k];
+                (k == PHS_SUN ? H.an_sun : H.an_sha)[pp] = an;
+                ph[k]->psn_z = 0.0;
+                ph[k]->rs_z = fmin90(rsmax0, 1.0 / (fmax90(bb[k] * gsmin, 1.0)) * cf);
+                ph[k]->ci_z = 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) ph[k]->gs_ph = cf / ph[k]->rs_z;
+        } else {
             s.tran_set = true;
             s.tran = soilflux;
             if (s.bad) bad = true;

@@ -111,11 +111,14 @@ __global__ void __launch_bounds__(256) k_phs_root_sink(PView V, ctsm_phs_state S
     S.qflx_phs_neg[cc] = neg;
 }
 
-// Three waves per SIMD (168 VGPRs, 124 B of scratch per lane): 4.52 ms against 4.93 ms
-// at the compiler's own choice of two, for 655,821 patches.
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) k_phs_calcstress(PView V, ctsm_phs_stress_state S, const double *__restrict__ T,
-                                                       int npft, int n, const int32_t *__restrict__ filter,
-                                                       ErrWord *err)
+// Bound by FP64 issue: up to 50 Newton passes of 8 powers, ~20 divides and the
+// root's 20-layer sum.  A patch per lane, its soil in LDS (stage_soil, 20 KB a
+// wave: two waves per SIMD, 219 VGPRs, no scratch).  262,144 patches: 2.24 ms when
+// every pass read its layers from HBM and took 28 powers, 0.65 ms so (0.69 ms with
+// the scheduler told of the two waves instead of asked for three).
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8)))
+k_phs_calcstress(PView V, ctsm_phs_stress_state S, const double *__restrict__ T, int npft, int n,
+                 const int32_t *__restrict__ filter, ErrWord *err)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -134,12 +137,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8)))
         P.psi50[k] = T[(T_PSI50 + k) * CTSM_MAX_PFT + ivt];
         P.ck[k] = T[(T_CK + k) * CTSM_MAX_PFT + ivt];
     }
-    P.k = S.k_soil_root + V.soip(p, 1);
-    P.smp = S.smp_l + V.soi(c, 1);
-    P.z = S.z + V.sno(c, 1);
-    P.sk = V.ldp;
-    P.ss = V.ldc;
-    P.n = V.nlevsoi;
+    __shared__ double soil[SOIL_LDS * SOIL_STRIDE];
+    stage_soil(P, S.k_soil_root + V.soip(p, 1), V.ldp, S.smp_l + V.soi(c, 1), S.z + V.sno(c, 1), V.ldc, V.nlevsoi,
+               soil + threadIdx.x);
     const double qsatl = S.qsatl[pp], qaf = S.qaf[pp];
     const double gs_sun_in = S.gs_mol_sun[pp], gs_sha_in = S.gs_mol_sha[pp];
     double x[4];

@@ -37,14 +37,77 @@ constexpr double TOL_LAI = 0.001;
 struct Leaf {
     double laisun, laisha, elai, esai, tsai, htop, fdry, thm, rho, pbot, gb;
     double kmax[4], psi50[4], ck[4];
-    const double *k, *smp, *z;   // layer 1 of k_soil_root(p, :), smp_l(c, :), z(c, :)
-    long sk, ss;
+    // The soil below the patch, staged once (stage_soil): k_soil_root(p, :) and
+    // 1000 z(c, :) in the lane's LDS column, and the sums over the layers that
+    // no potential enters -- of k, k smp, smp - 1000 z and k (smp - 1000 z).
+    const double *k, *g;
+    double sum_k, sum_ks, sum_w, sum_kw;
+    const double *smp;           // layer 1 of smp_l(c, :), stride ss
+    long ss;
     int n;
 };
+// LDS doubles per lane of a one-wave block, and the stride between layers
+constexpr int SOIL_LDS = 2 * MAX_NLEVSOI;
+constexpr int SOIL_STRIDE = 64;
 
-__device__ __forceinline__ double d1plc(double x, double psi50, double ck)
+// Fills P's soil members; lds is the lane's column of a one-wave block's
+// [SOIL_LDS][SOIL_STRIDE] array.  The loads of all layers are in flight at once.
+// Read from HBM layer by layer instead, as the sums of every Newton pass need
+// them, they were what a pass waited for.
+__device__ __forceinline__ void stage_soil(Leaf &P, const double *__restrict__ k, long sk,
+                                           const double *__restrict__ smp, const double *__restrict__ z, long ss, int n,
+                                           double *lds)
 {
-    return -ck * LN2 * cm_pow(2.0, -cm_pow(x / psi50, ck)) * cm_pow(x / psi50, ck) / x;
+    P.k = lds;
+    P.g = lds + MAX_NLEVSOI * SOIL_STRIDE;
+    P.smp = smp;
+    P.ss = ss;
+    P.n = n;
+    double kj[MAX_NLEVSOI], gj[MAX_NLEVSOI], wj[MAX_NLEVSOI];
+#pragma unroll
+    for (int j = 0; j < MAX_NLEVSOI; ++j) {
+        const int i = j < n ? j : n - 1;
+        kj[j] = k[i * sk];
+        gj[j] = 1000.0 * z[i * ss];
+        wj[j] = smp[i * ss];
+    }
+    double a = 0.0, b = 0.0, c = 0.0, d = 0.0;
+#pragma unroll
+    for (int j = 0; j < MAX_NLEVSOI; ++j) {
+        lds[j * SOIL_STRIDE] = kj[j];
+        lds[(MAX_NLEVSOI + j) * SOIL_STRIDE] = gj[j];
+        if (j >= n) continue;
+        a = a + kj[j];
+        b = b + kj[j] * wj[j];
+        c = c + (wj[j] - gj[j]);
+        d = d + kj[j] * (wj[j] - gj[j]);
+    }
+    P.sum_k = a;
+    P.sum_ks = b;
+    P.sum_w = c;
+    P.sum_kw = d;
+}
+
+// The four segments' vulnerability curves at x: u = (x/psi50)**ck, w = 2**-u,
+// v = plc (w cut to zero below 0.005); d1plc's value from the same powers.  One
+// Newton pass needs each curve and its slope; evaluated through plc and d1plc in
+// spacF and spacA apart, it took 28 powers instead of 8.
+struct Curves {
+    double u[4], w[4], v[4];
+};
+__device__ __forceinline__ void curves(const Leaf &P, const double *x, Curves &C)
+{
+#pragma unroll
+    for (int k = 0; k < 4; ++k) C.u[k] = cm_pow(x[k] / P.psi50[k], P.ck[k]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) C.w[k] = cm_pow(2.0, -C.u[k]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) C.v[k] = C.w[k] < 0.005 ? 0.0 : C.w[k];
+}
+// d1plc
+__device__ __forceinline__ double slope(const Leaf &P, const Curves &C, const double *x, int k)
+{
+    return -P.ck[k] * LN2 * C.w[k] * C.u[k] / x[k];
 }
 
 // getqflx (:5080-5164)
@@ -78,20 +141,30 @@ __device__ void getqflx(const Leaf &P, double qsatl, double qaf, bool havegs, do
     }
 }
 
+// the root's layer sum of spacF: k (x + 1000 z)
+__device__ __forceinline__ double root_sum(const Leaf &P, double x)
+{
+    double s = 0.0;
+    if (P.n == MAX_NLEVSOI) {
+#pragma unroll
+        for (int j = 0; j < MAX_NLEVSOI; ++j) s = s + P.k[j * SOIL_STRIDE] * (x + P.g[j * SOIL_STRIDE]);
+    } else {
+        for (int j = 0; j < P.n; ++j) s = s + P.k[j * SOIL_STRIDE] * (x + P.g[j * SOIL_STRIDE]);
+    }
+    return s;
+}
+
 // spacF (:4898-4976)
-__device__ void spacF(const Leaf &P, const double *x, double *f, double q_sun, double q_sha)
+__device__ __forceinline__ void spacF(const Leaf &P, const Curves &C, const double *x, double *f, double q_sun,
+                                      double q_sha)
 {
     const double grav1 = P.htop * 1000.0;
-    const double fsto1 = plc(x[0], P.psi50[0], P.ck[0]), fsto2 = plc(x[1], P.psi50[1], P.ck[1]);
-    const double fx = plc(x[2], P.psi50[2], P.ck[2]), fr = plc(x[3], P.psi50[3], P.ck[3]);
+    const double fsto1 = C.v[0], fsto2 = C.v[1], fx = C.v[2], fr = C.v[3];
     f[0] = q_sun * fsto1 - P.laisun * P.kmax[0] * fx * (x[2] - x[0]);
     f[1] = q_sha * fsto2 - P.laisha * P.kmax[1] * fx * (x[2] - x[1]);
     f[2] = P.laisun * P.kmax[0] * fx * (x[2] - x[0]) + P.laisha * P.kmax[1] * fx * (x[2] - x[1])
            - P.tsai * P.kmax[2] / P.htop * fr * (x[3] - x[2] - grav1);
-    double s1 = 0.0, s2 = 0.0;
-    for (int j = 0; j < P.n; ++j) s1 = s1 + P.k[j * P.sk] * (x[3] + P.z[j * P.ss] * 1000.0);
-    for (int j = 0; j < P.n; ++j) s2 = s2 + P.k[j * P.sk] * P.smp[j * P.ss];
-    f[3] = P.tsai * P.kmax[2] / P.htop * fr * (x[3] - x[2] - grav1) + s1 - s2;
+    f[3] = P.tsai * P.kmax[2] / P.htop * fr * (x[3] - x[2] - grav1) + root_sum(P, x[3]) - P.sum_ks;
     if (P.laisha < TOL_LAI) {
         const double t = f[0];
         f[0] = f[1];
@@ -100,7 +173,8 @@ __device__ void spacF(const Leaf &P, const double *x, double *f, double q_sun, d
 }
 
 // spacA (:4715-4893); invA row-major; returns true when not invertible
-__device__ bool spacA(const Leaf &P, const double *x, double *iA, double q_sun, double q_sha)
+__device__ __forceinline__ bool spacA(const Leaf &P, const Curves &C, const double *x, double *iA, double q_sun,
+                                      double q_sha)
 {
     double A[16];
 #pragma unroll
@@ -108,10 +182,9 @@ __device__ bool spacA(const Leaf &P, const double *x, double *iA, double q_sun, 
 #define AA(i, j) A[((i) - 1) * 4 + (j) - 1]
 #define IA(i, j) iA[((i) - 1) * 4 + (j) - 1]
     const double grav1 = P.htop * 1000.0;
-    const double fsto1 = plc(x[0], P.psi50[0], P.ck[0]), fsto2 = plc(x[1], P.psi50[1], P.ck[1]);
-    const double fx = plc(x[2], P.psi50[2], P.ck[2]), fr = plc(x[3], P.psi50[3], P.ck[3]);
-    const double dfsto1 = d1plc(x[0], P.psi50[0], P.ck[0]), dfsto2 = d1plc(x[1], P.psi50[1], P.ck[1]);
-    const double dfx = d1plc(x[2], P.psi50[2], P.ck[2]), dfr = d1plc(x[3], P.psi50[3], P.ck[3]);
+    const double fx = C.v[2], fr = C.v[3];
+    const double dfsto1 = slope(P, C, x, 0), dfsto2 = slope(P, C, x, 1);
+    const double dfx = slope(P, C, x, 2), dfr = slope(P, C, x, 3);
     const double ks = P.kmax[0], kh = P.kmax[1], kx = P.kmax[2];
     AA(1, 1) = -(P.laisun * ks * fx) - q_sun * dfsto1;
     AA(1, 3) = P.laisun * ks * dfx * (x[2] - x[0]) + P.laisun * ks * fx;
@@ -123,9 +196,7 @@ __device__ bool spacA(const Leaf &P, const double *x, double *iA, double q_sun, 
                - P.laisha * kh * fx - P.tsai * kx / P.htop * fr;
     AA(3, 4) = P.tsai * kx / P.htop * dfr * (x[3] - x[2] - grav1) + P.tsai * kx / P.htop * fr;
     AA(4, 3) = P.tsai * kx / P.htop * fr;
-    double sk = 0.0;
-    for (int j = 0; j < P.n; ++j) sk = sk + P.k[j * P.sk];
-    AA(4, 4) = -(P.tsai * kx / P.htop * fr) - P.tsai * kx / P.htop * dfr * (x[3] - x[2] - grav1) - sk;
+    AA(4, 4) = -(P.tsai * kx / P.htop * fr) - P.tsai * kx / P.htop * dfr * (x[3] - x[2] - grav1) - P.sum_k;
     if (P.laisun > TOL_LAI && P.laisha > TOL_LAI) {
         const double determ = AA(4, 4) * AA(2, 2) * AA(3, 3) * AA(1, 1) - AA(4, 4) * AA(2, 2) * AA(3, 1) * AA(1, 3)
                               - AA(4, 4) * AA(3, 2) * AA(2, 3) * AA(1, 1) - AA(4, 3) * AA(1, 1) * AA(2, 2) * AA(3, 4);
@@ -183,17 +254,8 @@ __device__ double getvegwp(const Leaf &P, double *x, double gs_sun, double gs_sh
     const double grav1 = 1000.0 * P.htop;
     double q_sun, q_sha;
     getqflx(P, qsatl, qaf, true, gs_sun, gs_sha, q_sun, q_sha);
-    double sk = 0.0;
-    for (int j = 0; j < P.n; ++j) sk = sk + P.k[j * P.sk];
-    if (fabs(sk) == 0.0) {
-        double s = 0.0;
-        for (int j = 0; j < P.n; ++j) s = s + (P.smp[j * P.ss] - 1000.0 * P.z[j * P.ss]);
-        x[3] = s / P.n;
-    } else {
-        double s = 0.0;
-        for (int j = 0; j < P.n; ++j) s = s + P.k[j * P.sk] * (P.smp[j * P.ss] - 1000.0 * P.z[j * P.ss]);
-        x[3] = (s - q_sun - q_sha) / sk;
-    }
+    if (fabs(P.sum_k) == 0.0) x[3] = P.sum_w / P.n;
+    else x[3] = (P.sum_kw - q_sun - q_sha) / P.sum_k;
     const double fr = plc(x[3], P.psi50[3], P.ck[3]);
     if (P.tsai > 0.0 && fr > 0.0)
         x[2] = x[3] - grav1 - (q_sun + q_sha) / (fr * P.kmax[3] / P.htop * P.tsai);
@@ -202,8 +264,13 @@ __device__ double getvegwp(const Leaf &P, double *x, double gs_sun, double gs_sh
     const double fx = plc(x[2], P.psi50[2], P.ck[2]);
     x[1] = (P.laisha > 0.0 && fx > 0.0) ? x[2] - (q_sha / (fx * P.kmax[2] * P.laisha)) : x[2];
     x[0] = (P.laisun > 0.0 && fx > 0.0) ? x[2] - (q_sun / (fx * P.kmax[2] * P.laisun)) : x[2];
+    double w[MAX_NLEVSOI];
+#pragma unroll
+    for (int j = 0; j < MAX_NLEVSOI; ++j) w[j] = P.smp[(j < P.n ? j : P.n - 1) * P.ss];
     double soilflux = 0.0;
-    for (int j = 0; j < P.n; ++j) soilflux = soilflux + P.k[j * P.sk] * (P.smp[j * P.ss] - x[3] - 1000.0 * P.z[j * P.ss]);
+#pragma unroll
+    for (int j = 0; j < MAX_NLEVSOI; ++j)
+        if (j < P.n) soilflux = soilflux + P.k[j * SOIL_STRIDE] * (w[j] - x[3] - P.g[j * SOIL_STRIDE]);
     return soilflux;
 }
 
@@ -226,13 +293,15 @@ __device__ __forceinline__ bool calcstress(const Leaf &P, double *x, double gs_s
         for (;;) {   // at most 51 passes: the iter > itmax exit
             iter = iter + 1;
             double f[4], iA[16], dx[4];
-            spacF(P, x, f, q_sun, q_sha);
+            Curves C;
+            curves(P, x, C);
+            spacF(P, C, x, f, q_sun, q_sha);
             double ff = 0.0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) ff = ff + f[k] * f[k];
             if (sqrt(ff) < 1.e-6 * (q_sun + q_sha)) { flag = false; break; }
             if (iter > 50) { flag = false; break; }
-            flag = spacA(P, x, iA, q_sun, q_sha);
+            flag = spacA(P, C, x, iA, q_sun, q_sha);
             if (flag) break;
             if (P.laisun > TOL_LAI && P.laisha > TOL_LAI) {
 #pragma unroll
