@@ -115,8 +115,8 @@ def autotune(ctx, ds, filter_dev=None, n=None, steps=8, reps=2, candidates=None,
 # (first-round iterations, later-round iterations) of the CanopyFluxes
 # leaf-temperature iteration; first > itmax is the one-pass kernel.
 CANOPY_CANDIDATES = [(1001, 1), (4, 2), (4, 4), (5, 3), (6, 3), (6, 6), (8, 4), (10, 5)]
-# register budgets (waves per SIMD) of the CanopyFluxes kernel
-CANOPY_WAVES = (1, 2, 3)
+# waves per SIMD of the CanopyFluxes kernel (3 is the two-wave kernel too)
+CANOPY_WAVES = (1, 2)
 
 
 def autotune_canopy(ctx, ds, filter_dev=None, n=None, reps=2, candidates=None, waves=None, dtime=1800.0,

@@ -1,7 +1,7 @@
-// canopy.hip -- CanopyFluxes (CanopyFluxesMod.F90:191-1765) for gfx950: one
-// lane per patch runs the whole time step (root stress, roughness, Monin-
-// Obukhov initialisation, the Newton / stability iteration with sun and shade
-// photosynthesis, the post-iteration fluxes) with its state in registers.
+// canopy.hip -- CanopyFluxes (CanopyFluxesMod.F90:191-1765) for gfx950, a lane
+// per patch: the set-up (root stress, roughness, Monin-Obukhov initialisation),
+// rounds of the Newton / stability iteration with sun and shade photosynthesis and
+// its state in registers, the post-iteration fluxes.
 //
 // Callees restated here: FrictionVelocity / StabilityFunc1/2 / MoninObukIni
 // (FrictionVelocityMod.F90:754-1209), QSat (QSatMod.F90:61-127),
@@ -19,6 +19,7 @@
 // (ft, fth, 2**x) depend on t_veg only, so they are evaluated once per
 // iteration and shared by the sun and shade phases (the same values the
 // reference computes twice).
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -72,6 +73,30 @@ struct CSwitch {
 __device__ __forceinline__ double p4(double x) { const double x2 = x * x; return x2 * x2; }
 __device__ __forceinline__ double p3(double x) { return (x * x) * x; }
 
+// Divisions by one denominator.  recip(b) holds the refined reciprocal that an IEEE
+// division by b forms (v_rcp_f64 and two Newton steps) and a / r finishes it (a
+// product, its remainder, one correction): the instructions of the compiler's own
+// division without the scaling that only operands near the ends of the exponent
+// range need, so the quotient is the correctly rounded one, for 4 instructions
+// instead of 11.  For denominators and quotients of magnitudes between 2^-900 and
+// 2^900 (zero, infinite and NaN operands are settled by v_div_fixup as in a
+// division).
+struct Recip {
+    double b, y;
+};
+__device__ __forceinline__ Recip recip(double b)
+{
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(y, fma(-b, y, 1.0), y);
+    y = fma(y, fma(-b, y, 1.0), y);
+    return Recip{b, y};
+}
+__device__ __forceinline__ double operator/(double a, const Recip &r)
+{
+    const double q = a * r.y;
+    return __builtin_amdgcn_div_fixup(fma(fma(-r.b, q, a), r.y, q), r.b, a);
+}
+
 // QSatMod.F90:61-127
 __device__ __forceinline__ void qsat(double T, double p, double &qs, double &es, double &qsdT)
 {
@@ -113,7 +138,8 @@ __device__ __forceinline__ double qsat_only(double T, double p, double &es)
 }
 
 // quadraticMod.F90:17-74; false where the reference calls endrun
-__device__ __forceinline__ bool quadratic(double a, double b, double c, double &r1, double &r2)
+template <class DIV>     // the type of a as a denominator: double, or Recip
+__device__ __forceinline__ bool quadratic(double a, const DIV &ra, double b, double c, double &r1, double &r2)
 {
     if (a == 0.0) { r1 = r2 = 0.0; return false; }
     double root = b * b - 4.0 * a * c;
@@ -125,21 +151,25 @@ __device__ __forceinline__ bool quadratic(double a, double b, double c, double &
     double q;
     if (b >= 0.0) q = -0.5 * (b + sqrt(root));
     else q = -0.5 * (b - sqrt(root));
-    r1 = q / a;
+    r1 = q / ra;
     r2 = (q != 0.0) ? c / q : 1.e36;
     return ok;
 }
+__device__ __forceinline__ bool quadratic(double a, double b, double c, double &r1, double &r2)
+{
+    return quadratic(a, a, b, c, r1, r2);
+}
 
-__device__ __forceinline__ double stab1(double zeta)
+__device__ __forceinline__ double stab1(double zeta, const double *lt)
 {
     const double chik2 = sqrt(1.0 - 16.0 * zeta);
     const double chik = sqrt(chik2);
-    return 2.0 * cm_log((1.0 + chik) * 0.5) + cm_log((1.0 + chik2) * 0.5) - 2.0 * cm_atan(chik) + PI * 0.5;
+    return 2.0 * cm_log_tab((1.0 + chik) * 0.5, lt) + cm_log_tab((1.0 + chik2) * 0.5, lt) - 2.0 * cm_atan(chik) + PI * 0.5;
 }
-__device__ __forceinline__ double stab2(double zeta)
+__device__ __forceinline__ double stab2(double zeta, const double *lt)
 {
     const double chik2 = sqrt(1.0 - 16.0 * zeta);
-    return 2.0 * cm_log((1.0 + chik2) * 0.5);
+    return 2.0 * cm_log_tab((1.0 + chik2) * 0.5, lt);
 }
 
 // the temperature / humidity profile block repeated in FrictionVelocityMod.F90:916-1060;
@@ -150,20 +180,21 @@ __device__ __forceinline__ double stab2(double zeta)
 // their height ratio, the two unstable ones stab2(z0 / obu)) rather than once
 // per regime branch.  Every lane computes its own regime's expression with
 // the same operations in the same order.
-__device__ double temp_profile(double zldis, double z0, double obu, double log_z)
+// lt: log's table in LDS.
+__device__ __forceinline__ double temp_profile(double zldis, double z0, const Recip &obu, double log_z, const double *lt)
 {
     const double zetat = 0.465;
     const double zeta = zldis / obu;
     const bool ra = zeta < -zetat, rb = !ra && zeta < 0.0, rc = !ra && !rb && zeta <= 1.0, rd = !(ra || rb || rc);
     double lg = 0.0, sa = 0.0, sb = 0.0, pw = 0.0, lz = 0.0;
-    if (ra || rd) lg = cm_log(ra ? -zetat * obu / z0 : obu / z0);
-    if (ra || rb) sb = stab2(z0 / obu);
+    if (ra || rd) lg = cm_log_tab(ra ? -zetat * obu.b / z0 : obu.b / z0, lt);
+    if (ra || rb) sb = stab2(z0 / obu, lt);
     if (ra) {
-        sa = stab2(-zetat);
-        pw = cm_pow(zetat, -0.333) - cm_pow(-zeta, -0.333);
+        sa = stab2(-zetat, cm_log_table());
+        pw = cm_pow(zetat, -0.333) - cm_pow_tab(-zeta, -0.333, lt);
     }
-    if (rb) sa = stab2(zeta);
-    if (rd) lz = cm_log(zeta);
+    if (rb) sa = stab2(zeta, lt);
+    if (rd) lz = cm_log_tab(zeta, lt);
     double den;
     if (ra) den = lg - sa + sb + 0.8 * pw;
     else if (rb) den = log_z - sa + sb;
@@ -172,12 +203,12 @@ __device__ double temp_profile(double zldis, double z0, double obu, double log_z
     return VKC / den;
 }
 
-__device__ __forceinline__ double fm_profile(double z)
+__device__ __forceinline__ double fm_profile(double z, const double *lt)
 {
     // dust-model fm of FrictionVelocityMod.F90:1072-1095 for z < 0
-    const double tmp1 = cm_pow(1.0 - 16.0 * z, 0.25);
-    const double tmp2 = cm_log((1.0 + tmp1 * tmp1) / 2.0);
-    const double tmp3 = cm_log((1.0 + tmp1) / 2.0);
+    const double tmp1 = cm_pow_tab(1.0 - 16.0 * z, 0.25, lt);
+    const double tmp2 = cm_log_tab((1.0 + tmp1 * tmp1) / 2.0, lt);
+    const double tmp3 = cm_log_tab((1.0 + tmp1) / 2.0, lt);
     return 2.0 * tmp3 + tmp2 - 2.0 * cm_atan(tmp1) + 1.5707963;
 }
 
@@ -187,42 +218,45 @@ struct FV {
 
 // FrictionVelocityMod.F90:754-1117 (patch form), the part the canopy
 // iteration consumes: ustar, the heat / moisture profile factors temp1 and
-// temp2, and the running mean of the dust-model fm.  The logarithms of
-// height over roughness length (lm: momentum, lh: heat, lq: moisture) are the
-// step's constants.
+// temp2, and the running mean of the dust-model fm.  The heights above the
+// displacement height (zldis, zht, zhq), the roughness length (one value for
+// momentum, heat and moisture over vegetation) and the logarithms of height over
+// it (lm: momentum, lh: heat) are the step's constants; the moisture height's is
+// taken where it differs from the heat's.  The regimes' divides by obu share its
+// reciprocal.
 struct FVLogs {
-    double lm, lh, lq;
+    double lm, lh;
 };
-__device__ __forceinline__ void friction_velocity(double hu, double ht, double hq, double displa, double z0m,
-                                                  double z0h, double z0q, const FVLogs &L, double obu, int iter,
-                                                  double um, FV &o)
+__device__ __forceinline__ void friction_velocity(double zldis, double zht, double zhq, double z0, const FVLogs &L,
+                                                  double obu_, int iter, double um, FV &o, const double *lt)
 {
     const double zetam = 1.574;
-    const double zldis = hu - displa;
+    const double z0m = z0, z0h = z0, z0q = z0;
+    const Recip obu = recip(obu_);
     const double zeta = zldis / obu;
     // each elementary function once for the lanes whose regime needs it (as
     // in temp_profile)
     const bool ra = zeta < -zetam, rb = !ra && zeta < 0.0, rc = !ra && !rb && zeta <= 1.0, rd = !(ra || rb || rc);
     double lg = 0.0, sa = 0.0, sb = 0.0, pw = 0.0, lz = 0.0;
-    if (ra || rd) lg = cm_log(ra ? -zetam * obu / z0m : obu / z0m);
-    if (ra || rb) sb = stab1(z0m / obu);
+    if (ra || rd) lg = cm_log_tab(ra ? -zetam * obu_ / z0m : obu_ / z0m, lt);
+    if (ra || rb) sb = stab1(z0m / obu, lt);
     if (ra) {
-        sa = stab1(-zetam);
-        pw = cm_pow(-zeta, 0.333) - cm_pow(zetam, 0.333);
+        sa = stab1(-zetam, cm_log_table());
+        pw = cm_pow_tab(-zeta, 0.333, lt) - cm_pow(zetam, 0.333);
     }
-    if (rb) sa = stab1(zeta);
-    if (rd) lz = cm_log(zeta);
+    if (rb) sa = stab1(zeta, lt);
+    if (rd) lz = cm_log_tab(zeta, lt);
     double den;
     if (ra) den = lg - sa + sb + 1.14 * pw;
     else if (rb) den = L.lm - sa + sb;
     else if (rc) den = L.lm + 5.0 * zeta - 5.0 * z0m / obu;
     else den = lg + 5.0 - 5.0 * z0m / obu + (5.0 * lz + zeta - 1.0);
     o.ustar = VKC * um / den;
-    o.temp1 = temp_profile(ht - displa, z0h, obu, L.lh);
-    if (hq == ht && z0q == z0h) o.temp2 = o.temp1;
-    else o.temp2 = temp_profile(hq - displa, z0q, obu, L.lq);
+    o.temp1 = temp_profile(zht, z0h, obu, L.lh, lt);
+    if (zhq == zht) o.temp2 = o.temp1;
+    else o.temp2 = temp_profile(zhq, z0q, obu, cm_log_tab(zhq / z0q, lt), lt);
     const double zm1 = fmin90(zeta, 1.0);
-    const double fmnew = (zm1 < 0.0) ? fm_profile(zm1) : -5.0 * zm1;
+    const double fmnew = (zm1 < 0.0) ? fm_profile(zm1, lt) : -5.0 * zm1;
     o.fm = (iter == 1) ? fmnew : 0.5 * (o.fm + fmnew);
 }
 
@@ -231,13 +265,14 @@ __device__ __forceinline__ void friction_velocity(double hu, double ht, double h
 // them, so they are evaluated once, from the inputs (obu, um) and the ustar
 // and fm of the last iteration: the same values the reference keeps from its
 // last call.
-__device__ void friction_velocity_diag(double hu, double displa, double z0m, double z0h, double z0q, double obu,
-                                       double ur, double um, FV &o)
+__device__ __forceinline__ void friction_velocity_diag(double hu, double displa, double z0m, double z0h, double z0q, double obu_,
+                                       double ur, double um, FV &o, const double *lt)
 {
     const double zetam = 1.574;
+    const Recip obu = recip(obu_);
     const double zldis = hu - displa;
     const double zeta = zldis / obu;
-    if (zeta < 0.0) o.vds = 2.e-3 * o.ustar * (1.0 + cm_pow(300.0 / (-obu), 0.666));
+    if (zeta < 0.0) o.vds = 2.e-3 * o.ustar * (1.0 + cm_pow_tab(300.0 / (-obu_), 0.666, lt));
     else o.vds = 2.e-3 * o.ustar;
     if (zldis - z0m <= 10.0) {
         o.u10_clm = um;
@@ -247,15 +282,15 @@ __device__ void friction_velocity_diag(double hu, double displa, double z0m, dou
         // regime needs it (as in friction_velocity)
         const bool ra = zeta < -zetam, rb = !ra && zeta < 0.0, rc = !ra && !rb && zeta <= 1.0;
         const bool rd = !(ra || rb || rc);
-        const double lg = cm_log(ra ? -zetam * obu / z10 : (rd ? obu / z10 : zldis / z10));
+        const double lg = cm_log_tab(ra ? -zetam * obu_ / z10 : (rd ? obu_ / z10 : zldis / z10), lt);
         double sa = 0.0, sb = 0.0, pw = 0.0, lz = 0.0;
-        if (ra || rb) sb = stab1(z10 / obu);
+        if (ra || rb) sb = stab1(z10 / obu, lt);
         if (ra) {
-            sa = stab1(-zetam);
-            pw = cm_pow(-zeta, 0.333) - cm_pow(zetam, 0.333);
+            sa = stab1(-zetam, cm_log_table());
+            pw = cm_pow_tab(-zeta, 0.333, lt) - cm_pow(zetam, 0.333);
         }
-        if (rb) sa = stab1(zeta);
-        if (rd) lz = cm_log(zeta);
+        if (rb) sa = stab1(zeta, lt);
+        if (rd) lz = cm_log_tab(zeta, lt);
         double t;
         if (ra) t = lg - sa + sb + 1.14 * pw;
         else if (rb) t = lg - sa + sb;
@@ -264,30 +299,22 @@ __device__ void friction_velocity_diag(double hu, double displa, double z0m, dou
         o.u10_clm = um - (o.ustar / VKC * t);
     }
     o.va = um;
-    o.temp12m = temp_profile(2.0 + z0h, z0h, obu, cm_log((2.0 + z0h) / z0h));
+    o.temp12m = temp_profile(2.0 + z0h, z0h, obu, cm_log_tab((2.0 + z0h) / z0h, lt), lt);
     if (z0q == z0h) o.temp22m = o.temp12m;
-    else o.temp22m = temp_profile(2.0 + z0q, z0q, obu, cm_log((2.0 + z0q) / z0q));
+    else o.temp22m = temp_profile(2.0 + z0q, z0q, obu, cm_log_tab((2.0 + z0q) / z0q, lt), lt);
     double zeta10 = fmin90(10.0 / obu, 1.0);
     if (zeta == 0.0) zeta10 = 0.0;
-    const double fm10 = (zeta10 < 0.0) ? fm_profile(zeta10) : -5.0 * zeta10;
-    const double tmp4 = cm_log(fmax90(1.0, hu / 10.0));
+    const double fm10 = (zeta10 < 0.0) ? fm_profile(zeta10, lt) : -5.0 * zeta10;
+    const double tmp4 = cm_log_tab(fmax90(1.0, hu / 10.0), lt);
     o.u10 = ur - o.ustar / VKC * (tmp4 - o.fm + fm10);
     o.fv = o.ustar;
 }
 
-// the exponents of ft and fth (PhotosynthesisMod.F90:2488-2561)
-__device__ __forceinline__ double ft_arg(double tl, double ha)
+// the exponents of ft and fth (PhotosynthesisMod.F90:2488-2561): haq is
+// ha / (rgas (tfrz + 25)), t25 = 1 - (tfrz + 25) / tl, rt the reciprocal of rgas tl
+__device__ __forceinline__ double fth_arg(double tl, const Recip &rt, double hd, double se)
 {
-    return ha / (RGAS * 1.e-3 * (TFRZ + 25.0)) * (1.0 - (TFRZ + 25.0) / tl);
-}
-__device__ __forceinline__ double fth_arg(double tl, double hd, double se)
-{
-    return (-hd + se * tl) / (RGAS * 1.e-3 * tl);
-}
-__device__ __forceinline__ double ft(double tl, double ha) { return cm_exp(ft_arg(tl, ha)); }
-__device__ __forceinline__ double fth(double tl, double hd, double se, double scaleFactor)
-{
-    return scaleFactor / (1.0 + cm_exp(fth_arg(tl, hd, se)));
+    return (-hd + se * tl) / rt;
 }
 __device__ __forceinline__ double fth25(double hd, double se)
 {
@@ -300,11 +327,12 @@ struct CiSolve {
     double forc_pbot, cair, oair, gb_mol, je, lmr_z, par_z, rh_can;
     double vcmax_z, tpu_z, kp_z, cp, kc, ko, qe, bbb, mbb, theta_cj, theta_ip, mslope, mint;
     double ac, aj, ap, ag, an, gs_mol;
+    Recip r_cj, r_ip, r_pbot, r_gbrh;   // of theta_cj, theta_ip, forc_pbot and Medlyn's gb_mol rh_can term
     bool bad;
 };
 
 // PhotosynthesisMod.F90:2564-2701
-__device__ double ci_func(double ci, CiSolve &s)
+__device__ __forceinline__ double ci_func(double ci, CiSolve &s)
 {
     double r1, r2;
     // the C3 Rubisco rate and the C4 PEP carboxylase rate are the one divide
@@ -321,18 +349,18 @@ __device__ double ci_func(double ci, CiSolve &s)
         s.aj = s.qe * s.par_z * 4.6;
         s.ap = q;
     }
-    if (!quadratic(s.theta_cj, -(s.ac + s.aj), s.ac * s.aj, r1, r2)) s.bad = true;
+    if (!quadratic(s.theta_cj, s.r_cj, -(s.ac + s.aj), s.ac * s.aj, r1, r2)) s.bad = true;
     const double ai = fmin90(r1, r2);
-    if (!quadratic(s.theta_ip, -(ai + s.ap), ai * s.ap, r1, r2)) s.bad = true;
+    if (!quadratic(s.theta_ip, s.r_ip, -(ai + s.ap), ai * s.ap, r1, r2)) s.bad = true;
     s.ag = fmax90(0.0, fmin90(r1, r2));
     s.an = s.ag - s.lmr_z;
     if (s.an < 0.0) return 0.0;
     double cs = s.cair - 1.4 / s.gb_mol * s.an * s.forc_pbot;
     cs = fmax90(cs, MAX_CS);
     if (s.medlyn) {
-        const double term = 1.6 * s.an / (cs / s.forc_pbot * 1.e06);
+        const double term = 1.6 * s.an / (cs / s.r_pbot * 1.e06);
         const double bq = -(2.0 * (s.mint * 1.e-06 + term)
-                            + (s.mslope * term) * (s.mslope * term) / (s.gb_mol * 1.e-06 * s.rh_can));
+                            + (s.mslope * term) * (s.mslope * term) / s.r_gbrh);
         const double cq = s.mint * s.mint * 1.e-12 + (2.0 * s.mint * 1.e-06 + term * (1.0 - s.mslope * s.mslope / s.rh_can)) * term;
         if (!quadratic(1.0, bq, cq, r1, r2)) s.bad = true;
         s.gs_mol = fmax90(r1, r2) * 1.e06;
@@ -346,43 +374,45 @@ __device__ double ci_func(double ci, CiSolve &s)
 }
 
 // hybrid (PhotosynthesisMod.F90:2251-2368) with its Brent fallback (brent,
-// :2371-2485), as one loop with a single evaluation of ci_func per pass: each
-// pass evaluates ci_func at the point the previous pass chose, then the
-// stage the lane is in (the two starting points, a secant step, the Brent
-// iteration, the re-evaluation at the best point) takes the result and
-// chooses the next point or ends.  Each lane makes exactly the reference's
-// sequence of evaluations and arithmetic; lanes in different stages share the
-// evaluation (only the ci_func side effects matter to the caller).
-__device__ void hybrid(double x0, CiSolve &s)
+// :2371-2485).  Nearly every solve takes the two starting points and one secant
+// step and is done; one in sixteen, but one in most waves, goes on.  So the three
+// evaluations of ci_func are straight-line code, and what follows is one loop
+// with a single evaluation per pass: the stage a lane is in (a secant step, the
+// Brent iteration, the re-evaluation at the best point) takes the last result and
+// chooses the next point or ends, and lanes in different stages share the
+// evaluation.  Each lane makes exactly the reference's sequence of evaluations and
+// arithmetic (only the ci_func side effects matter to the caller).  As one loop
+// over all the stages a pass spent as much on moving the lanes' state between the
+// stages as on the evaluation.
+__device__ __forceinline__ void hybrid(double x0, CiSolve &s)
 {
     const double eps = 1.e-2, eps1 = 1.e-4;
-    enum { F_X0, F_X1, SECANT, BRENT, LAST };
-    int stage = F_X0, iter = 0, biter = 0;
-    double f0 = 0.0, x1 = 0.0, f1 = 0.0, minx = x0, minf = 0.0, tol = 0.0;
+    double f0 = ci_func(x0, s);
+    if (f0 == 0.0) return;
+    double minx = x0, minf = f0;
+    double x1 = x0 * 0.99;
+    double f1 = ci_func(x1, s);
+    if (f1 == 0.0) return;
+    if (f1 < minf) {
+        minx = x1;
+        minf = f1;
+    }
+    double dx = -f1 * (x1 - x0) / (f1 - f0);
+    double x = x1 + dx;
+    double tol = fabs(x) * eps;
+    if (fabs(dx) < tol) return;
+    x0 = x1;
+    f0 = f1;
+    x1 = x;
+    double f = ci_func(x1, s);
+
+    enum { SECANT, BRENT, LAST };
+    int stage = SECANT, iter = 1, biter = 0;
     double a = 0.0, b = 0.0, c = 0.0, fa = 0.0, fb = 0.0, fc = 0.0, d = 0.0, e = 0.0;
-    double xe = x0;
     for (;;) {
-        const double f = ci_func(xe, s);
-        bool secant_next = false, brent_next = false;
-        if (stage == F_X0) {
-            f0 = f;
-            if (f0 == 0.0) return;
-            minx = x0;
-            minf = f0;
-            x1 = x0 * 0.99;
-            xe = x1;
-            stage = F_X1;
-            continue;
-        } else if (stage == F_X1) {
-            f1 = f;
-            if (f1 == 0.0) return;
-            if (f1 < minf) {
-                minx = x1;
-                minf = f1;
-            }
-            iter = 1;
-            secant_next = true;
-        } else if (stage == SECANT) {
+        double xe;
+        bool brent = false;
+        if (stage == SECANT) {
             f1 = f;
             if (f1 < minf) {
                 minx = x1;
@@ -390,97 +420,89 @@ __device__ void hybrid(double x0, CiSolve &s)
             }
             if (fabs(f1) <= eps1) return;
             if (f1 * f0 < 0.0) {
-                // brent(x0, x1, f0, f1, tol): the bracket and its first state
+                // brent(x0, x1, f0, f1, tol): the bracket, the signs opposite
                 a = x0;
                 b = x1;
                 fa = f0;
                 fb = f1;
-                if ((fa > 0.0 && fb > 0.0) || (fa < 0.0 && fb < 0.0)) {
-                    s.bad = true;
-                    return;
-                }
                 c = b;
                 fc = fb;
-                biter = 0;
-                brent_next = true;
+                brent = true;
             } else if (iter > 40) {
                 xe = minx;
                 stage = LAST;
-                continue;
             } else {
                 ++iter;
-                secant_next = true;
+                dx = -f1 * (x1 - x0) / (f1 - f0);
+                x = x1 + dx;
+                tol = fabs(x) * eps;
+                if (fabs(dx) < tol) return;
+                x0 = x1;
+                f0 = f1;
+                x1 = x;
+                xe = x1;
             }
         } else if (stage == BRENT) {
             fb = f;
             if (fb == 0.0) return;
             ++biter;
-            brent_next = true;
+            brent = true;
         } else {
             return;     // LAST: ci_func at the best point has run
         }
-        if (secant_next) {
-            const double dx = -f1 * (x1 - x0) / (f1 - f0);
-            const double x = x1 + dx;
-            tol = fabs(x) * eps;
-            if (fabs(dx) < tol) return;
-            x0 = x1;
-            f0 = f1;
-            x1 = x;
-            xe = x1;
-            stage = SECANT;
-            continue;
-        }
-        // one Brent iteration up to its evaluation of ci_func
-        if (biter >= 20) return;
-        if ((fb > 0.0 && fc > 0.0) || (fb < 0.0 && fc < 0.0)) {
-            c = a;
-            fc = fa;
-            d = b - a;
-            e = d;
-        }
-        if (fabs(fc) < fabs(fb)) {
-            a = b;
-            b = c;
-            c = a;
-            fa = fb;
-            fb = fc;
-            fc = fa;
-        }
-        const double tol1 = 2.0 * eps * fabs(b) + 0.5 * tol;
-        const double xm = 0.5 * (c - b);
-        if (fabs(xm) <= tol1 || fb == 0.0) return;
-        if (fabs(e) >= tol1 && fabs(fa) > fabs(fb)) {
-            const double ss = fb / fa;
-            double p, q;
-            if (a == c) {
-                p = 2.0 * xm * ss;
-                q = 1.0 - ss;
-            } else {
-                q = fa / fc;
-                const double r = fb / fc;
-                p = ss * (2.0 * xm * q * (q - r) - (b - a) * (r - 1.0));
-                q = (q - 1.0) * (r - 1.0) * (ss - 1.0);
-            }
-            if (p > 0.0) q = -q;
-            p = fabs(p);
-            if (2.0 * p < fmin90(3.0 * xm * q - fabs(tol1 * q), fabs(e * q))) {
+        if (brent) {
+            // one Brent iteration up to its evaluation of ci_func
+            if (biter >= 20) return;
+            if ((fb > 0.0 && fc > 0.0) || (fb < 0.0 && fc < 0.0)) {
+                c = a;
+                fc = fa;
+                d = b - a;
                 e = d;
-                d = p / q;
+            }
+            if (fabs(fc) < fabs(fb)) {
+                a = b;
+                b = c;
+                c = a;
+                fa = fb;
+                fb = fc;
+                fc = fa;
+            }
+            const double tol1 = 2.0 * eps * fabs(b) + 0.5 * tol;
+            const double xm = 0.5 * (c - b);
+            if (fabs(xm) <= tol1 || fb == 0.0) return;
+            if (fabs(e) >= tol1 && fabs(fa) > fabs(fb)) {
+                const double ss = fb / fa;
+                double p, q;
+                if (a == c) {
+                    p = 2.0 * xm * ss;
+                    q = 1.0 - ss;
+                } else {
+                    q = fa / fc;
+                    const double r = fb / fc;
+                    p = ss * (2.0 * xm * q * (q - r) - (b - a) * (r - 1.0));
+                    q = (q - 1.0) * (r - 1.0) * (ss - 1.0);
+                }
+                if (p > 0.0) q = -q;
+                p = fabs(p);
+                if (2.0 * p < fmin90(3.0 * xm * q - fabs(tol1 * q), fabs(e * q))) {
+                    e = d;
+                    d = p / q;
+                } else {
+                    d = xm;
+                    e = d;
+                }
             } else {
                 d = xm;
                 e = d;
             }
-        } else {
-            d = xm;
-            e = d;
+            a = b;
+            fa = fb;
+            if (fabs(d) > tol1) b = b + d;
+            else b = b + copysign(fabs(tol1), xm);
+            xe = b;
+            stage = BRENT;
         }
-        a = b;
-        fa = fb;
-        if (fabs(d) > tol1) b = b + d;
-        else b = b + copysign(fabs(tol1), xm);
-        xe = b;
-        stage = BRENT;
+        f = ci_func(xe, s);
     }
 }
 
@@ -504,22 +526,31 @@ struct TFac {
 // constants of the step for one patch
 struct PsnConst {
     bool c3;
-    double bbb, mbb, qe, lnc, vcmax25top, jmax25top, tpu25top, kp25top, lmr25top, lmrc;
-    double vcmaxse, jmaxse, tpuse, vcmaxc, jmaxc, tpuc, kc25, ko25, cp25;
+    double bbb, mbb, qe, lnc, vcmax25top, jmax25top, tpu25top, kp25top, lmr25top;
+    double t10c, vcmaxse, jmaxse, tpuse, vcmaxc, jmaxc, tpuc, kc25, ko25, cp25;
     double theta_cj, mslope, mint;
 };
 
+// Element `byte` bytes into an array, as a base in scalar registers and a 32-bit
+// offset (a patch or column array without levels is far below 4 GiB: the state of
+// 2^29 patches would not fit the card).
+template <class T>
+__device__ __forceinline__ T &at(T *base, uint32_t byte)
+{
+    return *(T *)((char *)base + byte);
+}
+
 // PhotosynthesisMod.F90:1243-2062 for one patch and one phase.
 template <class PRM>
-__device__ void photosynthesis(const CSwitch &sw, const PRM &P, const PsnConst &K, const TFac &T,
-                               int nrad, double par_z, double lai_z, double vcmaxcint, double o3v, double o3g,
-                               bool noon, double forc_pbot, double tgcm, double esat_tv, double eair, double oair,
+__device__ __forceinline__ void photosynthesis(const CSwitch &sw, const PRM &P, const PsnConst &K, const TFac &T,
+                               int nrad, double par_z, const double *lai_z_p, const double *vcmaxcint,
+                               const double *o3v, const double *o3g, uint32_t po, bool noon, double forc_pbot, double tgcm, double esat_tv, double eair, double oair,
                                double cair, double rb, double btran, Phase &ph, Shared &sh, bool &bad)
 {
     const bool medlyn = sw.stomatal == CTSM_STOMATA_MEDLYN2011;
     double jmax_z = 0.0;
     if (nrad >= 1) {
-        const double nscaler = vcmaxcint;
+        const double nscaler = at(vcmaxcint, po);
         const double lmr25 = K.lmr25top * nscaler;
         if (K.c3) {
             ph.lmr_z = lmr25 * T.ftL * T.fthL;
@@ -613,6 +644,10 @@ __device__ void photosynthesis(const CSwitch &sw, const PRM &P, const PsnConst &
             s.ag = sh.ag;
             s.an = sh.an;
             s.gs_mol = sh.gs_mol;
+            s.r_cj = recip(s.theta_cj);
+            s.r_ip = recip(s.theta_ip);
+            s.r_pbot = recip(forc_pbot);
+            s.r_gbrh = recip(s.gb_mol * 1.e-06 * rh_can);
             s.bad = false;
             hybrid(ci0, s);
             if (s.bad) bad = true;
@@ -631,9 +666,9 @@ __device__ void photosynthesis(const CSwitch &sw, const PRM &P, const PsnConst &
             ph.ci_z = fmax90(ph.ci_z, 1.e-06);
             const double gs = gs_mol / cf;
             ph.rs_z = fmin90(1.0 / gs, rsmax0);
-            ph.rs_z = ph.rs_z / o3g;
+            ph.rs_z = ph.rs_z / at(o3g, po);
             ph.psn_z = sh.ag;
-            ph.psn_z = ph.psn_z * o3v;
+            ph.psn_z = ph.psn_z * at(o3v, po);
             if (sh.ac <= sh.aj && sh.ac <= sh.ap) psn_wc_z = ph.psn_z;
             else if (sh.aj < sh.ac && sh.aj <= sh.ap) psn_wj_z = ph.psn_z;
             else if (sh.ap < sh.ac && sh.ap < sh.aj) psn_wp_z = ph.psn_z;
@@ -643,6 +678,7 @@ __device__ void photosynthesis(const CSwitch &sw, const PRM &P, const PsnConst &
     }
     double psncan = 0.0, psncan_wc = 0.0, psncan_wj = 0.0, psncan_wp = 0.0, lmrcan = 0.0, gscan = 0.0, laican = 0.0;
     if (nrad >= 1) {
+        const double lai_z = at(lai_z_p, po);
         psncan = psncan + ph.psn_z * lai_z;
         psncan_wc = psncan_wc + psn_wc_z * lai_z;
         psncan_wj = psncan_wj + psn_wj_z * lai_z;
@@ -680,13 +716,10 @@ namespace canopy {
 // phs: PhotosynthesisHydraulicStress's constants (:3117-3300): the
 // Ball-Berry minimum conductance without btran (the stress enters through
 // bsun / bsha) and the top-leaf nitrogen capped at 10 g/m2
-template <class PRM>
-__device__ void psn_constants(const CSwitch &sw, const PRM &P, const double *__restrict__ pft, int ivt,
-                              double forc_pbot, double oair, double t10, double btran, double dayl_factor,
-                              PsnConst &K, bool &bad, bool phs = false)
+__device__ __forceinline__ void psn_static(const CSwitch &sw, const double *__restrict__ pft, int ivt, double btran,
+                                           PsnConst &K, bool &bad, bool phs)
 {
     const bool medlyn = sw.stomatal == CTSM_STOMATA_MEDLYN2011;
-    K.lmrc = fth25(P.lmrhd, P.lmrse);
     K.c3 = ((int)rint(pft[F_C3PSN * CTSM_MAX_PFT + ivt]) == 1);
     double bbbopt = 0.0;
     if (K.c3) {
@@ -698,24 +731,39 @@ __device__ void psn_constants(const CSwitch &sw, const PRM &P, const double *__r
     }
     K.bbb = phs ? bbbopt : fmax90(bbbopt * btran, 1.0);
     K.mbb = pft[F_MBBOPT * CTSM_MAX_PFT + ivt];
-    K.kc25 = P.kc25_coef * forc_pbot;
-    K.ko25 = P.ko25_coef * forc_pbot;
-    const double sco = 0.5 * 0.209 / P.cp25_yr2000;
-    K.cp25 = 0.5 * oair / sco;
     const double slatop = pft[F_SLATOP * CTSM_MAX_PFT + ivt], leafcn = pft[F_LEAFCN * CTSM_MAX_PFT + ivt];
     if (slatop * leafcn <= 0.0) bad = true;
     K.lnc = 1.0 / (slatop * leafcn);
     if (phs) K.lnc = fmin90(K.lnc, 10.0);
-    K.vcmax25top = K.lnc * pft[F_FLNR * CTSM_MAX_PFT + ivt] * P.fnr * P.act25 * dayl_factor;
-    K.vcmax25top = K.vcmax25top * pft[F_FNITR * CTSM_MAX_PFT + ivt];
-    const double t10c = fmin90(fmax90(t10 - TFRZ, 11.0), 35.0);
-    K.jmax25top = ((2.59 - 0.035 * t10c) * K.vcmax25top) * P.jmax25top_sf;
+}
+
+// those that follow from vcmax25top, t10c and the forcing
+template <class PRM>
+__device__ __forceinline__ void psn_derive(const PRM &P, double forc_pbot, double oair, PsnConst &K)
+{
+    K.kc25 = P.kc25_coef * forc_pbot;
+    K.ko25 = P.ko25_coef * forc_pbot;
+    const double sco = 0.5 * 0.209 / P.cp25_yr2000;
+    K.cp25 = 0.5 * oair / sco;
+    K.jmax25top = ((2.59 - 0.035 * K.t10c) * K.vcmax25top) * P.jmax25top_sf;
     K.tpu25top = P.tpu25ratio * K.vcmax25top;
     K.kp25top = P.kp25ratio * K.vcmax25top;
     K.lmr25top = K.c3 ? K.vcmax25top * P.leaf_mr_vcm : K.vcmax25top * 0.025;
-    K.vcmaxse = (668.39 - 1.07 * t10c) * P.vcmaxse_sf;
-    K.jmaxse = (659.70 - 0.75 * t10c) * P.jmaxse_sf;
-    K.tpuse = (668.39 - 1.07 * t10c) * P.tpuse_sf;
+    K.vcmaxse = (668.39 - 1.07 * K.t10c) * P.vcmaxse_sf;
+    K.jmaxse = (659.70 - 0.75 * K.t10c) * P.jmaxse_sf;
+    K.tpuse = (668.39 - 1.07 * K.t10c) * P.tpuse_sf;
+}
+
+template <class PRM>
+__device__ void psn_constants(const CSwitch &sw, const PRM &P, const double *__restrict__ pft, int ivt,
+                              double forc_pbot, double oair, double t10, double btran, double dayl_factor,
+                              PsnConst &K, bool &bad, bool phs = false)
+{
+    psn_static(sw, pft, ivt, btran, K, bad, phs);
+    K.vcmax25top = K.lnc * pft[F_FLNR * CTSM_MAX_PFT + ivt] * P.fnr * P.act25 * dayl_factor;
+    K.vcmax25top = K.vcmax25top * pft[F_FNITR * CTSM_MAX_PFT + ivt];
+    K.t10c = fmin90(fmax90(t10 - TFRZ, 11.0), 35.0);
+    psn_derive(P, forc_pbot, oair, K);
     K.vcmaxc = fth25(P.vcmaxhd, K.vcmaxse);
     K.jmaxc = fth25(P.jmaxhd, K.jmaxse);
     K.tpuc = fth25(P.tpuhd, K.tpuse);
@@ -724,58 +772,72 @@ __device__ void psn_constants(const CSwitch &sw, const PRM &P, const double *__r
     K.mint = pft[F_MEDINT * CTSM_MAX_PFT + ivt];
 }
 
-template <class PRM>
-__device__ void temp_factors(const PRM &P, const PsnConst &K, double tv, bool anyday, TFac &T)
+// The leaf-temperature factors of one iteration.  All twelve exponentials are
+// straight-line code on every lane's own arguments, so they run through each
+// other: C3 and C4 lanes share a wave, each with its own pathway's argument where
+// both have a factor; a factor its lane does not need is computed and ignored.
+template <class PRM, class DRV>
+__device__ __forceinline__ void temp_factors(const PRM &P, const DRV &D, const PsnConst &K, double tv, bool anyday,
+                                             TFac &T)
 {
-    T.kc = K.kc25 * ft(tv, P.kcha);
-    T.ko = K.ko25 * ft(tv, P.koha);
-    T.cp = K.cp25 * ft(tv, P.cpha);
+    const double t25 = 1.0 - (TFRZ + 25.0) / tv;
+    const Recip rt = recip(RGAS * 1.e-3 * tv);
+    const double e_kc = cm_exp(D.kcha * t25), e_ko = cm_exp(D.koha * t25), e_cp = cm_exp(D.cpha * t25);
     T.pow2 = cm_pow(2.0, (tv - (TFRZ + 25.0)) / 10.0);
-    // C3 and C4 lanes share a wave: the exponentials of the two pathways'
-    // factors are evaluated once, each lane on its own pathway's argument
-    const double eL = cm_exp(K.c3 ? ft_arg(tv, P.lmrha) : 1.3 * (tv - (TFRZ + 55.0)));
-    if (K.c3) {
-        T.ftL = eL;
-        T.fthL = fth(tv, P.lmrhd, P.lmrse, K.lmrc);
-    } else {
-        T.dL4 = 1.0 + eL;
-    }
+    const double eL = cm_exp(K.c3 ? D.lmrha * t25 : 1.3 * (tv - (TFRZ + 55.0)));
+    const double eLh = cm_exp(fth_arg(tv, rt, P.lmrhd, P.lmrse));
+    T.kc = K.kc25 * e_kc;
+    T.ko = K.ko25 * e_ko;
+    T.cp = K.cp25 * e_cp;
+    T.ftL = eL;
+    T.fthL = D.lmrc / (1.0 + eLh);
+    T.dL4 = 1.0 + eL;
     if (anyday) {
-        const double eV1 = cm_exp(K.c3 ? ft_arg(tv, P.vcmaxha) : 0.2 * ((TFRZ + 15.0) - tv));
-        const double eV2 = cm_exp(K.c3 ? fth_arg(tv, P.vcmaxhd, K.vcmaxse) : 0.3 * (tv - (TFRZ + 40.0)));
-        if (K.c3) {
-            T.ftV = eV1;
-            T.fthV = K.vcmaxc / (1.0 + eV2);
-        } else {
-            T.dV1 = 1.0 + eV1;
-            T.dV2 = 1.0 + eV2;
-        }
-        T.ftJ = ft(tv, P.jmaxha);
-        T.fthJ = fth(tv, P.jmaxhd, K.jmaxse, K.jmaxc);
-        T.ftT = ft(tv, P.tpuha);
-        T.fthT = fth(tv, P.tpuhd, K.tpuse, K.tpuc);
+        const double eV1 = cm_exp(K.c3 ? D.vcmaxha * t25 : 0.2 * ((TFRZ + 15.0) - tv));
+        const double eV2 = cm_exp(K.c3 ? fth_arg(tv, rt, P.vcmaxhd, K.vcmaxse) : 0.3 * (tv - (TFRZ + 40.0)));
+        const double eJ = cm_exp(D.jmaxha * t25), eJh = cm_exp(fth_arg(tv, rt, P.jmaxhd, K.jmaxse));
+        const double eT = cm_exp(D.tpuha * t25), eTh = cm_exp(fth_arg(tv, rt, P.tpuhd, K.tpuse));
+        T.ftV = eV1;
+        T.fthV = K.vcmaxc / (1.0 + eV2);
+        T.dV1 = 1.0 + eV1;
+        T.dV2 = 1.0 + eV2;
+        T.ftJ = eJ;
+        T.fthJ = K.jmaxc / (1.0 + eJh);
+        T.ftT = eT;
+        T.fthT = K.tpuc / (1.0 + eTh);
     }
 }
 
 #define PF(f) pft[(f) * CTSM_MAX_PFT + ivt]
 
-// Iteration state of a patch carried between rounds, indexed by the patch's
-// position in the filter (structure of arrays).
+// What a patch keeps between the kernels of a call, indexed by its position in
+// the filter (structure of arrays).  Between rounds: the iteration state.  Once it
+// has finished: what the outputs are formed from and no output array holds --
+// FrictionVelocity's last um, obu and fm, temp1 in qsatl, temp2 in el, the leaf
+// temperature before the last step in t_veg and the step in del, rpp in efeb, wtgq
+// in qsatldT.  itlef: the iterations done, -1 for a patch whose set-up failed.
 struct CanopyWork {
-    double *t_veg, *del, *efeb, *obuold, *nmozsgn, *um, *obu, *fm, *qsatl, *el, *qsatldT, *taf, *qaf, *delq,
-        *itlef, *gs_mol;
+    double *t_veg, *del, *efeb, *nmozsgn, *um, *obu, *fm, *qsatl, *el, *qsatldT, *taf, *qaf, *delq, *itlef, *gs_mol,
+        *unused;
 };
 constexpr int N_WORK_FIELDS = 16;
 static_assert(sizeof(CanopyWork) == N_WORK_FIELDS * sizeof(double *), "one pointer per saved value");
 
-// One patch of CanopyFluxes for at most `budget` leaf-temperature
-// iterations.  first: the time step's set-up runs (root stress, roughness,
-// Monin-Obukhov initialisation); otherwise the iteration state is restored
-// from W.  Returns true when the patch is still iterating (its state saved in
-// W[i0]); false when it finished (outputs written) or failed.
-// PHS: CanopyFluxes with plant hydraulic stress, H its PhsArgs (unused
-// otherwise): PhotosynthesisHydraulicStress in place of the two Photosynthesis
-// calls and the branches of CanopyFluxesMod.F90:1219-1230, 1353-1356.
+// CanopyFluxes runs as three kernels over the filter's patches, a patch per lane:
+// the set-up (canopy_setup_patch: root stress, roughness, Monin-Obukhov
+// initialisation), the rounds of the leaf-temperature iteration
+// (canopy_iterate_patch), and the fluxes and outputs of the step
+// (canopy_finish_patch).  As one kernel it held the set-up's LDS and, across the
+// iteration, everything the outputs read: one wave per SIMD, and the outputs
+// written once per round with the few lanes that had finished in it.  The
+// iteration now keeps its state only; what the outputs need of its last pass is
+// written by the passes that can be the last one (the leaf temperature had settled
+// in the pass before, or itmax is reached), each later one over the earlier.
+// All three are bound by the issue of FP64 and scalar instructions and by the waits
+// of one or two waves per SIMD; HBM is at a sixth of its rate.  On 1,048,576 columns
+// (8.9 million patches) the one kernel took 31.4 ms for its first round and 43.6 ms
+// in all; the set-up 4.1, the rounds 24.7 and the finish 2.1 ms now.
+
 // The column-level half of calc_effective_soilporosity, calc_volumetric_h2oliq
 // and calc_root_moist_stress (SoilMoistStressMod.F90:70-126, 190-240,
 // 420-514): effective porosity, volumetric liquid water and, where the level
@@ -795,17 +857,18 @@ struct SoilTerms {
     double ratio;   // eff_porosity / watsat
 };
 
-// Returns the index of the lane's run (-1 for a lane without a valid patch);
-// every lane of the wave calls it.
-template <class COL, class CAN>
-__device__ int soil_terms_of_wave(const CView &V, const COL &col, const CAN &S, const int32_t *__restrict__ filter,
-                                  int i0, bool active, SoilTerms *terms, int *run_col)
+constexpr int SOIL_RUNS = 16;     // runs whose terms are in LDS at a time
+
+// The index of the lane's run (-1 for a lane without a valid patch), the runs'
+// columns in run_col and their number; every lane of the wave calls it.
+template <class CAN>
+__device__ int runs_of_wave(const CView &V, const CAN &S, int p, bool active, int *run_col, int &nruns)
 {
     const int lane = threadIdx.x;
     int c = -1;
     if (active) {
-        // the patches canopy_patch accepts (it reports the others)
-        const long pp = V.p1(filter ? filter[i0] : V.begp + i0);
+        // the patches canopy_setup_patch accepts (it reports the others)
+        const long pp = V.p1(p);
         const int cp = S.column[pp], g = S.gridcell[pp], ivt = S.itype[pp];
         if (!(ivt < 0 || ivt >= CTSM_MAX_PFT || cp < V.begc || cp >= V.begc + V.ldc || g < V.begg ||
               g >= V.begg + V.ldg))
@@ -815,12 +878,22 @@ __device__ int soil_terms_of_wave(const CView &V, const COL &col, const CAN &S, 
     const bool lead = c >= 0 && (lane == 0 || prev != c);
     const unsigned long long leaders = __ballot(lead);
     if (lead) run_col[__popcll(leaders & ((1ull << lane) - 1ull))] = c;
+    nruns = __popcll(leaders);
     wave_sync();
+    return c >= 0 ? __popcll(leaders & ((2ull << lane) - 1ull)) - 1 : -1;
+}
+
+// The terms of runs r0 .. r0 + SOIL_RUNS - 1 into terms; every lane calls it.
+template <class COL, class CAN>
+__device__ void soil_terms_of_runs(const CView &V, const COL &col, const CAN &S, const int *run_col, int r0, int nruns,
+                                   SoilTerms *terms, const double *lt)
+{
     const int nl = V.nlevgrnd;
-    const int items = __popcll(leaders) * nl;
-    for (int it = lane; it < items; it += 64) {
+    const int items = min(nruns - r0, SOIL_RUNS) * nl;
+    wave_sync();
+    for (int it = threadIdx.x; it < items; it += 64) {
         const int r = it / nl, j = it - r * nl + 1;
-        const int rc = run_col[r];
+        const int rc = run_col[r0 + r];
         const long cs = V.soi(rc, j), cn = V.sno(rc, j);
         const double watsat = col.watsat[cs], dz = col.dz[cn];
         const double vol_ice = fmin90(watsat, col.h2osoi_ice[cn] / (DENICE * dz));
@@ -831,47 +904,161 @@ __device__ int soil_terms_of_wave(const CView &V, const COL &col, const CAN &S, 
         SoilTerms t{__longlong_as_double(kNoUptake), 0.0};
         if (!(liqvol <= 0.0 || col.t_soisno[cn] <= TFRZ - 2.0)) {
             const double s_node = fmax90(liqvol / eff, 0.01);
-            t.smp = -col.sucsat[cs] * cm_pow(s_node, -col.bsw[cs]);
+            t.smp = -col.sucsat[cs] * cm_pow_tab(s_node, -col.bsw[cs], lt);
             t.ratio = eff / watsat;
         }
         terms[r * MAX_NLEVGRND + j - 1] = t;
     }
     wave_sync();
-    return c >= 0 ? __popcll(leaders & ((2ull << lane) - 1ull)) - 1 : -1;
 }
 
-template <bool PHS, class PRM, class COL, class CAN, class WRK, class PHA>
-__device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, const PRM &P,
-                             const double *__restrict__ pft, const COL &col, const CAN &S,
-                             int i0, const int32_t *__restrict__ filter, double dtime, ErrWord *err, bool first,
-                             int budget, const WRK &W, const PHA &H, const SoilTerms *soil, double *rr_lane,
-                             double *phs_lane)
+// Root moisture stress of one patch from its column's terms (SoilMoistStressMod.
+// F90:420-514): rresis, rootr normalised by btran (:480-500), btran.
+template <class CAN>
+__device__ __forceinline__ void root_stress(const CView &V, const CAN &S, const double *__restrict__ pft, int p, int ivt,
+                                            const SoilTerms *soil)
 {
-    const int p = filter ? filter[i0] : V.begp + i0;
+    const double smpsc = PF(F_SMPSC), smpso = PF(F_SMPSO);
+    double btran = 0.0;
+    double rr[MAX_NLEVGRND];
+#pragma unroll
+    for (int j = 0; j < MAX_NLEVGRND; ++j) rr[j] = j < V.nlevgrnd ? S.rootfr[V.soip(p, j + 1)] : 0.0;
+#pragma unroll
+    for (int j = 0; j < MAX_NLEVGRND; ++j) {
+        if (j >= V.nlevgrnd) continue;
+        const SoilTerms t = soil[j];
+        double r = 0.0;
+        if (__double_as_longlong(t.smp) != kNoUptake) {
+            double smp_node = t.smp;
+            smp_node = fmax90(smpsc, smp_node);
+            const double rres = fmin90(t.ratio * (smp_node - smpsc) / (smpso - smpsc), 1.0);
+            S.rresis[V.soip(p, j + 1)] = rres;
+            r = rr[j] * rres;
+            btran = btran + fmax90(r, 0.0);
+        }
+        rr[j] = r;
+    }
+#pragma unroll
+    for (int j = 0; j < MAX_NLEVGRND; ++j)
+        if (j < V.nlevgrnd) S.rootr[V.soip(p, j + 1)] = (btran > 0.0) ? rr[j] / btran : 0.0;
+    S.btran[V.p1(p)] = btran;
+}
+
+// The set-up of one patch after its root stress: roughness, leaf humidity,
+// initial profiles and the Monin-Obukhov initialisation.  Leaves the iteration
+// state in W; a patch that fails is reported and marked (W.itlef = -1).
+template <class PRM, class COL, class CAN, class WRK>
+__device__ __forceinline__ void canopy_setup_patch(const CView &V, const CSwitch &sw, const PRM &P,
+                                                   const double *__restrict__ pft, const COL &col, const CAN &S, int i0,
+                                                   int p, ErrWord *err, const WRK &W, const double *lt)
+{
     const long pp = V.p1(p);
     const int c = S.column[pp];
     const int g = S.gridcell[pp];
     const int ivt = S.itype[pp];
-    // indices that address other arrays must lie inside their allocations
-    if (ivt < 0 || ivt >= CTSM_MAX_PFT || c < V.begc || c >= V.begc + V.ldc || g < V.begg || g >= V.begg + V.ldg) {
-        report_error(err, p, CTSM_E_ARG);
-        return false;
-    }
     const long cc = V.c1(c), gg = V.g1(g);
-    const double btran0 = 0.0, zii = 1000.0, beta = 1.0, delmax = 1.0, dlemin = 0.1, dtmin = 0.01;
-    const int itmin = 2;
-    const double ria = 0.5;
+    bool bad = false;
+    const double elai = S.elai[pp], esai = S.esai[pp], htop = S.htop[pp];
+
+    // ---- aerodynamic parameters (CanopyFluxesMod.F90:897-943)
+    double displa = S.displa[pp], z0mv = S.z0mv[pp];
+    if (sw.z0param == CTSM_Z0_ZENGWANG2007) {
+        const double vai = fmin90(elai + esai, TLSAI_CRIT);
+        const double egvf = (1.0 - ALPHA_AERO * cm_exp(-vai)) / (1.0 - ALPHA_AERO * cm_exp(-TLSAI_CRIT));
+        displa = egvf * displa;
+        z0mv = cm_exp(egvf * cm_log_tab(z0mv, lt) + (1.0 - egvf) * cm_log_tab(S.z0mg[cc], lt));
+    } else {
+        double vai = fmax90(1.e-5, elai + esai);
+        displa = htop * (1.0 - (1.0 - cm_exp(-cm_pow_tab(CD1 * vai, 0.5, lt))) / cm_pow_tab(CD1 * vai, 0.5, lt));
+        vai = fmin90(vai, PF(F_Z0V_LAIMAX));
+        double delt = 2.0;
+        const double zc = PF(F_Z0V_C);
+        const double U_ustar_ini = cm_pow_tab(PF(F_Z0V_CS) + PF(F_Z0V_CR) * vai * 0.5, -0.5, lt) * zc * vai * 0.25;
+        double U_ustar = U_ustar_ini;
+        int guard = 0;
+        while (delt > 1.e-4) {
+            const double prev = U_ustar;
+            U_ustar = U_ustar_ini * cm_exp(prev);
+            delt = fabs(U_ustar - prev);
+            if (++guard > MAX_FIXED_POINT) { bad = true; break; }
+        }
+        U_ustar = 4.0 * U_ustar / vai / zc;
+        const double zcw = PF(F_Z0V_CW);
+        z0mv = htop * (1.0 - displa / htop) * cm_exp(-VKC * U_ustar + cm_log_tab(zcw, lt) - 1.0 + 1.0 / zcw);
+    }
+    const double z0hv = z0mv, z0qv = z0mv;
+    const double hu = S.forc_hgt_u[gg] + z0mv + displa;
+    const double ht = S.forc_hgt_t[gg] + z0hv + displa;
+    const double hq = S.forc_hgt_q[gg] + z0qv + displa;
+    S.displa[pp] = displa;
+    S.z0mv[pp] = z0mv;
+    S.z0hv[pp] = z0hv;
+    S.z0qv[pp] = z0qv;
+    S.forc_hgt_u_patch[pp] = hu;
+    S.forc_hgt_t_patch[pp] = ht;
+    S.forc_hgt_q_patch[pp] = hq;
+
+    // ---- leaf humidity, initial profiles (:945-1002)
+    const double forc_q = S.forc_q[cc], thm = S.thm[pp], qg = S.qg[cc];
+    const double fu = S.forc_u[gg], fvv = S.forc_v[gg];
+    const double ur = fmax90(P.wind_min, sqrt(fu * fu + fvv * fvv));
+    const double zldis = hu - displa;
+    const double t_veg = S.t_veg[pp];
+    double qsatl, el, qsatldT;
+    qsat(t_veg, S.forc_pbot[cc], qsatl, el, qsatldT);
+    const double taf = (col.t_grnd[cc] + thm) / 2.0;
+    const double qaf = (forc_q + qg) / 2.0;
+    const double dth = thm - taf;
+    const double dqh = forc_q - qaf;
+    const double dthv = dth * (1.0 + 0.61 * forc_q) + 0.61 * S.forc_th[cc] * dqh;
+    const int snl = col.snl[cc];
+    if (zldis < 0.0 || snl < -V.nlevsno || snl > 0) {
+        report_error(err, p, zldis < 0.0 ? ENDRUN : CTSM_E_ARG);
+        W.itlef[i0] = -1.0;
+        return;
+    }
+    // FrictionVelocityMod.F90:1158-1209
+    const double wc = 0.5;
+    double um;
+    if (dthv >= 0.0) um = fmax90(ur, 0.1);
+    else um = sqrt(ur * ur + wc * wc);
+    const double rib = GRAV * zldis * dthv / (S.thv[cc] * um * um);
+    double zeta0;
+    if (rib >= 0.0) {
+        zeta0 = rib * cm_log_tab(zldis / z0mv, lt) / (1.0 - 5.0 * fmin90(rib, 0.19));
+        zeta0 = fmin90(P.zetamaxstable, fmax90(zeta0, 0.01));
+    } else {
+        zeta0 = rib * cm_log_tab(zldis / z0mv, lt);
+        zeta0 = fmax90(-100.0, fmin90(zeta0, -0.01));
+    }
+    W.t_veg[i0] = t_veg;
+    W.del[i0] = 0.0;
+    W.efeb[i0] = 0.0;
+    W.nmozsgn[i0] = 0.0;
+    W.um[i0] = um;
+    W.obu[i0] = zldis / zeta0;
+    W.fm[i0] = 0.0;
+    W.qsatl[i0] = qsatl;
+    W.el[i0] = el;
+    W.qsatldT[i0] = qsatldT;
+    W.taf[i0] = taf;
+    W.qaf[i0] = qaf;
+    W.delq[i0] = qg - qaf;
+    W.itlef[i0] = 0.0;
+    W.gs_mol[i0] = S.gs_mol[pp];
+    if (bad) report_error(err, p, ENDRUN);
+}
+
+// Biomass heat capacities (CanopyFluxesMod.F90:717-819), step constants.
+struct Biomass {
+    double frac_rad_abs_by_stem, sa_leaf, sa_stem, sa_internal, cp_leaf, cp_stem, rstem, stem_biomass, leaf_biomass;
+};
+template <class PRM>
+__device__ __forceinline__ void biomass(const CSwitch &sw, const PRM &, const double *__restrict__ pft, int ivt,
+                                        double elai, double esai, double htop, Biomass &B)
+{
     const double k_vert = 0.1, k_cyl_vol = 1.0, k_cyl_area = 1.0, k_internal = 0.0;
     const double min_stem_diameter = 0.05, min_lai = 0.1;
-    bool bad = false;
-
-    const double elai = S.elai[pp], esai = S.esai[pp], htop = S.htop[pp];
-    const double emv = S.emv[pp], thm = S.thm[pp];
-    const double forc_pbot = S.forc_pbot[cc], forc_q = S.forc_q[cc], forc_th = S.forc_th[cc];
-    const double forc_rho = S.forc_rho[cc], thv = S.thv[cc], qg = S.qg[cc];
-    const double t_grnd = col.t_grnd[cc], emg = col.emg[cc];
-
-    // ---- biomass heat capacities (CanopyFluxesMod.F90:717-819)
     double frac_rad_abs_by_stem, sa_leaf, sa_stem, sa_internal, cp_leaf, cp_stem, rstem;
     double stem_biomass = 0.0, leaf_biomass = 0.0;
     if (sw.biomass) {
@@ -899,8 +1086,6 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
         cp_stem = stem_biomass * (CDRYBIO * (1.0 - fbw) + (fbw) * CWATER);
         cp_stem = k_cyl_vol * cp_stem;
         rstem = PF(F_RSTEM) * dbh;
-        S.leaf_biomass[pp] = leaf_biomass;
-        S.stem_biomass[pp] = stem_biomass;
     } else {
         sa_leaf = (elai + esai);
         frac_rad_abs_by_stem = 0.0;
@@ -910,204 +1095,214 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
         cp_stem = 0.0;
         rstem = 0.0;
     }
-    const double dayl = S.dayl[gg], max_dayl = S.max_dayl[gg];
-    const double dayl_factor = fmin90(1.0, fmax90(0.01, (dayl * dayl) / (max_dayl * max_dayl)));
+    B = Biomass{frac_rad_abs_by_stem, sa_leaf, sa_stem, sa_internal, cp_leaf, cp_stem, rstem, stem_biomass,
+                leaf_biomass};
+}
 
-    // ---- effective porosity, volumetric liquid water, root moisture stress
-    double btran = btran0;
-    if (!first) {
-        btran = S.btran[pp];
-    } else {
-        // rootfr * rresis waits in the lane's LDS column (rr_lane, stride 64)
-        // until btran is known; rootr is then written once, normalised
-        // (SoilMoistStressMod.F90:480-500).  A run-time level loop keeps the
-        // per-level offsets out of the kernel's uniform registers.  The
-        // column's terms (effective porosity, liquid water, the matric
-        // potential) are the wave's, in soil[] (soil_terms_of_wave).
-        const double smpsc = PF(F_SMPSC), smpso = PF(F_SMPSO);
-        for (int j = 1; j <= V.nlevgrnd; ++j) {
-            const SoilTerms t = soil[j - 1];
-            double rr = 0.0;
-            if (__double_as_longlong(t.smp) != kNoUptake) {
-                double smp_node = t.smp;
-                smp_node = fmax90(smpsc, smp_node);
-                const double rres = fmin90(t.ratio * (smp_node - smpsc) / (smpso - smpsc), 1.0);
-                S.rresis[V.soip(p, j)] = rres;
-                rr = S.rootfr[V.soip(p, j)] * rres;
-                btran = btran + fmax90(rr, 0.0);
-            }
-            rr_lane[(j - 1) * 64] = rr;
-        }
-        for (int j = 1; j <= V.nlevgrnd; ++j) {
-            const long sp = V.soip(p, j);
-            S.rootr[sp] = (btran > btran0) ? rr_lane[(j - 1) * 64] / btran : 0.0;
-        }
-        S.btran[pp] = btran;
-    }
+// The weights of the heat and the moisture equation (CanopyFluxesMod.F90:1119-1250)
+// from the resistances, as the iteration and the outputs need them.
+struct HeatWeights {
+    double wta, wtl, wtg, wtstem, wtl0, wtg0, wta0, wtstem0, wtga, wtal;
+};
+__device__ __forceinline__ HeatWeights heat_weights(double rah1, double rb, double rah2, double sa_leaf, double sa_stem,
+                                                    double rstem)
+{
+    HeatWeights w;
+    w.wta = 1.0 / rah1;
+    w.wtl = sa_leaf / rb;
+    w.wtg = 1.0 / rah2;
+    w.wtstem = sa_stem / (rstem + rb);
+    const double wtshi = 1.0 / (w.wta + w.wtl + w.wtstem + w.wtg);
+    w.wtl0 = w.wtl * wtshi;
+    w.wtg0 = w.wtg * wtshi;
+    w.wta0 = w.wta * wtshi;
+    w.wtstem0 = w.wtstem * wtshi;
+    w.wtga = w.wta0 + w.wtg0 + w.wtstem0;
+    w.wtal = w.wta0 + w.wtl0 + w.wtstem0;
+    return w;
+}
+struct MoistureWeights {
+    double wtlq, wtgq0, wtlq0, wtaq0, wtgaq, wtalq;
+};
+__device__ __forceinline__ MoistureWeights moisture_weights(double fvn, double lai, double raw1, double rb, double rpp,
+                                                            double wtgq)
+{
+    MoistureWeights w;
+    const double wtaq = fvn / raw1;
+    w.wtlq = fvn * lai / rb * rpp;
+    const double wtsqi = 1.0 / (wtaq + w.wtlq + wtgq);
+    w.wtgq0 = wtgq * wtsqi;
+    w.wtlq0 = w.wtlq * wtsqi;
+    w.wtaq0 = wtaq * wtsqi;
+    w.wtgaq = w.wtaq0 + w.wtgq0;
+    w.wtalq = w.wtaq0 + w.wtlq0;
+    return w;
+}
 
-    // ---- aerodynamic parameters (CanopyFluxesMod.F90:897-943)
-    double displa = S.displa[pp], z0mv = S.z0mv[pp];
-    if (!first) {
-        // already updated in place by the first round
-    } else if (sw.z0param == CTSM_Z0_ZENGWANG2007) {
-        const double lt = fmin90(elai + esai, TLSAI_CRIT);
-        const double egvf = (1.0 - ALPHA_AERO * cm_exp(-lt)) / (1.0 - ALPHA_AERO * cm_exp(-TLSAI_CRIT));
-        displa = egvf * displa;
-        z0mv = cm_exp(egvf * cm_log(z0mv) + (1.0 - egvf) * cm_log(S.z0mg[cc]));
-    } else {
-        double lt = fmax90(1.e-5, elai + esai);
-        displa = htop * (1.0 - (1.0 - cm_exp(-cm_pow(CD1 * lt, 0.5))) / cm_pow(CD1 * lt, 0.5));
-        lt = fmin90(lt, PF(F_Z0V_LAIMAX));
-        double delt = 2.0;
-        const double zc = PF(F_Z0V_C);
-        const double U_ustar_ini = cm_pow(PF(F_Z0V_CS) + PF(F_Z0V_CR) * lt * 0.5, -0.5) * zc * lt * 0.25;
-        double U_ustar = U_ustar_ini;
-        int guard = 0;
-        while (delt > 1.e-4) {
-            const double prev = U_ustar;
-            U_ustar = U_ustar_ini * cm_exp(prev);
-            delt = fabs(U_ustar - prev);
-            if (++guard > MAX_FIXED_POINT) { bad = true; break; }
-        }
-        U_ustar = 4.0 * U_ustar / lt / zc;
-        const double zcw = PF(F_Z0V_CW);
-        z0mv = htop * (1.0 - displa / htop) * cm_exp(-VKC * U_ustar + cm_log(zcw) - 1.0 + 1.0 / zcw);
+// The outputs of one leaf phase, and of both, in a pass that can be the last.
+// Photosynthesis writes some of them only on branches fixed for the step (nrad,
+// par, the stomatal model): they are stored under the same conditions (otherwise
+// the arrays keep their values, as in the reference); the PHS path writes some
+// itself, to arrays of its own.
+template <bool PHS, class CAN>
+__device__ __forceinline__ void store_phase(const CAN &S, uint32_t po, bool sun, const Phase &ph, int nrad, bool lit)
+{
+    if (nrad >= 1) {
+        at(sun ? S.rssun_z : S.rssha_z, po) = ph.rs_z;
+        at(sun ? S.cisun_z : S.cisha_z, po) = ph.ci_z;
+        at(sun ? S.lmrsun_z : S.lmrsha_z, po) = ph.lmr_z;
+        at(sun ? S.psnsun_z : S.psnsha_z, po) = ph.psn_z;
+        at(sun ? S.gs_mol_sun : S.gs_mol_sha, po) = ph.gs_ph;
     }
-    const double z0hv = z0mv, z0qv = z0mv;
-    const double hu = S.forc_hgt_u[gg] + z0mv + displa;
-    const double ht = S.forc_hgt_t[gg] + z0hv + displa;
-    const double hq = S.forc_hgt_q[gg] + z0qv + displa;
-    if (first) {
-        S.displa[pp] = displa;
-        S.z0mv[pp] = z0mv;
-        S.z0hv[pp] = z0hv;
-        S.z0qv[pp] = z0qv;
-        S.forc_hgt_u_patch[pp] = hu;
-        S.forc_hgt_t_patch[pp] = ht;
-        S.forc_hgt_q_patch[pp] = hq;
-    }
+    if (!PHS && lit) at(sun ? S.gs_mol_sun_ln : S.gs_mol_sha_ln, po) = ph.gs_ln;
+    at(sun ? S.rssun : S.rssha, po) = ph.rs;
+    at(sun ? S.lmrsun : S.lmrsha, po) = ph.lmr;
+    at(sun ? S.psnsun : S.psnsha, po) = ph.psn;
+    at(sun ? S.psnsun_wc : S.psnsha_wc, po) = ph.psn_wc;
+    at(sun ? S.psnsun_wj : S.psnsha_wj, po) = ph.psn_wj;
+    at(sun ? S.psnsun_wp : S.psnsha_wp, po) = ph.psn_wp;
+}
+template <bool PHS, class CAN>
+__device__ __forceinline__ void store_shared(const CAN &S, uint32_t po, const CSwitch &sw, const Shared &sh, int nrad,
+                                             double parsun, double parsha)
+{
+    at(S.gb_mol, po) = sh.gb_mol;
+    if (PHS) return;
+    at(S.gs_mol, po) = sh.gs_mol;
+    if (nrad < 1) return;
+    const bool medlyn = sw.stomatal == CTSM_STOMATA_MEDLYN2011;
+    const bool lit_sun = parsun > 0.0, lit_sha = parsha > 0.0;
+    at(S.vcmax_z, po) = sh.vcmax_z;
+    at(S.tpu_z, po) = sh.tpu_z;
+    at(S.kp_z, po) = sh.kp_z;
+    at(S.ac, po) = sh.ac;
+    at(S.aj, po) = sh.aj;
+    at(S.ap, po) = sh.ap;
+    at(S.ag, po) = sh.ag;
+    at(S.an, po) = sh.an;
+    // rh_leaf: a dark phase writes 0, a lit one under Ball-Berry its value;
+    // vpd_can: a lit phase under Medlyn (the last writer wins)
+    if (!medlyn || !lit_sun || !lit_sha) at(S.rh_leaf, po) = sh.rh_leaf;
+    if (medlyn && (lit_sun || lit_sha)) at(S.vpd_can, po) = sh.vpd_can;
+}
 
-    // ---- radiation terms, leaf humidity, initial profiles (:945-1002)
-    const double forc_lwrad = col.forc_lwrad[cc];
-    const double air = emv * (1.0 + (1.0 - emv) * (1.0 - emg)) * forc_lwrad;
-    const double bir = -(2.0 - emv * (1.0 - emg)) * emv * SB;
-    const double cir = emv * emg * SB;
-    double t_veg, qsatl, el, qsatldT, taf, qaf, dth = 0.0, dqh = 0.0, delq, um, obu;
-    int nmozsgn;
-    const double co2 = S.forc_pco2[gg], o2 = S.forc_po2[gg];
-    const double fu = S.forc_u[gg], fvv = S.forc_v[gg];
-    const double ur = fmax90(P.wind_min, sqrt(fu * fu + fvv * fvv));
-    const double zldis = hu - displa;
-    if (first) {
-        t_veg = S.t_veg[pp];
-        qsat(t_veg, forc_pbot, qsatl, el, qsatldT);
-        nmozsgn = 0;
-        taf = (t_grnd + thm) / 2.0;
-        qaf = (forc_q + qg) / 2.0;
-        dth = thm - taf;
-        dqh = forc_q - qaf;
-        delq = qg - qaf;
-        const double dthv = dth * (1.0 + 0.61 * forc_q) + 0.61 * forc_th * dqh;
-        if (zldis < 0.0) {
-            report_error(err, p, ENDRUN);
-            return false;
-        }
-        // FrictionVelocityMod.F90:1158-1209
-        const double wc = 0.5;
-        if (dthv >= 0.0) um = fmax90(ur, 0.1);
-        else um = sqrt(ur * ur + wc * wc);
-        const double rib = GRAV * zldis * dthv / (thv * um * um);
-        double zeta0;
-        if (rib >= 0.0) {
-            zeta0 = rib * cm_log(zldis / z0mv) / (1.0 - 5.0 * fmin90(rib, 0.19));
-            zeta0 = fmin90(P.zetamaxstable, fmax90(zeta0, 0.01));
-        } else {
-            zeta0 = rib * cm_log(zldis / z0mv);
-            zeta0 = fmax90(-100.0, fmin90(zeta0, -0.01));
-        }
-        obu = zldis / zeta0;
-    } else {
-        t_veg = W.t_veg[i0];
-        qsatl = W.qsatl[i0];
-        el = W.el[i0];
-        qsatldT = W.qsatldT[i0];
-        taf = W.taf[i0];
-        qaf = W.qaf[i0];
-        delq = W.delq[i0];
-        um = W.um[i0];
-        obu = W.obu[i0];
-        nmozsgn = (int)W.nmozsgn[i0];
-    }
-    const double tl_ini = S.t_veg[pp];
-    double t_stem = S.t_stem[pp];
-    const double ts_ini = t_stem;
+// Step constants of the iteration that wait in LDS ([KC_N][64], the lane's column)
+// instead of in registers: with log's table 20,104 bytes a wave, room for two waves
+// per SIMD.  Values formed from them in a few operations are formed anew.
+enum {
+    KC_T10C, KC_VCMAXC, KC_JMAXC, KC_TPUC, KC_VCMAX25, KC_STOM0, KC_STOM1, KC_THETA, KC_LM, KC_LH, KC_WVEG, KC_DLEXT,
+    KC_SALEAF, KC_SASTEM, KC_RSTEM, KC_CPL, KC_FR, KC_ZL, KC_ZT, KC_ZQ, KC_BIR, KC_RAD, KC_CIRLW, KC_UR, KC_SQDLEAF,
+    KC_H2OCAN, KC_LAI, KC_ELAI, KC_LAISUN, KC_LAISHA, KC_FDRY, KC_FWET, KC_THM, KC_TLINI, KC_TSTEM, KC_N
+};
 
-    // per-step constants of Photosynthesis
+// At most `budget` leaf-temperature iterations of one patch from the state in W.
+// Returns true when the patch is still iterating (its state saved in W); false when
+// it finished or its set-up had failed.
+// PHS: CanopyFluxes with plant hydraulic stress, H its PhsArgs (unused
+// otherwise): PhotosynthesisHydraulicStress in place of the two Photosynthesis
+// calls and the branches of CanopyFluxesMod.F90:1219-1230, 1353-1356.
+template <bool PHS, class PRM, class COL, class CAN, class WRK, class PHA, class DRV>
+__device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwitch &sw, const PRM &P,
+                             const double *__restrict__ pft, const COL &col, const CAN &S,
+                             int i0, int p, double dtime, ErrWord *err,
+                             int budget, const WRK &W, const PHA &H, const DRV &D, const double *lt, double *kc,
+                             double *phs_lane)
+{
+    const double it_done = W.itlef[i0];
+    if (it_done < 0.0) return false;
+    const long pp = V.p1(p);
+    const int c = S.column[pp];
+    const int g = S.gridcell[pp];
+    const int ivt = S.itype[pp];
+    const long cc = V.c1(c), gg = V.g1(g);
+    const double btran0 = 0.0, zii = 1000.0, beta = 1.0, delmax = 1.0, dlemin = 0.1, dtmin = 0.01;
+    const int itmin = 2;
+    const double ria = 0.5;
+    bool bad = false;
+
+    // ---- the step's constants
     const int nrad = S.nrad[pp];
     const double parsun = S.parsun_z[pp], parsha = S.parsha_z[pp];
     const bool noon = S.near_local_noon[gg] != 0;
     const bool anyday = nrad >= 1 && (parsun > 0.0 || parsha > 0.0);
-    const double lai_z_sun = S.laisun_z[pp], lai_z_sha = S.laisha_z[pp];
-    const double vcint_sun = S.vcmaxcintsun[pp], vcint_sha = S.vcmaxcintsha[pp];
-    const double o3v_sun = S.o3coefvsun[pp], o3v_sha = S.o3coefvsha[pp];
-    const double o3g_sun = S.o3coefgsun[pp], o3g_sha = S.o3coefgsha[pp];
-    PsnConst K;
-    psn_constants(sw, P, pft, ivt, forc_pbot, o2, S.t_a10[pp], btran, dayl_factor, K, bad, PHS);
-    // The iteration carries only its state from one iteration to the next
-    // (and, through W, from round to round); every value the outputs read
-    // after the last iteration is that iteration's own, so nothing else stays
-    // live across the loop.  Photosynthesis writes some of its outputs only
-    // on branches fixed for the step (nrad, par, the stomatal model): those
-    // are stored under the same conditions (otherwise the arrays keep their
-    // values, as in the reference).
-    double gs_mol_c = first ? S.gs_mol[pp] : W.gs_mol[i0];
-    double del = first ? 0.0 : W.del[i0], efeb = first ? 0.0 : W.efeb[i0];
-    double obuold = first ? 0.0 : W.obuold[i0];
-    double fm_c = first ? 0.0 : W.fm[i0];
-    const double laisun = S.laisun[pp], laisha = S.laisha[pp], fdry = S.fdry[pp], fwet = S.fwet[pp];
-    const double liqcan0 = S.liqcan[pp], snocan0 = S.snocan[pp];
-    const double h2ocan = liqcan0 + snocan0;
-    const double sabv = S.sabv[pp];
-    const double fvn = (double)S.frac_veg_nosno[pp];
-    const double z0mg = S.z0mg[cc];
-    const double dleaf = PF(F_DLEAF);
-    const int snl = col.snl[cc];
-    if (snl < -V.nlevsno || snl > 0) {
-        report_error(err, p, CTSM_E_ARG);
-        return false;
+    const bool medlyn = sw.stomatal == CTSM_STOMATA_MEDLYN2011;
+    double btran = S.btran[pp], sa_lw;
+    bool c3;
+    {
+        const double elai = S.elai[pp], esai = S.esai[pp], emv = S.emv[pp], emg = col.emg[cc];
+        Biomass B;
+        biomass(sw, P, pft, ivt, elai, esai, S.htop[pp], B);
+        kc[KC_SALEAF * 64] = B.sa_leaf;
+        kc[KC_SASTEM * 64] = B.sa_stem;
+        kc[KC_RSTEM * 64] = B.rstem;
+        kc[KC_CPL * 64] = B.cp_leaf / dtime;
+        kc[KC_FR * 64] = B.frac_rad_abs_by_stem;
+        sa_lw = B.sa_internal * emv * SB;
+        const double dayl = S.dayl[gg], max_dayl = S.max_dayl[gg];
+        const double dayl_factor = fmin90(1.0, fmax90(0.01, (dayl * dayl) / (max_dayl * max_dayl)));
+        PsnConst K;
+        psn_constants(sw, P, pft, ivt, S.forc_pbot[cc], S.forc_po2[gg], S.t_a10[pp], btran, dayl_factor, K, bad, PHS);
+        c3 = K.c3;
+        kc[KC_T10C * 64] = K.t10c;
+        kc[KC_VCMAXC * 64] = K.vcmaxc;
+        kc[KC_JMAXC * 64] = K.jmaxc;
+        kc[KC_TPUC * 64] = K.tpuc;
+        kc[KC_VCMAX25 * 64] = K.vcmax25top;
+        kc[KC_STOM0 * 64] = medlyn ? K.mslope : K.bbb;
+        kc[KC_STOM1 * 64] = medlyn ? K.mint : K.mbb;
+        kc[KC_THETA * 64] = K.theta_cj;
+        kc[KC_SQDLEAF * 64] = sqrt(PF(F_DLEAF));
+        kc[KC_H2OCAN * 64] = (S.liqcan[pp] + S.snocan[pp]) / dtime;
+        kc[KC_LAI * 64] = elai + esai;
+        kc[KC_ELAI * 64] = elai;
+        kc[KC_LAISUN * 64] = S.laisun[pp];
+        kc[KC_LAISHA * 64] = S.laisha[pp];
+        kc[KC_FDRY * 64] = S.fdry[pp];
+        kc[KC_FWET * 64] = S.fwet[pp];
+        kc[KC_THM * 64] = S.thm[pp];
+        kc[KC_TLINI * 64] = S.t_veg[pp];
+        kc[KC_TSTEM * 64] = S.t_stem[pp];
+        const double displa = S.displa[pp], z0mv = S.z0mv[pp];
+        const double hu = S.forc_hgt_u[gg] + z0mv + displa;
+        const double ht = S.forc_hgt_t[gg] + z0mv + displa;
+        const double hq = S.forc_hgt_q[gg] + z0mv + displa;
+        const double zl = hu - displa, zt = ht - displa, zq = hq - displa;
+        kc[KC_ZL * 64] = zl;
+        kc[KC_ZT * 64] = zt;
+        kc[KC_ZQ * 64] = zq;
+        kc[KC_LM * 64] = cm_log_tab(zl / z0mv, lt);
+        kc[KC_LH * 64] = cm_log_tab(zt / z0mv, lt);
+        kc[KC_WVEG * 64] = cm_exp(-(elai + esai));
+        const double lai_dl_eff = P.lai_dl * (1.0 - fmin90(col.snow_depth[cc] / P.z_dl, 1.0));
+        kc[KC_DLEXT * 64] = 1.0 - cm_exp(-lai_dl_eff);
+        const int snl = col.snl[cc];
+        const double frac_sno = col.frac_sno_eff[cc], frac_h2osfc = col.frac_h2osfc[cc];
+        const double t_top = col.t_soisno[V.sno(c, snl + 1)], t_soi1 = col.t_soisno[V.sno(c, 1)];
+        const double t_h2osfc = col.t_h2osfc[cc];
+        const double lw_grnd = (frac_sno * p4(t_top) + (1.0 - frac_sno - frac_h2osfc) * p4(t_soi1)
+                                + frac_h2osfc * p4(t_h2osfc));
+        const double air = emv * (1.0 + (1.0 - emv) * (1.0 - emg)) * col.forc_lwrad[cc];
+        const double cir = emv * emg * SB;
+        kc[KC_BIR * 64] = -(2.0 - emv * (1.0 - emg)) * emv * SB;
+        kc[KC_RAD * 64] = S.sabv[pp] + air;
+        kc[KC_CIRLW * 64] = cir * lw_grnd;
+        const double fu = S.forc_u[gg], fvv = S.forc_v[gg];
+        kc[KC_UR * 64] = fmax90(P.wind_min, sqrt(fu * fu + fvv * fvv));
     }
-    const double frac_sno = col.frac_sno_eff[cc], frac_h2osfc = col.frac_h2osfc[cc];
-    const double t_top = col.t_soisno[V.sno(c, snl + 1)], t_soi1 = col.t_soisno[V.sno(c, 1)];
-    const double t_h2osfc = col.t_h2osfc[cc];
-    const double lw_grnd = (frac_sno * p4(t_top) + (1.0 - frac_sno - frac_h2osfc) * p4(t_soi1)
-                            + frac_h2osfc * p4(t_h2osfc));
-    const double lai_dl_eff = P.lai_dl * (1.0 - fmin90(col.snow_depth[cc] / P.z_dl, 1.0));
-    // step constants of the iteration
-    const double w_veg = cm_exp(-(elai + esai));
-    const double dl_ext = 1.0 - cm_exp(-lai_dl_eff);
-    FVLogs fvlog;
-    fvlog.lm = cm_log(zldis / z0mv);
-    fvlog.lh = cm_log((ht - displa) / z0hv);
-    fvlog.lq = cm_log((hq - displa) / z0qv);
-
-    int itlef = first ? 0 : (int)W.itlef[i0];
-    // values of the iteration that the outputs read: the loop leaves for the
-    // outputs only after a whole iteration, so each holds that iteration's value
-    double ustar, temp1, temp2, tlbef, del2, ram1, rah1, raw1, uaf, rb, rah2, raw2, svpts, eah, rh_af, vpd;
-    double wtg, wtl0, wta0, wtstem0, wtga, wtal, lw_stem, lw_leaf, qflx_tran_veg, wtlq0, wtaq0, wtalq;
-    double wtgq, eflx_sh_stem, efe, dt_veg, errp, qflx_evap_veg, eflx_sh_veg, zeta, num_iter;
-    double obu_fv, um_fv;
-    FV fv;
-    TFac T;
-    Phase sun, sha;
-    Shared sh;
+    // ---- the iteration's state
+    double t_veg = W.t_veg[i0], qsatl = W.qsatl[i0], el = W.el[i0], qsatldT = W.qsatldT[i0], taf = W.taf[i0],
+           qaf = W.qaf[i0], delq = W.delq[i0], um = W.um[i0], obu = W.obu[i0];
+    int nmozsgn = (int)W.nmozsgn[i0];
+    double gs_mol_c = W.gs_mol[i0];
+    double del = W.del[i0], efeb = W.efeb[i0], fm_c = W.fm[i0];
+    int itlef = (int)it_done;
+    const uint32_t po0 = (uint32_t)pp * 8u, co0 = (uint32_t)cc * 8u, go0 = (uint32_t)gg * 8u;
     for (int it = 0;; ++it) {
         if (it >= budget) {
             // still iterating: keep the state for the next round
             W.t_veg[i0] = t_veg;
             W.del[i0] = del;
             W.efeb[i0] = efeb;
-            W.obuold[i0] = obuold;
             W.nmozsgn[i0] = (double)nmozsgn;
             W.um[i0] = um;
             W.obu[i0] = obu;
@@ -1123,90 +1318,147 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
             if (bad) report_error(err, p, ENDRUN);
             return true;
         }
-        wtgq = 0.0;
+        // whether this pass can be the patch's last: a patch converges only where
+        // the pass before moved the leaf by less than dtmin too
+        const bool last = itlef >= sw.itmax || (itlef >= itmin && !(del >= dtmin));
+        // (offsets made opaque, here and before each part of the pass: the step's
+        // constants are read where they are used, not held in registers across the
+        // loop or the pass)
+#define KC(name) kc[KC_##name * 64 + k_]
+#define OPAQUE asm volatile("" : "+v"(k_), "+v"(po), "+v"(co), "+v"(go))
+        uint32_t po = po0, co = co0, go = go0;
+        int k_ = 0;
+        OPAQUE;
+        FV fv;
+        double wtgq = 0.0;
         fv.fm = fm_c;
-        friction_velocity(hu, ht, hq, displa, z0mv, z0hv, z0qv, fvlog, obu, itlef + 1, um, fv);
-        obu_fv = obu;       // the inputs of this FrictionVelocity call
-        um_fv = um;
-        ustar = fv.ustar;
-        temp1 = fv.temp1;
-        temp2 = fv.temp2;
-        tlbef = t_veg;
-        del2 = del;
-        ram1 = 1.0 / (ustar * ustar / um);
-        rah1 = 1.0 / (temp1 * ustar);
-        raw1 = 1.0 / (temp2 * ustar);
-        uaf = um * sqrt(1.0 / (ram1 * um));
-        const double uuc = fmin90(0.4, (0.03 * um / ustar));
-        const double cf = P.cv / (sqrt(uaf) * sqrt(dleaf));
-        rb = 1.0 / (cf * uaf);
-        const double w = w_veg;
-        const double csoilb = VKC / (P.a_coef * cm_pow(z0mg * uaf / NU, P.a_exp));
-        const double ri = (GRAV * htop * (taf - t_grnd)) / (taf * (uaf * uaf));
-        double csoilcn;
-        if (sw.undercanopy && (taf - t_grnd) > 0.0) {
-            const double ricsoilc = P.csoilc / (1.00 + ria * fmin90(ri, 10.0));
-            csoilcn = csoilb * w + ricsoilc * (1.0 - w);
-        } else {
-            csoilcn = csoilb * w + P.csoilc * (1.0 - w);
+        {
+            const FVLogs fvlog{KC(LM), KC(LH)};
+            friction_velocity(KC(ZL), KC(ZT), KC(ZQ), at(S.z0mv, po), fvlog, obu, itlef + 1, um, fv, lt);
         }
-        rah2 = sw.biomass ? 1.0 / (csoilcn * uuc) : 1.0 / (csoilcn * uaf);
-        raw2 = rah2;
-        svpts = el;
-        eah = forc_pbot * qaf / 0.622;
-        rh_af = eah / svpts;
-        vpd = fmax90((svpts - eah), 50.0) * 0.001;
+        const double ustar = fv.ustar, temp1 = fv.temp1, temp2 = fv.temp2;
+        const double tlbef = t_veg;
+        const double del2 = del;
+        const double ram1 = 1.0 / (ustar * ustar / um);
+        const double rah1 = 1.0 / (temp1 * ustar);
+        const double raw1 = 1.0 / (temp2 * ustar);
+        const double uaf = um * sqrt(1.0 / (ram1 * um));
+        const double uuc = fmin90(0.4, (0.03 * um / ustar));
+        const double cf = P.cv / (sqrt(uaf) * KC(SQDLEAF));
+        const double rb = 1.0 / (cf * uaf);
+        const double csoilb = VKC / (P.a_coef * cm_pow_tab(at(S.z0mg, co) * uaf / NU, P.a_exp, lt));
+        double csoilcn;
+        {
+            const double w = KC(WVEG), t_grnd = at(col.t_grnd, co);
+            if (sw.undercanopy && (taf - t_grnd) > 0.0) {
+                const double ri = (GRAV * at(S.htop, po) * (taf - t_grnd)) / (taf * (uaf * uaf));
+                const double ricsoilc = P.csoilc / (1.00 + ria * fmin90(ri, 10.0));
+                csoilcn = csoilb * w + ricsoilc * (1.0 - w);
+            } else {
+                csoilcn = csoilb * w + P.csoilc * (1.0 - w);
+            }
+        }
+        const double rah2 = sw.biomass ? 1.0 / (csoilcn * uuc) : 1.0 / (csoilcn * uaf);
+        const double raw2 = rah2;
+        const double svpts = el;
+        const double eah = at(S.forc_pbot, co) * qaf / 0.622;
+        if (last) {
+            W.obu[i0] = obu;        // the inputs of this FrictionVelocity call
+            W.um[i0] = um;
+            W.fm[i0] = fv.fm;
+            W.qsatl[i0] = temp1;
+            W.el[i0] = temp2;
+            at(S.ustar, po) = ustar;
+            at(S.ram1, po) = ram1;
+            at(S.rah1, po) = rah1;
+            at(S.raw1, po) = raw1;
+            at(S.rah2, po) = rah2;
+            at(S.raw2, po) = raw2;
+            at(S.uaf, po) = uaf;
+            at(S.rb1, po) = rb;
+            at(S.rh_af, po) = eah / svpts;
+            at(S.vpd, po) = fmax90((svpts - eah), 50.0) * 0.001;
+        }
 
         // Photosynthesis, sun then shade
-        sun = Phase{};
-        sha = Phase{};
-        sh = Shared{};
+        Shared sh = Shared{};
         sh.gs_mol = gs_mol_c;
-        temp_factors(P, K, t_veg, anyday, T);
-        if constexpr (PHS) {
-            // sun and shade together; btran and the transpiration come from the hydraulics
-            btran = photosynthesis_phs(V, sw, P, K, T, H, S, p, c, ivt, nrad, noon, forc_pbot, thm, svpts, eah, o2,
-                                       co2, rb, qsatl, qaf, sun, sha, sh, bad, phs_lane);
-            S.btran[pp] = btran;
-            qflx_tran_veg = S.qflx_tran_veg[pp];
-        } else {
-            // one call site for both phases: sun (k = 0), then shade
-#pragma nounroll
-            for (int k = 0; k < 2; ++k) {
-                const bool ks = k == 0;
-                Phase ph{};
-                photosynthesis(sw, P, K, T, nrad, ks ? parsun : parsha, ks ? lai_z_sun : lai_z_sha,
-                               ks ? vcint_sun : vcint_sha, ks ? o3v_sun : o3v_sha, ks ? o3g_sun : o3g_sha, noon,
-                               forc_pbot, thm, svpts, eah, o2, co2, rb, btran, ph, sh, bad);
-                if (ks) sun = ph;
-                else sha = ph;
+        double rs_sun, rs_sha, qflx_tran_veg = 0.0;
+        {
+            OPAQUE;
+            const double o2 = at(S.forc_po2, go), co2 = at(S.forc_pco2, go), forc_pbot = at(S.forc_pbot, co);
+            const double thm = KC(THM);
+            PsnConst K;
+            K.c3 = c3;
+            K.qe = c3 ? 0.0 : 0.05;
+            K.t10c = KC(T10C);
+            K.vcmax25top = KC(VCMAX25);
+            psn_derive(P, forc_pbot, o2, K);
+            K.vcmaxc = KC(VCMAXC);
+            K.jmaxc = KC(JMAXC);
+            K.tpuc = KC(TPUC);
+            K.bbb = K.mslope = KC(STOM0);
+            K.mbb = K.mint = KC(STOM1);
+            K.theta_cj = KC(THETA);
+            TFac T;
+            temp_factors(P, D, K, t_veg, anyday, T);
+            if (last) {
+                at(S.kc, po) = T.kc;
+                at(S.ko, po) = T.ko;
+                at(S.cp, po) = T.cp;
             }
+            if constexpr (PHS) {
+                // sun and shade together; btran and the transpiration come from the hydraulics
+                Phase sun = Phase{}, sha = Phase{};
+                btran = photosynthesis_phs(V, sw, P, K, T, H, S, p, c, ivt, nrad, noon, forc_pbot, thm, svpts, eah, o2,
+                                           co2, rb, qsatl, qaf, sun, sha, sh, bad, phs_lane, lt);
+                at(S.btran, po) = btran;
+                qflx_tran_veg = at(S.qflx_tran_veg, po);
+                rs_sun = sun.rs;
+                rs_sha = sha.rs;
+                if (last) {
+                    store_phase<PHS>(S, po, true, sun, nrad, false);
+                    store_phase<PHS>(S, po, false, sha, nrad, false);
+                }
+            } else {
+                rs_sun = rs_sha = 0.0;
+                // one call site for both phases: sun (k = 0), then shade
+#pragma nounroll
+                for (int k = 0; k < 2; ++k) {
+                    const bool ks = k == 0;
+                    const double par = ks ? parsun : parsha;
+                    Phase ph{};
+                    photosynthesis(sw, P, K, T, nrad, par, ks ? S.laisun_z : S.laisha_z,
+                                   ks ? S.vcmaxcintsun : S.vcmaxcintsha, ks ? S.o3coefvsun : S.o3coefvsha,
+                                   ks ? S.o3coefgsun : S.o3coefgsha, po,
+                                   noon, forc_pbot, thm, svpts, eah, o2, co2, rb, btran, ph, sh, bad);
+                    if (ks) rs_sun = ph.rs;
+                    else rs_sha = ph.rs;
+                    if (last) store_phase<PHS>(S, po, ks, ph, nrad, nrad >= 1 && par > 0.0);
+                }
+            }
+            if (last) store_shared<PHS>(S, po, sw, sh, nrad, parsun, parsha);
         }
 
         // conductances and the leaf-temperature Newton step (:1119-1331)
-        const double wta = 1.0 / rah1;
-        const double wtl = sa_leaf / rb;
-        wtg = 1.0 / rah2;
-        const double wtstem = sa_stem / (rstem + rb);
-        const double wtshi = 1.0 / (wta + wtl + wtstem + wtg);
-        wtl0 = wtl * wtshi;
-        const double wtg0 = wtg * wtshi;
-        wta0 = wta * wtshi;
-        wtstem0 = wtstem * wtshi;
-        wtga = wta0 + wtg0 + wtstem0;
-        wtal = wta0 + wtl0 + wtstem0;
-        lw_stem = sa_internal * emv * SB * p4(t_stem);
-        lw_leaf = sa_internal * emv * SB * p4(t_veg);
+        OPAQUE;
+        const double fvn = (double)at(S.frac_veg_nosno, po / 2);
+        const double forc_rho = at(S.forc_rho, co), forc_q = at(S.forc_q, co), qg = at(S.qg, co);
+        const double t_grnd = at(col.t_grnd, co), thm = KC(THM), lai = KC(LAI), t_stem = KC(TSTEM), h2ocan_dt = KC(H2OCAN);
+        const HeatWeights hw = heat_weights(rah1, rb, rah2, KC(SALEAF), KC(SASTEM), KC(RSTEM));
+        const double lw_stem = sa_lw * p4(t_stem);
+        const double lw_leaf = sa_lw * p4(t_veg);
+        const double fdry = KC(FDRY), fwet = KC(FWET);
         double rppdry;
-        if (fdry > 0.0) rppdry = fdry * rb * (laisun / (rb + sun.rs) + laisha / (rb + sha.rs)) / elai;
+        if (fdry > 0.0) rppdry = fdry * rb * (KC(LAISUN) / (rb + rs_sun) + KC(LAISHA) / (rb + rs_sha)) / KC(ELAI);
         else rppdry = 0.0;
-        double efpot = forc_rho * ((elai + esai) / rb) * (qsatl - qaf);
+        double efpot = forc_rho * (lai / rb) * (qsatl - qaf);
         double rpp;
         if (PHS) {
             if (efpot > 0.0) {
                 if (btran > btran0) rpp = rppdry + fwet;
                 else rpp = fwet;
-                rpp = fmin90(rpp, (qflx_tran_veg + h2ocan / dtime) / efpot);
+                rpp = fmin90(rpp, (qflx_tran_veg + h2ocan_dt) / efpot);
             } else {
                 rpp = 1.0;
             }
@@ -1218,80 +1470,76 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
                 rpp = fwet;
                 qflx_tran_veg = 0.0;
             }
-            rpp = fmin90(rpp, (qflx_tran_veg + h2ocan / dtime) / efpot);
+            rpp = fmin90(rpp, (qflx_tran_veg + h2ocan_dt) / efpot);
         } else {
             rpp = 1.0;
             qflx_tran_veg = 0.0;
         }
-        const double wtaq = fvn / raw1;
-        const double wtlq = fvn * (elai + esai) / rb * rpp;
-        const double rdl = dl_ext / (0.004 * uaf);
+        const double rdl = KC(DLEXT) / (0.004 * uaf);
         // the branches' divides share one evaluation (operands per lane)
         {
             const bool lee = sw.soil_resis == CTSM_SOILRESIS_LEEPIELKE1992, sl14 = sw.soil_resis == CTSM_SOILRESIS_SL14;
             if (delq < 0.0 || lee || sl14) {
                 const bool wet = delq < 0.0;
-                const double num = (wet || !lee) ? fvn : S.soilbeta[cc] * fvn;
-                const double den = (wet || lee) ? raw2 + rdl : raw2 + S.soilresis[cc];
+                const double num = (wet || !lee) ? fvn : at(S.soilbeta, co) * fvn;
+                const double den = (wet || lee) ? raw2 + rdl : raw2 + at(S.soilresis, co);
                 wtgq = num / den;
             }
         }
-        const double wtsqi = 1.0 / (wtaq + wtlq + wtgq);
-        const double wtgq0 = wtgq * wtsqi;
-        wtlq0 = wtlq * wtsqi;
-        wtaq0 = wtaq * wtsqi;
-        const double wtgaq = wtaq0 + wtgq0;
-        wtalq = wtaq0 + wtlq0;
-        const double dc1 = forc_rho * CPAIR * wtl;
-        const double dc2 = HVAP * forc_rho * wtlq;
-        const double efsh = dc1 * (wtga * t_veg - wtg0 * t_grnd - wta0 * thm - wtstem0 * t_stem);
-        eflx_sh_stem = forc_rho * CPAIR * wtstem * ((wta0 + wtg0 + wtl0) * t_stem - wtg0 * t_grnd - wta0 * thm - wtl0 * t_veg);
-        efe = dc2 * (wtgaq * qsatl - wtgq0 * qg - wtaq0 * forc_q);
+        const MoistureWeights mw = moisture_weights(fvn, lai, raw1, rb, rpp, wtgq);
+        const double dc1 = forc_rho * CPAIR * hw.wtl;
+        const double dc2 = HVAP * forc_rho * mw.wtlq;
+        const double efsh = dc1 * (hw.wtga * t_veg - hw.wtg0 * t_grnd - hw.wta0 * thm - hw.wtstem0 * t_stem);
+        double eflx_sh_stem = forc_rho * CPAIR * hw.wtstem
+                              * ((hw.wta0 + hw.wtg0 + hw.wtl0) * t_stem - hw.wtg0 * t_grnd - hw.wta0 * thm
+                                 - hw.wtl0 * t_veg);
+        double efe = dc2 * (mw.wtgaq * qsatl - mw.wtgq0 * qg - mw.wtaq0 * forc_q);
         double erre = 0.0;
         if (efe * efeb < 0.0) {
             const double efeold = efe;
             efe = 0.1 * efeold;
             erre = efe - efeold;
         }
-        const double fr = frac_rad_abs_by_stem;
-        dt_veg = ((1.0 - fr) * (sabv + air + bir * p4(t_veg) + cir * lw_grnd)
-                  - efsh - efe - lw_leaf + lw_stem - (cp_leaf / dtime) * (t_veg - tl_ini))
-                 / ((1.0 - fr) * (-4.0 * bir * p3(t_veg)) + 4.0 * sa_internal * emv * SB * p3(t_veg)
-                    + dc1 * wtga + dc2 * wtgaq * qsatldT + cp_leaf / dtime);
+        const double fr = KC(FR), bir = KC(BIR), rad = KC(RAD), cirlw = KC(CIRLW), cpl = KC(CPL);
+        double dt_veg = ((1.0 - fr) * (rad + bir * p4(t_veg) + cirlw)
+                         - efsh - efe - lw_leaf + lw_stem - cpl * (t_veg - KC(TLINI)))
+                        / ((1.0 - fr) * (-4.0 * bir * p3(t_veg)) + 4.0 * sa_lw * p3(t_veg)
+                           + dc1 * hw.wtga + dc2 * mw.wtgaq * qsatldT + cpl);
         t_veg = tlbef + dt_veg;
         const double dels = dt_veg;
         del = fabs(dels);
-        errp = 0.0;
+        double errp = 0.0;
         if (del > delmax) {
             dt_veg = delmax * dels / del;
             t_veg = tlbef + dt_veg;
-            errp = (1.0 - fr) * (sabv + air + bir * p3(tlbef) * (tlbef + 4.0 * dt_veg) + cir * lw_grnd)
-                   - sa_internal * emv * SB * p3(tlbef) * (tlbef + 4.0 * dt_veg)
+            errp = (1.0 - fr) * (rad + bir * p3(tlbef) * (tlbef + 4.0 * dt_veg) + cirlw)
+                   - sa_lw * p3(tlbef) * (tlbef + 4.0 * dt_veg)
                    + lw_stem
-                   - (efsh + dc1 * wtga * dt_veg) - (efe + dc2 * wtgaq * qsatldT * dt_veg)
-                   - (cp_leaf / dtime) * (t_veg - tl_ini);
+                   - (efsh + dc1 * hw.wtga * dt_veg) - (efe + dc2 * mw.wtgaq * qsatldT * dt_veg)
+                   - cpl * (t_veg - KC(TLINI));
         }
-        efpot = forc_rho * ((elai + esai) / rb) * (wtgaq * (qsatl + qsatldT * dt_veg) - wtgq0 * qg - wtaq0 * forc_q);
-        qflx_evap_veg = rpp * efpot;
+        efpot = forc_rho * (lai / rb) * (mw.wtgaq * (qsatl + qsatldT * dt_veg) - mw.wtgq0 * qg - mw.wtaq0 * forc_q);
+        double qflx_evap_veg = rpp * efpot;
         if (!PHS) {
             if (efpot > 0.0 && btran > btran0) qflx_tran_veg = efpot * rppdry;
             else qflx_tran_veg = 0.0;
         }
-        const double ecidif = fmax90(0.0, qflx_evap_veg - qflx_tran_veg - h2ocan / dtime);
-        qflx_evap_veg = fmin90(qflx_evap_veg, qflx_tran_veg + h2ocan / dtime);
-        eflx_sh_veg = efsh + dc1 * wtga * dt_veg + errp + erre + HVAP * ecidif;
-        eflx_sh_stem = eflx_sh_stem + forc_rho * CPAIR * wtstem * (-wtl0 * dt_veg);
-        lw_leaf = sa_internal * emv * SB * p3(tlbef) * (tlbef + 4.0 * dt_veg);
-        qsat(t_veg, forc_pbot, qsatl, el, qsatldT);
-        taf = wtg0 * t_grnd + wta0 * thm + wtl0 * t_veg + wtstem0 * t_stem;
-        qaf = wtlq0 * qsatl + wtgq0 * qg + forc_q * wtaq0;
-        dth = thm - taf;
-        dqh = forc_q - qaf;
-        delq = wtalq * qg - wtlq0 * qsatl - wtaq0 * forc_q;
+        const double ecidif = fmax90(0.0, qflx_evap_veg - qflx_tran_veg - h2ocan_dt);
+        qflx_evap_veg = fmin90(qflx_evap_veg, qflx_tran_veg + h2ocan_dt);
+        const double eflx_sh_veg = efsh + dc1 * hw.wtga * dt_veg + errp + erre + HVAP * ecidif;
+        eflx_sh_stem = eflx_sh_stem + forc_rho * CPAIR * hw.wtstem * (-hw.wtl0 * dt_veg);
+        qsat(t_veg, at(S.forc_pbot, co), qsatl, el, qsatldT);
+        taf = hw.wtg0 * t_grnd + hw.wta0 * thm + hw.wtl0 * t_veg + hw.wtstem0 * t_stem;
+        qaf = mw.wtlq0 * qsatl + mw.wtgq0 * qg + forc_q * mw.wtaq0;
+        const double dth = thm - taf;
+        const double dqh = forc_q - qaf;
+        delq = mw.wtalq * qg - mw.wtlq0 * qsatl - mw.wtaq0 * forc_q;
         const double tstar = temp1 * dth;
         const double qstar = temp2 * dqh;
+        const double forc_th = at(S.forc_th, co), thv = at(S.thv, co);
         const double thvstar = tstar * (1.0 + 0.61 * forc_q) + 0.61 * forc_th * qstar;
-        zeta = zldis * VKC * GRAV * thvstar / ((ustar * ustar) * thv);
+        const double zldis = KC(ZL), ur = KC(UR);
+        double zeta = zldis * VKC * GRAV * thvstar / ((ustar * ustar) * thv);
         if (zeta >= 0.0) {
             zeta = fmin90(P.zetamaxstable, fmax90(zeta, 0.01));
             um = fmax90(ur, 0.1);
@@ -1299,19 +1547,19 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
             zeta = fmax90(-100.0, fmin90(zeta, -0.01));
             double wc;
             if (ustar * thvstar > 0.0) wc = 0.0;
-            else wc = beta * cm_pow(-GRAV * ustar * thvstar * zii / thv, 0.333);
+            else wc = beta * cm_pow_tab(-GRAV * ustar * thvstar * zii / thv, 0.333, lt);
             um = sqrt(ur * ur + wc * wc);
         }
+        const double obuold = itlef > 0 ? obu : 0.0;
         obu = zldis / zeta;
         if (obuold * obu < 0.0) nmozsgn = nmozsgn + 1;
         if (nmozsgn >= 4) obu = zldis / (-0.01);
-        obuold = obu;
 
         gs_mol_c = sh.gs_mol;
         fm_c = fv.fm;
         itlef = itlef + 1;
         bool converged = false;
-        num_iter = 0.0;
+        double num_iter = 0.0;
         if (itlef > itmin) {
             const double dele = fabs(efe - efeb);
             efeb = efe;
@@ -1319,17 +1567,105 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
             num_iter = (double)itlef;
             converged = det < dtmin && dele < dlemin;
         }
+        if (last) {
+            W.t_veg[i0] = tlbef;
+            W.del[i0] = dt_veg;
+            W.efeb[i0] = rpp;
+            W.qsatldT[i0] = wtgq;
+            at(S.eflx_sh_stem, po) = eflx_sh_stem;
+            at(S.eflx_sh_veg, po) = eflx_sh_veg;
+            at(S.qflx_tran_veg, po) = qflx_tran_veg;
+            at(S.qflx_evap_veg, po) = qflx_evap_veg;
+            at(S.um, po) = um;
+            at(S.obu, po) = obu;
+            at(S.taf, po) = taf;
+            at(S.qaf, po) = qaf;
+            at(S.zeta, po) = zeta;
+            at(S.num_iter, po) = num_iter;
+        }
         if (converged || itlef > sw.itmax) break;
+#undef KC
+#undef OPAQUE
     }
+    if (bad) report_error(err, p, ENDRUN);
+    return false;
+}
 
-    // ---- the last iteration is done: the fluxes and outputs of the step
-    friction_velocity_diag(hu, displa, z0mv, z0hv, z0qv, obu_fv, ur, um_fv, fv);
-    const double temp12m = fv.temp12m;
-    const double temp22m = fv.temp22m;
+// The fluxes and outputs of one patch that has finished its iteration.
+template <bool PHS, class PRM, class COL, class CAN, class WRK>
+__device__ __forceinline__ void canopy_finish_patch(const CView &V, const CSwitch &sw, const PRM &P,
+                                                    const double *__restrict__ pft, const COL &col, const CAN &S,
+                                                    int i0, int p, double dtime, const WRK &W, const double *lt)
+{
+    if (W.itlef[i0] < 0.0) return;
+    const long pp = V.p1(p);
+    const int c = S.column[pp];
+    const int g = S.gridcell[pp];
+    const int ivt = S.itype[pp];
+    const long cc = V.c1(c), gg = V.g1(g);
+    const double elai = S.elai[pp], esai = S.esai[pp], htop = S.htop[pp];
+    const double emv = S.emv[pp], emg = col.emg[cc], thm = S.thm[pp];
+    const double forc_pbot = S.forc_pbot[cc], forc_q = S.forc_q[cc], forc_rho = S.forc_rho[cc];
+    const double qg = S.qg[cc], t_grnd = col.t_grnd[cc];
+    const double fu = S.forc_u[gg], fvv = S.forc_v[gg];
+    const double laisun = S.laisun[pp], laisha = S.laisha[pp];
+    const double sabv = S.sabv[pp], dleaf = PF(F_DLEAF);
+    const double liqcan0 = S.liqcan[pp], snocan0 = S.snocan[pp];
+    const bool noon = S.near_local_noon[gg] != 0;
+    Biomass B;
+    biomass(sw, P, pft, ivt, elai, esai, htop, B);
+    if (sw.biomass) {
+        S.leaf_biomass[pp] = B.leaf_biomass;
+        S.stem_biomass[pp] = B.stem_biomass;
+    }
+    const double fr = B.frac_rad_abs_by_stem, cp_leaf = B.cp_leaf, cp_stem = B.cp_stem, stem_biomass = B.stem_biomass;
+    const double tl_ini = S.t_veg[pp];
+    double t_stem = S.t_stem[pp];
+    const double ts_ini = t_stem;
+
+    // ---- diagnostics of the last FrictionVelocity call
+    const double displa = S.displa[pp], z0mv = S.z0mv[pp];
+    const double hu = S.forc_hgt_u[gg] + z0mv + displa;
+    const double ur = fmax90(P.wind_min, sqrt(fu * fu + fvv * fvv));
+    FV fv;
+    fv.ustar = S.ustar[pp];
+    fv.fm = W.fm[i0];
+    friction_velocity_diag(hu, displa, z0mv, z0mv, z0mv, W.obu[i0], ur, W.um[i0], fv, lt);
+
+    // ---- the last pass again, from what it left
+    const double temp1 = W.qsatl[i0], temp2 = W.el[i0];
+    const double tlbef = W.t_veg[i0], dt_veg = W.del[i0];
+    const double t_veg = tlbef + dt_veg;
+    const double wtgq = W.qsatldT[i0];
+    const double ram1 = S.ram1[pp], rb = S.rb1[pp];
+    const HeatWeights hw = heat_weights(S.rah1[pp], rb, S.rah2[pp], B.sa_leaf, B.sa_stem, B.rstem);
+    const MoistureWeights mw = moisture_weights((double)S.frac_veg_nosno[pp], elai + esai, S.raw1[pp], rb, W.efeb[i0],
+                                                wtgq);
+    double qsatl, el, qsatldT;
+    qsat(t_veg, forc_pbot, qsatl, el, qsatldT);
+    const double dth = thm - S.taf[pp];
+    const double dqh = forc_q - S.qaf[pp];
+    const double delq = mw.wtalq * qg - mw.wtlq0 * qsatl - mw.wtaq0 * forc_q;
+    const double eflx_sh_veg = S.eflx_sh_veg[pp], eflx_sh_stem = S.eflx_sh_stem[pp];
+    const double qflx_evap_veg = S.qflx_evap_veg[pp], qflx_tran_veg = S.qflx_tran_veg[pp];
+    const double lw_stem = B.sa_internal * emv * SB * p4(ts_ini);
+    const double lw_leaf = B.sa_internal * emv * SB * p3(tlbef) * (tlbef + 4.0 * dt_veg);
+
+    // ---- radiation terms (:945-1002)
+    const double forc_lwrad = col.forc_lwrad[cc];
+    const double air = emv * (1.0 + (1.0 - emv) * (1.0 - emg)) * forc_lwrad;
+    const double bir = -(2.0 - emv * (1.0 - emg)) * emv * SB;
+    const double cir = emv * emg * SB;
+    const int snl = col.snl[cc];
+    const double frac_sno = col.frac_sno_eff[cc], frac_h2osfc = col.frac_h2osfc[cc];
+    const double t_top = col.t_soisno[V.sno(c, snl + 1)], t_soi1 = col.t_soisno[V.sno(c, 1)];
+    const double t_h2osfc = col.t_h2osfc[cc];
+    const double lw_grnd = (frac_sno * p4(t_top) + (1.0 - frac_sno - frac_h2osfc) * p4(t_soi1)
+                            + frac_h2osfc * p4(t_h2osfc));
+    const double temp12m = fv.temp12m, temp22m = fv.temp22m;
 
     // ---- fluxes after the iteration (:1467-1615)
-    const double fr = frac_rad_abs_by_stem;
-    errp = (1.0 - fr) * (sabv + air + bir * p3(tlbef) * (tlbef + 4.0 * dt_veg) + cir * lw_grnd)
+    const double errp = (1.0 - fr) * (sabv + air + bir * p3(tlbef) * (tlbef + 4.0 * dt_veg) + cir * lw_grnd)
            - lw_leaf + lw_stem - eflx_sh_veg - HVAP * qflx_evap_veg - ((t_veg - tl_ini) * cp_leaf / dtime);
     double dt_stem = 0.0;
     double dhsdt_canopy = 0.0;
@@ -1343,22 +1679,22 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
         dhsdt_canopy = dt_stem * cp_stem / dtime + (t_veg - tl_ini) * cp_leaf / dtime;
         t_stem = t_stem + dt_stem;
     }
-    const double delt = wtal * t_grnd - wtl0 * t_veg - wta0 * thm - wtstem0 * t_stem;
+    const double delt = hw.wtal * t_grnd - hw.wtl0 * t_veg - hw.wta0 * thm - hw.wtstem0 * t_stem;
     S.taux[pp] = -forc_rho * fu / ram1;
     S.tauy[pp] = -forc_rho * fvv / ram1;
-    S.eflx_sh_grnd[pp] = CPAIR * forc_rho * wtg * delt;
-    const double delt_snow = wtal * t_top - wtl0 * t_veg - wta0 * thm - wtstem0 * t_stem;
-    const double delt_soil = wtal * t_soi1 - wtl0 * t_veg - wta0 * thm - wtstem0 * t_stem;
-    const double delt_h2osfc = wtal * t_h2osfc - wtl0 * t_veg - wta0 * thm - wtstem0 * t_stem;
-    S.eflx_sh_snow[pp] = CPAIR * forc_rho * wtg * delt_snow;
-    S.eflx_sh_soil[pp] = CPAIR * forc_rho * wtg * delt_soil;
-    S.eflx_sh_h2osfc[pp] = CPAIR * forc_rho * wtg * delt_h2osfc;
+    S.eflx_sh_grnd[pp] = CPAIR * forc_rho * hw.wtg * delt;
+    const double delt_snow = hw.wtal * t_top - hw.wtl0 * t_veg - hw.wta0 * thm - hw.wtstem0 * t_stem;
+    const double delt_soil = hw.wtal * t_soi1 - hw.wtl0 * t_veg - hw.wta0 * thm - hw.wtstem0 * t_stem;
+    const double delt_h2osfc = hw.wtal * t_h2osfc - hw.wtl0 * t_veg - hw.wta0 * thm - hw.wtstem0 * t_stem;
+    S.eflx_sh_snow[pp] = CPAIR * forc_rho * hw.wtg * delt_snow;
+    S.eflx_sh_soil[pp] = CPAIR * forc_rho * hw.wtg * delt_soil;
+    S.eflx_sh_h2osfc[pp] = CPAIR * forc_rho * hw.wtg * delt_h2osfc;
     S.qflx_evap_soi[pp] = forc_rho * wtgq * delq;
-    const double delq_snow = wtalq * S.qg_snow[cc] - wtlq0 * qsatl - wtaq0 * forc_q;
+    const double delq_snow = mw.wtalq * S.qg_snow[cc] - mw.wtlq0 * qsatl - mw.wtaq0 * forc_q;
     S.qflx_ev_snow[pp] = forc_rho * wtgq * delq_snow;
-    const double delq_soil = wtalq * S.qg_soil[cc] - wtlq0 * qsatl - wtaq0 * forc_q;
+    const double delq_soil = mw.wtalq * S.qg_soil[cc] - mw.wtlq0 * qsatl - mw.wtaq0 * forc_q;
     S.qflx_ev_soil[pp] = forc_rho * wtgq * delq_soil;
-    const double delq_h2osfc = wtalq * S.qg_h2osfc[cc] - wtlq0 * qsatl - wtaq0 * forc_q;
+    const double delq_h2osfc = mw.wtalq * S.qg_h2osfc[cc] - mw.wtlq0 * qsatl - mw.wtaq0 * forc_q;
     S.qflx_ev_h2osfc[pp] = forc_rho * wtgq * delq_h2osfc;
     const double t_ref2m = thm + temp1 * dth * (1.0 / temp12m - 1.0 / temp1);
     S.t_ref2m[pp] = t_ref2m;
@@ -1379,8 +1715,8 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
                    + emv * (1.0 + (1.0 - emg) * (1.0 - emv)) * SB * p3(ts_ini) * (ts_ini + 4.0 * dt_stem) * fr
                    + emg * (1.0 - emv) * SB * lw_grnd);
     S.t_skin[pp] = emv * t_veg + (1.0 - emv) * sqrt(sqrt(lw_grnd));
-    const double cgrnds = S.cgrnds[pp] + CPAIR * forc_rho * wtg * wtal;
-    const double cgrndl = S.cgrndl[pp] + forc_rho * wtgq * wtalq * S.dqgdT[cc];
+    const double cgrnds = S.cgrnds[pp] + CPAIR * forc_rho * hw.wtg * hw.wtal;
+    const double cgrndl = S.cgrndl[pp] + forc_rho * wtgq * mw.wtalq * S.dqgdT[cc];
     S.cgrnds[pp] = cgrnds;
     S.cgrndl[pp] = cgrndl;
     S.cgrnd[pp] = cgrnds + cgrndl * col.htvp[cc];
@@ -1400,120 +1736,65 @@ __device__ __forceinline__ bool canopy_patch(const CView &V, const CSwitch &sw, 
     S.liqcan[pp] = liqcan;
 
     // ---- PhotosynthesisTotal and the noon water-use efficiency
-    const double fpsn = sun.psn * laisun + sha.psn * laisha;
+    const double psn_sun = S.psnsun[pp], psn_sha = S.psnsha[pp];
+    const double fpsn = psn_sun * laisun + psn_sha * laisha;
     S.fpsn[pp] = fpsn;
-    S.fpsn_wc[pp] = sun.psn_wc * laisun + sha.psn_wc * laisha;
-    S.fpsn_wj[pp] = sun.psn_wj * laisun + sha.psn_wj * laisha;
-    S.fpsn_wp[pp] = sun.psn_wp * laisun + sha.psn_wp * laisha;
+    S.fpsn_wc[pp] = S.psnsun_wc[pp] * laisun + S.psnsha_wc[pp] * laisha;
+    S.fpsn_wj[pp] = S.psnsun_wj[pp] * laisun + S.psnsha_wj[pp] * laisha;
+    S.fpsn_wp[pp] = S.psnsun_wp[pp] * laisun + S.psnsha_wp[pp] * laisha;
     double iwue = SPVAL;
-    if (noon && fpsn > 0.0) {
-        const double gs = 1.e-6 * (laisun * sun.gs_ph + laisha * sha.gs_ph);
+    if (noon && fpsn > 0.0) {       // fpsn > 0 only where nrad >= 1, whose phases have written gs_mol
+        const double gs = 1.e-6 * (laisun * S.gs_mol_sun[pp] + laisha * S.gs_mol_sha[pp]);
         iwue = (gs > 0.0) ? fpsn / gs : SPVAL;
     }
     S.iwue_ln[pp] = iwue;
 
     // ---- remaining outputs
-    S.btran[pp] = btran;
     S.dhsdt_canopy[pp] = dhsdt_canopy;
-    S.eflx_sh_stem[pp] = eflx_sh_stem;
-    S.eflx_sh_veg[pp] = eflx_sh_veg;
-    S.qflx_tran_veg[pp] = qflx_tran_veg;
-    S.qflx_evap_veg[pp] = qflx_evap_veg;
     S.t_veg[pp] = t_veg;
     S.t_stem[pp] = t_stem;
-    S.um[pp] = um;
-    S.obu[pp] = obu;
-    S.num_iter[pp] = num_iter;
-    S.ustar[pp] = ustar;
     S.u10[pp] = fv.u10;
     S.u10_clm[pp] = fv.u10_clm;
     S.va[pp] = fv.va;
     S.fv[pp] = fv.fv;
     S.vds[pp] = fv.vds;
-    S.ram1[pp] = ram1;
-    S.rb1[pp] = rb;
-    S.rah1[pp] = rah1;
-    S.rah2[pp] = rah2;
-    S.raw1[pp] = raw1;
-    S.raw2[pp] = raw2;
-    S.uaf[pp] = uaf;
-    S.taf[pp] = taf;
-    S.qaf[pp] = qaf;
-    S.zeta[pp] = zeta;
-    S.vpd[pp] = vpd;
-    S.rh_af[pp] = rh_af;
     S.dleaf_patch[pp] = dleaf;
     S.canopy_err[pp] = errp;
     // photosyns_inst
+    PsnConst K;
+    bool bad = false;       // the iteration has reported it
+    psn_static(sw, pft, ivt, PHS ? 0.0 : S.btran[pp], K, bad, PHS);
     S.c3flag[pp] = K.c3 ? 1 : 0;
     S.qe[pp] = K.qe;
     if (sw.stomatal == CTSM_STOMATA_BB1987) {
         S.bbb[pp] = K.bbb;
         S.mbb[pp] = K.mbb;
     }
-    S.kc[pp] = T.kc;
-    S.ko[pp] = T.ko;
-    S.cp[pp] = T.cp;
     S.lnca[pp] = K.lnc;
-    S.gb_mol[pp] = sh.gb_mol;
-    if (!PHS) S.gs_mol[pp] = sh.gs_mol;
-    const bool medlyn = sw.stomatal == CTSM_STOMATA_MEDLYN2011;
-    const bool lit_sun = nrad >= 1 && parsun > 0.0, lit_sha = nrad >= 1 && parsha > 0.0;
-    if (nrad >= 1) {
-        // written by both phases' canopy layer whether lit or not (the PHS
-        // path has arrays of its own for these, written as it goes)
-        if (!PHS) {
-            S.vcmax_z[pp] = sh.vcmax_z;
-            S.tpu_z[pp] = sh.tpu_z;
-            S.kp_z[pp] = sh.kp_z;
-            S.ac[pp] = sh.ac;
-            S.aj[pp] = sh.aj;
-            S.ap[pp] = sh.ap;
-            S.ag[pp] = sh.ag;
-            S.an[pp] = sh.an;
-        }
-        S.rssun_z[pp] = sun.rs_z;
-        S.rssha_z[pp] = sha.rs_z;
-        S.cisun_z[pp] = sun.ci_z;
-        S.cisha_z[pp] = sha.ci_z;
-        S.lmrsun_z[pp] = sun.lmr_z;
-        S.lmrsha_z[pp] = sha.lmr_z;
-        S.psnsun_z[pp] = sun.psn_z;
-        S.psnsha_z[pp] = sha.psn_z;
-        S.gs_mol_sun[pp] = sun.gs_ph;
-        S.gs_mol_sha[pp] = sha.gs_ph;
-        // rh_leaf: a dark phase writes 0, a lit one under Ball-Berry its
-        // value; vpd_can: a lit phase under Medlyn (the last writer wins)
-        if (!PHS && (!medlyn || !lit_sun || !lit_sha)) S.rh_leaf[pp] = sh.rh_leaf;
-        if (!PHS && medlyn && (lit_sun || lit_sha)) S.vpd_can[pp] = sh.vpd_can;
-    }
-    if (!PHS && lit_sun) S.gs_mol_sun_ln[pp] = sun.gs_ln;
-    if (!PHS && lit_sha) S.gs_mol_sha_ln[pp] = sha.gs_ln;
-    S.rssun[pp] = sun.rs;
-    S.rssha[pp] = sha.rs;
-    S.lmrsun[pp] = sun.lmr;
-    S.lmrsha[pp] = sha.lmr;
-    S.psnsun[pp] = sun.psn;
-    S.psnsha[pp] = sha.psn;
-    S.psnsun_wc[pp] = sun.psn_wc;
-    S.psnsun_wj[pp] = sun.psn_wj;
-    S.psnsun_wp[pp] = sun.psn_wp;
-    S.psnsha_wc[pp] = sha.psn_wc;
-    S.psnsha_wj[pp] = sha.psn_wj;
-    S.psnsha_wp[pp] = sha.psn_wp;
-    if (bad) report_error(err, p, ENDRUN);
-    return false;
 }
 
-// Everything one launch of k_canopy_round reads: the kernel's only argument.
+// Values of the parameters alone, formed on the host (the same operations): the
+// activation energies over rgas (tfrz + 25) and respiration's scaling at 25 C.
+struct CanopyDerived {
+    double kcha, koha, cpha, lmrha, vcmaxha, jmaxha, tpuha, lmrc;
+};
+static CanopyDerived canopy_derived(const ctsm_canopy_params &P)
+{
+    const double r25 = RGAS * 1.e-3 * (TFRZ + 25.0);
+    return CanopyDerived{P.kcha / r25,    P.koha / r25,   P.cpha / r25, P.lmrha / r25, P.vcmaxha / r25,
+                         P.jmaxha / r25, P.tpuha / r25, 1.0 + cm_exp((-P.lmrhd + P.lmrse * (TFRZ + 25.0)) / r25)};
+}
+
+// Everything one launch of the three kernels reads: a kernel's only argument.
 struct RoundArgs {
     CView V;
     CSwitch sw;
     ctsm_canopy_params P;
+    CanopyDerived D;
     const double *pft;
     ctsm_col_state col;
     ctsm_canopy_state S;
-    int n;
+    int n, pfirst;                  // patches; the first one where there is no filter
     const int32_t *filter;
     double dtime;
     ErrWord *err;
@@ -1529,62 +1810,84 @@ struct RoundArgsPhs {
 };
 #define KARG __attribute__((address_space(4)))
 
-// One round of CanopyFluxes over the patches still iterating (round 0: the
+// The arguments are read in place from the kernel-argument segment, each member
+// where it is used: loaded all at once on entry, their few hundred uniform
+// pointers would not fit the scalar registers and spill.
+#define CANOPY_VIEW(A)                                                                                             \
+    CView { (A)->V.begc, (A)->V.ldc, (A)->V.begp, (A)->V.ldp, (A)->V.begg, (A)->V.ldg, (A)->V.nlevsno,              \
+            (A)->V.nlevsoi, (A)->V.nlevgrnd }
+#define CANOPY_SWITCH(A)                                                                                           \
+    CSwitch { (A)->sw.z0param, (A)->sw.stomatal, (A)->sw.soil_resis, (A)->sw.biomass, (A)->sw.undercanopy,          \
+              (A)->sw.light_inhibit, (A)->sw.itmax }
+
+// The set-up of every patch of the filter, one wave per block.
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_canopy_setup(RoundArgs)
+{
+    const KARG RoundArgs *A = (const KARG RoundArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    __shared__ SoilTerms terms[SOIL_RUNS * MAX_NLEVGRND];
+    __shared__ int run_col[64];
+    LOG_TABLE(logt);
+    const int i0 = blockIdx.x * 64 + threadIdx.x;
+    const bool active = i0 < A->n;
+    const CView V = CANOPY_VIEW(A);
+    const int p = !active ? V.begp : A->filter ? A->filter[i0] : A->pfirst + i0;
+    int nruns;
+    const int run = runs_of_wave(V, A->S, p, active, run_col, nruns);
+    const int ivt = run >= 0 ? A->S.itype[V.p1(p)] : 0;
+    for (int r0 = 0; r0 < nruns; r0 += SOIL_RUNS) {
+        soil_terms_of_runs(V, A->col, A->S, run_col, r0, nruns, terms, logt);
+        if (run >= r0 && run < r0 + SOIL_RUNS)
+            root_stress(V, A->S, A->pft, p, ivt, terms + (run - r0) * MAX_NLEVGRND);
+    }
+    if (!active) return;
+    if (run < 0) {      // an index that addresses other arrays lies outside their allocations
+        report_error(A->err, p, CTSM_E_ARG);
+        A->W.itlef[i0] = -1.0;
+        return;
+    }
+    const CSwitch sw = CANOPY_SWITCH(A);
+    canopy_setup_patch(V, sw, A->P, A->pft, A->col, A->S, i0, p, A->err, A->W, logt);
+}
+
+// One round of the iteration over the patches still iterating (round 0: the
 // whole filter), compacting those that continue into list_out with one atomic
 // per wavefront.  Blocks are one wavefront, a patch per lane.  Round 0
 // (STRIDE false) covers the filter with its grid; later rounds (STRIDE true)
-// stride a capped grid over the round's count.
-// The argument is read in place from the kernel-argument segment, each member
-// where it is used: loaded all at once on entry, its few hundred uniform
-// pointers would not fit the scalar registers and spill.  In the striding
-// form the segment pointer is made opaque on every pass, so those loads stay
-// inside the pass instead of being hoisted in front of the loop.
-// WAVES: the register budget the kernel is compiled for (waves per SIMD);
-// above one wave the compiler spills what does not fit to scratch.  The
-// launch picks the instance (a launch shape the autotuner times).
+// stride a capped grid over the round's count; there the segment pointer is made
+// opaque on every pass, so its loads stay inside the pass instead of being
+// hoisted in front of the loop.
+// WAVES: the register budget the kernel is compiled for (waves per SIMD).  One wave
+// needs 310 registers; the two-wave instance (256, and 240 B/lane of scratch) pays
+// once a filter has a second wave for the SIMDs: launch_canopy has the rule.
 // PHS: CanopyFluxes with plant hydraulic stress (argument RoundArgsPhs).
 template <int WAVES, bool STRIDE, bool PHS = false>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
-k_canopy_round(typename std::conditional<PHS, RoundArgsPhs, RoundArgs>::type args)
+k_canopy_round(typename std::conditional<PHS, RoundArgsPhs, RoundArgs>::type)
 {
     const KARG RoundArgs *Ap = (const KARG RoundArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    __shared__ double consts[KC_N * 64];
+    LOG_TABLE(logt);
     const int round = Ap->round;
     const int count = (round == 0) ? Ap->n : *Ap->cnt_in;
     const int lane = threadIdx.x;
-    // round 0 runs the step's set-up; it is always launched with STRIDE false
-    // (the instance that holds the LDS of the soil terms)
-    const bool first = round == 0;
     for (int base = blockIdx.x * 64; base < count; base += gridDim.x * 64) {
         const KARG RoundArgs *A = Ap;
         if (STRIDE) asm volatile("" : "+s"(A));
         const int idx = base + lane;
         bool cont = false;
         int i0 = (idx < count) ? ((round == 0) ? idx : A->list_in[idx]) : 0;
-        const CView V{A->V.begc, A->V.ldc, A->V.begp, A->V.ldp, A->V.begg, A->V.ldg, A->V.nlevsno,
-                      A->V.nlevsoi, A->V.nlevgrnd};
-        const SoilTerms *soil = nullptr;
-        double *rr_lane = nullptr;
-        if constexpr (!STRIDE) {
-            if (first) {
-                __shared__ SoilTerms terms[64 * MAX_NLEVGRND];
-                __shared__ double rr[MAX_NLEVGRND * 64];
-                __shared__ int run_col[64];
-                const int run = soil_terms_of_wave(V, A->col, A->S, A->filter, i0, idx < count, terms, run_col);
-                soil = terms + (run < 0 ? 0 : run) * MAX_NLEVGRND;
-                rr_lane = rr + lane;
-            }
-        }
         if (idx < count) {
-            const CSwitch sw{A->sw.z0param, A->sw.stomatal, A->sw.soil_resis, A->sw.biomass, A->sw.undercanopy,
-                             A->sw.light_inhibit, A->sw.itmax};
+            const CView V = CANOPY_VIEW(A);
+            const CSwitch sw = CANOPY_SWITCH(A);
+            const int p = A->filter ? A->filter[i0] : A->pfirst + i0;
             if constexpr (PHS) {
                 const KARG RoundArgsPhs *B = (const KARG RoundArgsPhs *)A;
                 __shared__ double phs_soil[phs::SOIL_LDS * phs::SOIL_STRIDE];
-                cont = canopy_patch<true>(V, sw, A->P, A->pft, A->col, A->S, i0, A->filter, A->dtime, A->err,
-                                          first, A->budget, A->W, B->phs, soil, rr_lane, phs_soil + lane);
+                cont = canopy_iterate_patch<true>(V, sw, A->P, A->pft, A->col, A->S, i0, p, A->dtime, A->err,
+                                                  A->budget, A->W, B->phs, A->D, logt, consts + lane, phs_soil + lane);
             } else {
-                cont = canopy_patch<false>(V, sw, A->P, A->pft, A->col, A->S, i0, A->filter, A->dtime, A->err,
-                                           first, A->budget, A->W, *A, soil, rr_lane, nullptr);
+                cont = canopy_iterate_patch<false>(V, sw, A->P, A->pft, A->col, A->S, i0, p, A->dtime, A->err,
+                                                   A->budget, A->W, *A, A->D, logt, consts + lane, nullptr);
             }
         }
         const unsigned long long mask = __ballot(cont);
@@ -1597,6 +1900,20 @@ k_canopy_round(typename std::conditional<PHS, RoundArgsPhs, RoundArgs>::type arg
         }
         if (!STRIDE) break;
     }
+}
+
+// The outputs of every patch of the filter.
+template <bool PHS>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_canopy_finish(RoundArgs)
+{
+    const KARG RoundArgs *A = (const KARG RoundArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    LOG_TABLE(logt);
+    const int i0 = blockIdx.x * 64 + threadIdx.x;
+    if (i0 >= A->n) return;
+    const CView V = CANOPY_VIEW(A);
+    const CSwitch sw = CANOPY_SWITCH(A);
+    const int p = A->filter ? A->filter[i0] : A->pfirst + i0;
+    canopy_finish_patch<PHS>(V, sw, A->P, A->pft, A->col, A->S, i0, p, A->dtime, A->W, logt);
 }
 
 __global__ void __launch_bounds__(64) k_zero_counts(int32_t *cnt, int n)
@@ -1758,38 +2075,59 @@ __global__ void __launch_bounds__(RS_COLS *RS_GROUPS) k_root_sink_staged(CView V
 
 }  // namespace canopy
 
+constexpr int SIMDS = 1024;      // 256 CUs
+
+// Iterations of round r >= 1: round_its twice, then twice as many each time.  The
+// late rounds hold a few thousand patches at most, whose waves fit the chip at once:
+// packing them again gains nothing there and costs a launch and a cold start:
+// 20,000 columns 3391 us in 13 rounds of 3, 3133 us in 6 of 3, 3, 6, 12, 24.
+static int canopy_round_budget(int r, int round_its)
+{
+    return r <= 2 ? round_its : (int)std::min<long>((long)round_its << std::min(r - 2, 30), INT_MAX);
+}
+
 // Rounds after the first one: enough to take a patch from first_its
 // iterations to itmax + 1.
 static int canopy_later_rounds(int itmax, int first_its, int round_its)
 {
-    const int left = itmax + 1 - first_its;
-    return left > 0 ? (left + round_its - 1) / round_its : 0;
+    int r = 0;
+    for (long left = (long)itmax + 1 - first_its; left > 0; left -= canopy_round_budget(r, round_its)) ++r;
+    return r;
 }
 
-// Round buffer: N_WORK_FIELDS doubles per patch of the filter, two patch
-// lists, one counter per round.  0 when the iteration runs in one pass.
+// Work buffer: N_WORK_FIELDS doubles per patch of the filter and, where the
+// iteration runs in rounds, two patch lists and one counter per round.
 size_t canopy_work_bytes(int n, int itmax, int first_its, int round_its)
 {
     using namespace canopy;
+    if (n <= 0) return 0;
     const int R = canopy_later_rounds(itmax, first_its, round_its);
-    if (R == 0 || n <= 0) return 0;
-    return (size_t)N_WORK_FIELDS * n * sizeof(double) + 2 * (size_t)n * sizeof(int32_t) +
-           (size_t)(R + 1) * sizeof(int32_t);
+    const size_t w = (size_t)N_WORK_FIELDS * n * sizeof(double);
+    return R == 0 ? w : w + 2 * (size_t)n * sizeof(int32_t) + (size_t)(R + 1) * sizeof(int32_t);
 }
 
+// Patches a work buffer of `bytes` takes per pass where the iteration runs
+// without rounds (launch_canopy then goes over a longer filter in parts); 0 where
+// it runs in rounds, which take the whole filter at once.
+int canopy_one_pass_patches(size_t bytes, int itmax, int first_its, int round_its)
+{
+    using namespace canopy;
+    if (canopy_later_rounds(itmax, first_its, round_its) != 0) return 0;
+    const size_t m = bytes / (N_WORK_FIELDS * sizeof(double)) / 64 * 64;
+    return m > (size_t)INT_MAX ? INT_MAX : (int)m;
+}
+
+// work: canopy_work_bytes(n, ...) or, without rounds, room for `part` patches
+// (part = 0: for all).
 void launch_canopy(hipStream_t st, const ctsm_layout &L, const ctsm_config &cfg, const ctsm_canopy_params &prm,
                    const double *pft_dev, const ctsm_col_state &col, const ctsm_canopy_state &can, int n,
-                   const int32_t *filter, double dtime, ErrWord *err, void *work, int first_its, int round_its,
-                   bool zero_cgrnd, int waves, bool bounds_are_filter, const ctsm_phs_state *phs_q,
+                   const int32_t *filter, double dtime, ErrWord *err, void *work, int part, int first_its,
+                   int round_its, bool zero_cgrnd, int waves, bool bounds_are_filter, const ctsm_phs_state *phs_q,
                    const ctsm_phs_canopy_state *phs_h, const double *phs_table)
 {
     using namespace canopy;
     const GptlRange range("canflux");
     const bool hydrstress = phs_h != nullptr;
-    auto first_kernel = waves == 3 ? k_canopy_round<3, false> : waves == 2 ? k_canopy_round<2, false>
-                                                                          : k_canopy_round<1, false>;
-    auto later_kernel = waves == 3 ? k_canopy_round<3, true> : waves == 2 ? k_canopy_round<2, true>
-                                                                         : k_canopy_round<1, true>;
     CView V{L.begc_alloc, L.ldc, L.begp_alloc, L.ldp, L.begg_alloc, L.ldg, cfg.nlevsno, cfg.nlevsoi, cfg.nlevgrnd};
     CSwitch sw{cfg.z0param_method, cfg.stomatalcond_method, cfg.soil_resis_method, cfg.use_biomass_heat_storage,
                cfg.use_undercanopy_stability, cfg.light_inhibit, cfg.itmax_canopy_fluxes};
@@ -1802,51 +2140,71 @@ void launch_canopy(hipStream_t st, const ctsm_layout &L, const ctsm_config &cfg,
     if (n <= 0) return;
     if (zero_cgrnd)
         hipLaunchKernelGGL(k_zero_cgrnd, dim3((n + 255) / 256), dim3(256), 0, st, n, filter, L.begp_alloc, can);
-    const int R = work ? canopy_later_rounds(cfg.itmax_canopy_fluxes, first_its, round_its) : 0;
-    const int blocks = (n + 63) / 64;
-    RoundArgs a{V, sw, prm, pft_dev, col, can, n, filter, dtime, err, 0, 0, nullptr, nullptr, nullptr, nullptr,
-                CanopyWork{}};
-    // round 0 also runs the part of the routine before the iteration
-    const GptlRange iter_range("can_iter");
-    // the PHS form: one instance, built for one wave per SIMD
-    RoundArgsPhs b{};
-    if (hydrstress) b.phs = PhsArgs{*phs_q, *phs_h, phs_table, cfg.nlevsoi, cfg.modifyphoto_and_lmr_forcrop};
-    auto launch = [&](bool later, int grid) {
-        if (hydrstress) {
-            b.r = a;
-            if (later) hipLaunchKernelGGL((k_canopy_round<1, true, true>), dim3(grid), dim3(64), 0, st, b);
-            else hipLaunchKernelGGL((k_canopy_round<1, false, true>), dim3(grid), dim3(64), 0, st, b);
-        } else if (later) {
-            hipLaunchKernelGGL(later_kernel, dim3(grid), dim3(64), 0, st, a);
-        } else {
-            hipLaunchKernelGGL(first_kernel, dim3(grid), dim3(64), 0, st, a);
+    int R = canopy_later_rounds(cfg.itmax_canopy_fluxes, first_its, round_its);
+    if (part <= 0 || part > n) part = n;
+    for (int done = 0; done < n; done += part) {
+        const int m = n - done < part ? n - done : part;
+        const int blocks = (m + 63) / 64;
+        RoundArgs a{V, sw, prm, canopy_derived(prm), pft_dev, col, can, m, L.begp_alloc + done, filter ? filter + done : nullptr, dtime, err,
+                    0, 0, nullptr, nullptr, nullptr, nullptr, CanopyWork{}};
+        // The two-wave instance from the first block that has no SIMD to itself.  65,536
+        // columns (8,704 waves): 3380 us with one wave per SIMD, 3150 us with two; 762
+        // waves: 1469 and 1566 us.  About a quarter of the patches goes on to round 1.
+        const bool two = waves > 1 && blocks > SIMDS, two_later = waves > 1 && blocks > 4 * SIMDS;
+        auto first_kernel = two ? k_canopy_round<2, false> : k_canopy_round<1, false>;
+        auto later_kernel = two_later ? k_canopy_round<2, true> : k_canopy_round<1, true>;
+        double *w = (double *)work;
+        auto field = [&](int k) { return w + (size_t)k * m; };
+        a.W = CanopyWork{field(0), field(1), field(2),  field(3),  field(4),  field(5),  field(6),  field(7),
+                         field(8), field(9), field(10), field(11), field(12), field(13), field(14), field(15)};
+        hipLaunchKernelGGL(k_canopy_setup, dim3(blocks), dim3(64), 0, st, a);
+        {
+            const GptlRange iter_range("can_iter");
+            // the PHS form: one instance, built for one wave per SIMD
+            RoundArgsPhs b{};
+            if (hydrstress) b.phs = PhsArgs{*phs_q, *phs_h, phs_table, cfg.nlevsoi, cfg.modifyphoto_and_lmr_forcrop};
+            auto launch = [&](bool later, int grid) {
+                if (hydrstress) {
+                    b.r = a;
+                    if (later) hipLaunchKernelGGL((k_canopy_round<1, true, true>), dim3(grid), dim3(64), 0, st, b);
+                    else hipLaunchKernelGGL((k_canopy_round<1, false, true>), dim3(grid), dim3(64), 0, st, b);
+                } else if (later) {
+                    hipLaunchKernelGGL(later_kernel, dim3(grid), dim3(64), 0, st, a);
+                } else {
+                    hipLaunchKernelGGL(first_kernel, dim3(grid), dim3(64), 0, st, a);
+                }
+            };
+            if (R == 0) {
+                // one pass: every patch finishes (converged or itmax reached) in round 0
+                a.budget = cfg.itmax_canopy_fluxes + 1;
+                launch(false, blocks);
+            } else {
+                int32_t *list[2] = {(int32_t *)(w + (size_t)N_WORK_FIELDS * m), nullptr};
+                list[1] = list[0] + m;
+                int32_t *cnt = list[1] + m;
+                hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, cnt, R + 1);
+                // Where every wave has a SIMD to itself there is nothing to pack the
+                // survivors for but the lanes, and one later round takes them to the end:
+                // 35,000 patches (544 waves) 1125 us against 1231 us in the rounds below,
+                // 1088 waves 1309 and 1379, 2176 waves 1691 and 1621.
+                const bool alone = blocks <= SIMDS;
+                if (alone) R = std::min(R, 1);
+                // later rounds stride over the patches still iterating with a grid that
+                // keeps every wave slot of the chip busy
+                const int later_blocks = blocks < 8192 ? blocks : 8192;
+                for (int r = 0; r <= R; ++r) {
+                    a.round = r;
+                    a.budget = r == 0 ? first_its : alone ? cfg.itmax_canopy_fluxes + 1 : canopy_round_budget(r, round_its);
+                    a.list_in = list[(r + 1) & 1];
+                    a.cnt_in = r ? cnt + r - 1 : nullptr;
+                    a.list_out = list[r & 1];
+                    a.cnt_out = cnt + r;
+                    launch(r > 0, r == 0 ? blocks : later_blocks);
+                }
+            }
         }
-    };
-    if (R == 0) {
-        // one pass: every patch finishes (converged or itmax reached) in round 0
-        a.budget = cfg.itmax_canopy_fluxes + 1;
-        launch(false, blocks);
-        return;
-    }
-    double *w = (double *)work;
-    auto field = [&](int k) { return w + (size_t)k * n; };
-    a.W = CanopyWork{field(0), field(1), field(2),  field(3),  field(4),  field(5),  field(6),  field(7),
-                     field(8), field(9), field(10), field(11), field(12), field(13), field(14), field(15)};
-    int32_t *list[2] = {(int32_t *)(w + (size_t)N_WORK_FIELDS * n), nullptr};
-    list[1] = list[0] + n;
-    int32_t *cnt = list[1] + n;
-    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, cnt, R + 1);
-    // later rounds stride over the patches still iterating with a grid that
-    // keeps every wave slot of the chip busy
-    const int later_blocks = blocks < 8192 ? blocks : 8192;
-    for (int r = 0; r <= R; ++r) {
-        a.round = r;
-        a.budget = r == 0 ? first_its : round_its;
-        a.list_in = list[(r + 1) & 1];
-        a.cnt_in = r ? cnt + r - 1 : nullptr;
-        a.list_out = list[r & 1];
-        a.cnt_out = cnt + r;
-        launch(r > 0, r == 0 ? blocks : later_blocks);
+        if (hydrstress) hipLaunchKernelGGL(k_canopy_finish<true>, dim3(blocks), dim3(64), 0, st, a);
+        else hipLaunchKernelGGL(k_canopy_finish<false>, dim3(blocks), dim3(64), 0, st, a);
     }
 }
 

@@ -336,7 +336,7 @@ __device__ __forceinline__ double photosynthesis_phs(const CView &V, const CSwit
                                                   int ivt, int nrad, bool noon, double forc_pbot, double tgcm,
                                                   double esat_tv, double eair, double oair, double cair, double rb,
                                                   double qsatl, double qaf, Phase &sun, Phase &sha, Shared &sh,
-                                                  bool &bad, double *soil_lane)
+                                                  bool &bad, double *soil_lane, const double *lt)
 {
     const auto &H = A.H;
     const long pp = V.p1(p), cc = V.c1(c), ldp = V.ldp;
@@ -423,7 +423,7 @@ __device__ __forceinline__ double photosynthesis_phs(const CView &V, const CSwit
             s.leaf.ck[k] = A.table[(phs::T_CK + k) * CTSM_MAX_PFT + ivt];
         }
         phs::stage_soil(s.leaf, A.Q.k_soil_root + V.soip(p, 1), ldp, A.Q.smp_l + V.soi(c, 1), A.Q.z + V.sno(c, 1),
-                        V.ldc, A.nlevsoi, soil_lane);
+                        V.ldc, A.nlevsoi, soil_lane, lt);
         s.qsatl = qsatl;
         s.qaf = qaf;
         s.morning = H.local_morning[pp] != 0;

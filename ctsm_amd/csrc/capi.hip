@@ -39,9 +39,10 @@ size_t soilwater_plain_workspace_doubles(int n);
 void launch_soilwater_plain(hipStream_t, const View &, const Params &, const ctsm_col_state &, int, const int32_t *,
                             double, double *, long, ErrWord *);
 size_t canopy_work_bytes(int n, int itmax, int first_its, int round_its);
+int canopy_one_pass_patches(size_t bytes, int itmax, int first_its, int round_its);
 void launch_canopy(hipStream_t, const ctsm_layout &, const ctsm_config &, const ctsm_canopy_params &, const double *,
                    const ctsm_col_state &, const ctsm_canopy_state &, int, const int32_t *, double, ErrWord *,
-                   void *, int, int, bool, int, bool, const ctsm_phs_state *, const ctsm_phs_canopy_state *,
+                   void *, int part, int, int, bool, int, bool, const ctsm_phs_state *, const ctsm_phs_canopy_state *,
                    const double *);
 void launch_root_sink(hipStream_t, const ctsm_layout &, const ctsm_config &, const ctsm_col_state &,
                       const ctsm_canopy_state &, int, const int32_t *, ErrWord *);
@@ -401,7 +402,7 @@ struct ctsm_ctx {
     void *scratch_dev = nullptr;      // this device's copy of `scratch`
     ctsm_config cfg{};
     Params prm{};
-    ctsm_tuning tun{4, 128, 128, 0, 6, 3, 4, 0, 1};
+    ctsm_tuning tun{4, 128, 128, 0, 6, 3, 4, 0, 2};
     static constexpr int kMaxStreams = 4;
     hipStream_t side[kMaxStreams - 1] = {nullptr, nullptr, nullptr};   // concurrent parts of a step
     hipEvent_t ev_fork = nullptr, ev_join[kMaxStreams - 1] = {nullptr, nullptr, nullptr};
@@ -1005,9 +1006,10 @@ static int check_canopy_layout(const ctsm_ctx *ctx, const ctsm_layout *L)
     return CTSM_OK;
 }
 
-// Grows the canopy round buffer to n patches and launches CanopyFluxes.
-// With fixed_work, the rounds use that buffer of fixed_bytes instead and
-// nothing is allocated (CTSM_E_SCRATCH when it is too small).  With
+// Grows the canopy work buffer to n patches and launches CanopyFluxes.
+// With fixed_work, the kernels use that buffer of fixed_bytes instead and
+// nothing is allocated (CTSM_E_SCRATCH when it is too small for the rounds; an
+// iteration without rounds goes over the filter in parts that fit).  With
 // bounds_are_filter the per-step resets of the bounds (rb1, the
 // photosynthesis outputs) cover the filter's patches instead of the whole
 // layout: a caller whose layout holds other, independent runs (the ensemble
@@ -1024,8 +1026,10 @@ static int run_canopy(ctsm_ctx *ctx, const ctsm_layout *lay, const ctsm_col_stat
     const int k = one_pass ? 1 : ctx->tun.canopy_round_iterations;
     const size_t wb = canopy_work_bytes(n, ctx->cfg.itmax_canopy_fluxes, k0, k);
     void *work = nullptr;
+    int part = 0;
     if (wb && fixed_work) {
-        if (wb > fixed_bytes) {
+        part = canopy_one_pass_patches(fixed_bytes, ctx->cfg.itmax_canopy_fluxes, k0, k);
+        if (wb > fixed_bytes && part == 0) {
             ctx->last_code = CTSM_E_SCRATCH;
             ctx->last_index = (int32_t)std::min<size_t>((wb + 1023) / 1024, INT32_MAX);
             return CTSM_E_SCRATCH;
@@ -1037,7 +1041,7 @@ static int run_canopy(ctsm_ctx *ctx, const ctsm_layout *lay, const ctsm_col_stat
         work = ctx->cwork.p;
     }
     launch_canopy(ctx->stream, *lay, ctx->cfg, ctx->cprm, (const double *)ctx->pft.p, col, can, n, filter_dev, dtime,
-                  ctx->err, work, k0, k, zero_cgrnd, ctx->tun.canopy_waves, bounds_are_filter, phs_q, phs_h,
+                  ctx->err, work, part, k0, k, zero_cgrnd, ctx->tun.canopy_waves, bounds_are_filter, phs_q, phs_h,
                   (const double *)ctx->phs_tab.p);
     return CTSM_OK;
 }

@@ -93,4 +93,10 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// log's table in the LDS of a one-wave block (ctsm_math.h)
+#define LOG_TABLE(name)                                                                                            \
+    __shared__ double name[CM_LOGT_N * 3];                                                                         \
+    for (int i_ = threadIdx.x; i_ < CM_LOGT_N * 3; i_ += 64) name[i_] = cm_log_table()[i_];                         \
+    wave_sync()
+
 }  // namespace ctsm

@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(256) k_phs_conductance(PView V, ctsm_phs_state
         const double rai = lai * froot_leaf * rf;
         const double r_soil = sqrt(1.0 / (RPI * rld));
         double soil_c = fmin90(S.hksat[V.soi(c, j)], S.hk_l[V.soi(c, j)]) / (1.e3 * r_soil);
-        const double fs = plc(S.smp_l[V.soi(c, j)], psi50, ck);
+        const double fs = plc(S.smp_l[V.soi(c, j)], psi50, ck, cm_log_table());
         double root_c = (fs * rai * krmax) / (CROOT_LATERAL_LENGTH + zj);
         soil_c = fmax90(soil_c, 1.e-16);
         root_c = fmax90(root_c, 1.e-16);
@@ -120,6 +120,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8)))
 k_phs_calcstress(PView V, ctsm_phs_stress_state S, const double *__restrict__ T, int npft, int n,
                  const int32_t *__restrict__ filter, ErrWord *err)
 {
+    LOG_TABLE(logt);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int p = filter ? filter[i] : V.begp + i;
@@ -139,7 +140,7 @@ k_phs_calcstress(PView V, ctsm_phs_stress_state S, const double *__restrict__ T,
     }
     __shared__ double soil[SOIL_LDS * SOIL_STRIDE];
     stage_soil(P, S.k_soil_root + V.soip(p, 1), V.ldp, S.smp_l + V.soi(c, 1), S.z + V.sno(c, 1), V.ldc, V.nlevsoi,
-               soil + threadIdx.x);
+               soil + threadIdx.x, logt);
     const double qsatl = S.qsatl[pp], qaf = S.qaf[pp];
     const double gs_sun_in = S.gs_mol_sun[pp], gs_sha_in = S.gs_mol_sha[pp];
     double x[4];

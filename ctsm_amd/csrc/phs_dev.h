@@ -18,9 +18,10 @@ constexpr double CROOT_LATERAL_LENGTH = 0.25;      // m (:2910)
 enum { T_KRMAX = 0, T_RADIUS = 1, T_DENSITY = 2, T_FROOT_LEAF = 3, T_PSI50 = 4, T_CK = 8, T_KMAX = 12, T_CROP = 16, T_ROWS = 17 };
 
 // plc, vegetation_weibull branch: 2**(-(x/psi50)**ck), cut to zero below 0.005
-__device__ __forceinline__ double plc(double x, double psi50, double ck)
+// (lt: log's table)
+__device__ __forceinline__ double plc(double x, double psi50, double ck, const double *lt)
 {
-    double v = cm_pow(2.0, -cm_pow(x / psi50, ck));
+    double v = cm_pow(2.0, -cm_pow_tab(x / psi50, ck, lt));
     if (v < 0.005) v = 0.0;
     return v;
 }
@@ -42,6 +43,7 @@ struct Leaf {
     // no potential enters -- of k, k smp, smp - 1000 z and k (smp - 1000 z).
     const double *k, *g;
     double sum_k, sum_ks, sum_w, sum_kw;
+    const double *lt;            // log's table in LDS
     const double *smp;           // layer 1 of smp_l(c, :), stride ss
     long ss;
     int n;
@@ -56,10 +58,11 @@ constexpr int SOIL_STRIDE = 64;
 // them, they were what a pass waited for.
 __device__ __forceinline__ void stage_soil(Leaf &P, const double *__restrict__ k, long sk,
                                            const double *__restrict__ smp, const double *__restrict__ z, long ss, int n,
-                                           double *lds)
+                                           double *lds, const double *lt)
 {
     P.k = lds;
     P.g = lds + MAX_NLEVSOI * SOIL_STRIDE;
+    P.lt = lt;
     P.smp = smp;
     P.ss = ss;
     P.n = n;
@@ -98,7 +101,7 @@ struct Curves {
 __device__ __forceinline__ void curves(const Leaf &P, const double *x, Curves &C)
 {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) C.u[k] = cm_pow(x[k] / P.psi50[k], P.ck[k]);
+    for (int k = 0; k < 4; ++k) C.u[k] = cm_pow_tab(x[k] / P.psi50[k], P.ck[k], P.lt);
 #pragma unroll
     for (int k = 0; k < 4; ++k) C.w[k] = cm_pow(2.0, -C.u[k]);
 #pragma unroll
@@ -256,12 +259,12 @@ __device__ double getvegwp(const Leaf &P, double *x, double gs_sun, double gs_sh
     getqflx(P, qsatl, qaf, true, gs_sun, gs_sha, q_sun, q_sha);
     if (fabs(P.sum_k) == 0.0) x[3] = P.sum_w / P.n;
     else x[3] = (P.sum_kw - q_sun - q_sha) / P.sum_k;
-    const double fr = plc(x[3], P.psi50[3], P.ck[3]);
+    const double fr = plc(x[3], P.psi50[3], P.ck[3], P.lt);
     if (P.tsai > 0.0 && fr > 0.0)
         x[2] = x[3] - grav1 - (q_sun + q_sha) / (fr * P.kmax[3] / P.htop * P.tsai);
     else
         x[2] = x[3] - grav1;
-    const double fx = plc(x[2], P.psi50[2], P.ck[2]);
+    const double fx = plc(x[2], P.psi50[2], P.ck[2], P.lt);
     x[1] = (P.laisha > 0.0 && fx > 0.0) ? x[2] - (q_sha / (fx * P.kmax[2] * P.laisha)) : x[2];
     x[0] = (P.laisun > 0.0 && fx > 0.0) ? x[2] - (q_sun / (fx * P.kmax[2] * P.laisun)) : x[2];
     double w[MAX_NLEVSOI];
@@ -354,14 +357,14 @@ __device__ __forceinline__ bool calcstress(const Leaf &P, double *x, double gs_s
     }
     if (flag) {
         (void)getvegwp(P, x, gs0sun, gs0sha, qsatl, qaf);
-        bsun = plc(x[0], P.psi50[0], P.ck[0]);
-        bsha = plc(x[1], P.psi50[1], P.ck[1]);
+        bsun = plc(x[0], P.psi50[0], P.ck[0], P.lt);
+        bsha = plc(x[1], P.psi50[1], P.ck[1], P.lt);
     } else {
-        double qs = q_sun * plc(x[0], P.psi50[0], P.ck[0]);
-        double qh = q_sha * plc(x[1], P.psi50[1], P.ck[1]);
+        double qs = q_sun * plc(x[0], P.psi50[0], P.ck[0], P.lt);
+        double qh = q_sha * plc(x[1], P.psi50[1], P.ck[1], P.lt);
         getqflx(P, qsatl, qaf, false, gs0sun, gs0sha, qs, qh);
-        bsun = (q_sun > 0.0) ? gs0sun / gs_sun_in : plc(x[0], P.psi50[0], P.ck[0]);
-        bsha = (q_sha > 0.0) ? gs0sha / gs_sha_in : plc(x[1], P.psi50[1], P.ck[1]);
+        bsun = (q_sun > 0.0) ? gs0sun / gs_sun_in : plc(x[0], P.psi50[0], P.ck[0], P.lt);
+        bsha = (q_sha > 0.0) ? gs0sha / gs_sha_in : plc(x[1], P.psi50[1], P.ck[1], P.lt);
     }
     if (bsun < 0.01) bsun = 0.0;
     if (bsha < 0.01) bsha = 0.0;

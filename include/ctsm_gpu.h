@@ -602,10 +602,11 @@ typedef struct ctsm_phs_canopy_state {
  * canopy_first_iterations, canopy_round_iterations: CanopyFluxes runs its
  *   leaf-temperature iteration in rounds; the first round takes every patch of
  *   the filter for at most canopy_first_iterations iterations, each later round
- *   only the patches still iterating (compacted) for at most
- *   canopy_round_iterations more.  canopy_first_iterations > itmax_canopy_fluxes
- *   runs the whole iteration in one pass.  Both >= 1; results do not depend on
- *   them.
+ *   only the patches still iterating (compacted): the next two for at most
+ *   canopy_round_iterations more, the following ones for twice as many as the one
+ *   before.  A filter of at most 65,536 patches takes a single later round.
+ *   canopy_first_iterations > itmax_canopy_fluxes runs the whole iteration in one
+ *   pass.  Both >= 1; results do not depend on them.
  * step_streams: the fused soil step splits its filter into this many
  *   contiguous parts run on as many streams of the context at once, joined
  *   before the call's later work (1..4).  A batch stored in work-binned
@@ -616,9 +617,10 @@ typedef struct ctsm_phs_canopy_state {
  *   the *_dev entries' `plain` argument), CanopyFluxes as one launch that
  *   iterates every patch to convergence (no compacted rounds).  The comparison
  *   baseline of the batched step; results are the same.
- * canopy_waves: the register budget of the CanopyFluxes kernel, in waves per
- *   SIMD (1, 2 or 3: one compiled instance each; a larger budget spills more
- *   to scratch).  Results do not depend on it. */
+ * canopy_waves: the waves per SIMD the CanopyFluxes iteration is built for, at
+ *   most: 1, or 2 and 3 for the two-wave kernel on filters that have a second
+ *   wave for the SIMDs (more than 65,536 patches).  Results do not depend on
+ *   it. */
 typedef struct ctsm_tuning {
     int32_t richards_lanes;
     int32_t richards_block;

@@ -156,6 +156,49 @@ def test_canopy_rounds_bitwise(cctx, first, later, itmax, waves):
         assert g.can["num_iter"].max() == itmax + 1
 
 
+@pytest.mark.parametrize("n,waves", [
+    (65536, 2),      # a wave for every SIMD: one later round
+    (65537, 2),      # one more: growing rounds, the two-wave kernel in the first
+    (65537, 1),
+    (262145, 2),     # the two-wave kernel in the later rounds as well
+])
+def test_canopy_launch_rules_bitwise(cctx, n, waves):
+    """Either side of the sizes at which the launch changes kernel and rounds."""
+    ctx = cctx()
+    before = ctx.get_tuning()
+    st = S.canopy_workload("canopy_uneven", ncol=n // 8)
+    filt = np.arange(1, n + 1, dtype=np.int32)
+    assert st.dims.npatch >= n
+    print(f"case: CanopyFluxes of {n} patches, canopy_waves={waves}", flush=True)
+    ctx.set_tuning(canopy_waves=waves)
+    try:
+        g = st.copy()
+        ctx.canopyfluxes(g, filter_p=filt)
+    finally:
+        ctx.set_tuning(**before)
+    rc, bad = O.canopyfluxes(st, _oracle_cfg(ctx), S.canopy_params(), O.PftStruct(S.pft_table()), filter_p=filt)
+    assert rc == 0, bad
+    _assert_same(g, st)
+
+
+@pytest.mark.parametrize("which", ["one patch per column", "shuffled"])
+def test_canopy_many_columns_per_wave_bitwise(cctx, which):
+    """Waves whose patches lie in up to 64 columns: the set-up's soil terms in
+    several parts, and a last wave that is not full."""
+    ctx = cctx()
+    st = S.canopy_workload("canopy_uneven", ncol=203)
+    if which == "shuffled":
+        filt = np.random.default_rng(3).permutation(np.arange(1, st.dims.npatch + 1)).astype(np.int32)
+    else:
+        filt = np.unique(st.pch["column"], return_index=True)[1].astype(np.int32) + 1
+    print(f"case: CanopyFluxes, {which}, {len(filt)} patches", flush=True)
+    g = st.copy()
+    ctx.canopyfluxes(g, filter_p=filt)
+    rc, bad = O.canopyfluxes(st, _oracle_cfg(ctx), S.canopy_params(), O.PftStruct(S.pft_table()), filter_p=filt)
+    assert rc == 0, bad
+    _assert_same(g, st)
+
+
 def test_canopy_error_reports_patch(cctx):
     ctx = cctx(z0param_method=0)
     st = S.canopy_workload("canopy", ncol=16)

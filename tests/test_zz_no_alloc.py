@@ -105,3 +105,23 @@ def test_noalloc_refuses_a_batch_beyond_its_scratch():
             ds.free()
     finally:
         ctx.close()
+
+
+def test_noalloc_one_pass_in_parts():
+    """Without rounds the scratch holds part of a long filter, and the call goes
+    over it in parts: the same results as the allocating entry's one part."""
+    from ctsm_amd.lib import Context
+    ctx = Context()
+    try:
+        ctx.set_canopy_params(S.canopy_params(), S.pft_table())
+        ctx.set_tuning(canopy_first_iterations=41)
+        room = NOALLOC_SCRATCH_BYTES // 128
+        st = S.canopy_workload("canopy", ncol=room // 8)
+        filt = np.arange(st.dims.npatch, 0, -1, dtype=np.int32)
+        assert len(filt) > room
+        print(f"case: no-allocation CanopyFluxes in one pass, {len(filt)} patches", flush=True)
+        g_dev, _ = _run(ctx, st, noalloc=False, filt=filt)
+        g_na, _ = _run(ctx, st, noalloc=True, filt=filt)
+        _same(g_na, g_dev)
+    finally:
+        ctx.close()
