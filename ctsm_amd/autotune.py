@@ -26,7 +26,6 @@ DEFAULT_CANDIDATES = [
     dict(richards_lanes=8, richards_block=128, soiltemp_block=64, fused_single_kernel=0, step_streams=1),
     dict(richards_lanes=8, richards_block=256, soiltemp_block=64, fused_single_kernel=0, step_streams=4),
     dict(richards_lanes=4, richards_block=128, soiltemp_block=128, fused_single_kernel=0, step_streams=4),
-    dict(richards_lanes=2, richards_block=128, soiltemp_block=128, fused_single_kernel=0, step_streams=4),
     dict(richards_lanes=1, richards_block=64, soiltemp_block=128, fused_single_kernel=0, step_streams=4),
     dict(richards_lanes=1, richards_block=64, soiltemp_block=64, fused_single_kernel=1, step_streams=1),
 ]

@@ -73,30 +73,6 @@ struct CSwitch {
 __device__ __forceinline__ double p4(double x) { const double x2 = x * x; return x2 * x2; }
 __device__ __forceinline__ double p3(double x) { return (x * x) * x; }
 
-// Divisions by one denominator.  recip(b) holds the refined reciprocal that an IEEE
-// division by b forms (v_rcp_f64 and two Newton steps) and a / r finishes it (a
-// product, its remainder, one correction): the instructions of the compiler's own
-// division without the scaling that only operands near the ends of the exponent
-// range need, so the quotient is the correctly rounded one, for 4 instructions
-// instead of 11.  For denominators and quotients of magnitudes between 2^-900 and
-// 2^900 (zero, infinite and NaN operands are settled by v_div_fixup as in a
-// division).
-struct Recip {
-    double b, y;
-};
-__device__ __forceinline__ Recip recip(double b)
-{
-    double y = __builtin_amdgcn_rcp(b);
-    y = fma(y, fma(-b, y, 1.0), y);
-    y = fma(y, fma(-b, y, 1.0), y);
-    return Recip{b, y};
-}
-__device__ __forceinline__ double operator/(double a, const Recip &r)
-{
-    const double q = a * r.y;
-    return __builtin_amdgcn_div_fixup(fma(fma(-r.b, q, a), r.y, q), r.b, a);
-}
-
 // QSatMod.F90:61-127
 __device__ __forceinline__ void qsat(double T, double p, double &qs, double &es, double &qsdT)
 {

@@ -402,7 +402,7 @@ struct ctsm_ctx {
     void *scratch_dev = nullptr;      // this device's copy of `scratch`
     ctsm_config cfg{};
     Params prm{};
-    ctsm_tuning tun{4, 128, 128, 0, 6, 3, 4, 0, 2};
+    ctsm_tuning tun{8, 128, 128, 0, 6, 3, 4, 0, 2};
     static constexpr int kMaxStreams = 4;
     hipStream_t side[kMaxStreams - 1] = {nullptr, nullptr, nullptr};   // concurrent parts of a step
     hipEvent_t ev_fork = nullptr, ev_join[kMaxStreams - 1] = {nullptr, nullptr, nullptr};

@@ -93,10 +93,39 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Divisions by one denominator.  recip(b) holds the refined reciprocal that an IEEE
+// division by b forms (v_rcp_f64 and two Newton steps) and a / r finishes it (a
+// product, its remainder, one correction): the instructions of the compiler's own
+// division without the scaling that only operands near the ends of the exponent
+// range need, so the quotient is the correctly rounded one, for 4 instructions
+// instead of 11.  For denominators and quotients of magnitudes between 2^-900 and
+// 2^900 (zero, infinite and NaN operands are settled by v_div_fixup as in a
+// division).
+struct Recip {
+    double b, y;
+};
+__device__ __forceinline__ Recip recip(double b)
+{
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(y, fma(-b, y, 1.0), y);
+    y = fma(y, fma(-b, y, 1.0), y);
+    return Recip{b, y};
+}
+__device__ __forceinline__ double operator/(double a, const Recip &r)
+{
+    const double q = a * r.y;
+    return __builtin_amdgcn_div_fixup(fma(fma(-r.b, q, a), r.y, q), r.b, a);
+}
+
 // log's table in the LDS of a one-wave block (ctsm_math.h)
 #define LOG_TABLE(name)                                                                                            \
     __shared__ double name[CM_LOGT_N * 3];                                                                         \
     for (int i_ = threadIdx.x; i_ < CM_LOGT_N * 3; i_ += 64) name[i_] = cm_log_table()[i_];                         \
     wave_sync()
+// the same for a block of any size; before anything a thread may leave the kernel by
+#define LOG_TABLE_BLOCK(name)                                                                                      \
+    __shared__ double name[CM_LOGT_N * 3];                                                                         \
+    for (int i_ = threadIdx.x; i_ < CM_LOGT_N * 3; i_ += blockDim.x) name[i_] = cm_log_table()[i_];                 \
+    __syncthreads()
 
 }  // namespace ctsm

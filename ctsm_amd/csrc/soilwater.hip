@@ -57,12 +57,10 @@ k_soilwater_fractions(View V, ctsm_col_state S, int n, const int32_t *__restrict
 }
 
 // G lanes per column (richards_group.h).  Groups are aligned to G lanes, so a
-// column's lanes retire together.  The solve is latency-bound (a trial is a
-// serial elimination chain), so for G = 8 the register budget is capped at 168
-// VGPRs for three waves per SIMD: the few values that then live in scratch
-// (10 VGPRs) cost less than the latency the extra wave hides.  Measured on the
-// columns ordered by their previous sub-step count, 1,048,576 uneven columns:
-// 5.07 ms at four waves (77 VGPRs spilled), 4.37 at three, 5.17 at two.
+// column's lanes retire together.  For G = 8 the register budget is capped at 168
+// VGPRs for three waves per SIMD (192 B/lane of scratch): 262,144 uneven columns
+// 3.61 ms, 4.09 at two waves and 4.77 at four.  G = 4 needs 374 registers: 4.24 ms
+// at one wave per SIMD, 4.52 at two, 5.89 at three.
 template <int G> struct RichardsWaves { static constexpr int value = 1; };
 template <> struct RichardsWaves<8> { static constexpr int value = 3; };
 
@@ -71,12 +69,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Richar
 k_soilwater_g(View V, Params P, ctsm_col_state S, int n, const int32_t *__restrict__ filter, double dtime,
               ErrWord *err)
 {
+    LOG_TABLE_BLOCK(logt);
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int i = t / G, g = t % G;
     if (i >= n) return;
     const int c = filter ? filter[i] : V.begc + i;
     if (!col_in_range(V, c)) { if (g == 0) report_error(err, c, CTSM_E_ARG); return; }
-    const int rc = richards_group<G, WT>(V, P, S, c, dtime, g);
+    const int rc = richards_group<G, WT>(V, P, S, c, dtime, g, logt);
     if (rc && g == 0) report_error(err, c, richards_error_code(rc));
 }
 
@@ -88,10 +87,10 @@ k_soilwater_g(View V, Params P, ctsm_col_state S, int n, const int32_t *__restri
 // smallest group its columns allow, so no lane holds only empty layers; the
 // results do not depend on the group size.  Built for three waves per SIMD
 // (168 VGPRs): at four (128 VGPRs, 120 spilled) the solve of 1,048,576
-// uneven columns took 8.3 ms, at three 7.4, at two 8.1; with the columns
-// ordered by sub-step count and depth class (SubstepDepthKey) 6.3-7.0 ms.
-// A deep block runs its 32 columns in four passes of 8, so the 8-lane kernel
-// (4.4 ms with its order) stays the default.
+// uneven columns took 8.3 ms, at three 7.4, at two 8.1.
+// A deep block runs its 32 columns in four passes of 8, so that 20,000 columns in
+// their own order take 3.53 ms a land step against the 8-lane kernel's 2.80; on
+// 262,144 ordered ones 3.26 and 3.39 ms.
 constexpr int ADAPT_SPAN = 32;
 constexpr int ADAPT_K = 3;
 template <bool WT>
@@ -99,6 +98,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 k_soilwater_adaptive(View V, Params P, ctsm_col_state S, int n, const int32_t *__restrict__ filter, double dtime,
                      ErrWord *err)
 {
+    LOG_TABLE(logt);
     const int lane = threadIdx.x;
     const int i0 = blockIdx.x * ADAPT_SPAN;
     const int i1 = min(i0 + ADAPT_SPAN, n);
@@ -118,7 +118,7 @@ k_soilwater_adaptive(View V, Params P, ctsm_col_state S, int n, const int32_t *_
             if (!col_in_range(V, c)) {
                 if (g == 0) report_error(err, c, CTSM_E_ARG);
             } else {
-                const int rc = richards_group<0, WT, ADAPT_K>(V, P, S, c, dtime, g, gsz);
+                const int rc = richards_group<0, WT, ADAPT_K>(V, P, S, c, dtime, g, logt, gsz);
                 if (rc && g == 0) report_error(err, c, richards_error_code(rc));
             }
         }
@@ -150,16 +150,17 @@ void launch_soilwater_k(hipStream_t st, const View &V, const Params &P, const ct
                            st, V, P, S, n, filter, dtime, err);
         return;
     }
-    if (block <= 0 || block > 256) block = (lanes == 1) ? 64 : 128;
-    if (lanes != 2 && lanes != 4 && lanes != 8) block = 64;     /* k_soilwater: __launch_bounds__(64) */
-    const long threads = (long)n * (lanes > 0 ? lanes : 1);
-    const dim3 grid((unsigned)((threads + block - 1) / block)), blk(block);
-    switch (lanes) {
-    case 2: hipLaunchKernelGGL((k_soilwater_g<2, WT>), grid, blk, 0, st, V, P, S, n, filter, dtime, err); break;
-    case 4: hipLaunchKernelGGL((k_soilwater_g<4, WT>), grid, blk, 0, st, V, P, S, n, filter, dtime, err); break;
-    case 8: hipLaunchKernelGGL((k_soilwater_g<8, WT>), grid, blk, 0, st, V, P, S, n, filter, dtime, err); break;
-    default: hipLaunchKernelGGL(k_soilwater<WT>, grid, blk, 0, st, V, P, S, n, filter, dtime, err); break;
+    if (lanes == 2 || lanes == 4 || lanes == 8) {
+        // two lanes run as four: 262,144 columns 6.12 ms at two lanes of 10 layers, which
+        // spill, 3.83 at four and 3.39 at eight
+        if (block <= 0 || block > 256) block = 128;
+        const int G = lanes == 8 ? 8 : 4;
+        const dim3 grid((unsigned)(((long)n * G + block - 1) / block));
+        auto kernel = G == 8 ? k_soilwater_g<8, WT> : k_soilwater_g<4, WT>;
+        hipLaunchKernelGGL(kernel, grid, dim3(block), 0, st, V, P, S, n, filter, dtime, err);
+        return;
     }
+    hipLaunchKernelGGL(k_soilwater<WT>, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, V, P, S, n, filter, dtime, err);
 }
 // ---- the Richards solve's column order ----------------------------------
 // The solve sub-steps adaptively, and the lanes of a wave iterate until the
