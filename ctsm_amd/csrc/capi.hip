@@ -454,6 +454,8 @@ Params make_params(const ctsm_config &c)
     p.lower_bc = c.lower_boundary_condition;
     p.flux_calculation = c.flux_calculation;
     p.snow_thermal_cond = c.snow_thermal_cond_method;
+    cm_log_dd(TKWAT, cm_log_table(), &p.log_tkwat[0], &p.log_tkwat[1]);
+    cm_log_dd(TKICE, cm_log_table(), &p.log_tkice[0], &p.log_tkice[1]);
     return p;
 }
 

@@ -59,6 +59,7 @@ struct View {
 struct Params {
     double dtmin, verySmall, xTolerUpper, xTolerLower, e_ice;
     int lower_bc, flux_calculation, snow_thermal_cond;
+    double log_tkwat[2], log_tkice[2];   // log of the conductivities of water and ice (double-double)
 };
 
 // Error word of a launch: first failing column index (atomicMin) and a code.

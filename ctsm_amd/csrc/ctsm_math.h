@@ -315,15 +315,17 @@ CM_FN double cm_log_tab(double x, const double *tab)
 
 CM_FN double cm_log(double x) { return cm_log_tab(x, cm_log_table()); }
 
-CM_FN double cm_log10(double x)
+CM_FN double cm_log10_tab(double x, const double *tab)
 {
     if (!(x > 0.0)) return (x == 0.0) ? -HUGE_VAL : (x - x) / (x - x);
     if (x == HUGE_VAL) return x;
     double h, l, rh, rl;
-    cm_log_dd(x, cm_log_table(), &h, &l);
+    cm_log_dd(x, tab, &h, &l);
     cm_dd_mul(h, l, CM_INV_LN10_H, CM_INV_LN10_L, &rh, &rl);
     return rh + rl;
 }
+
+CM_FN double cm_log10(double x) { return cm_log10_tab(x, cm_log_table()); }
 
 /* arctangent.  |x| > 1 is folded to pi/2 - atan(1/|x|) with 1/|x| kept as a
  * double-double; the reduced argument a is split as a = c + (a - c) with
@@ -421,15 +423,21 @@ CM_FN double cm_pow_special(double x, double y, const double *tab)
 
 /* x**y; the physics takes it of x > 0 only.  x**0 = 1 and x**1 = x exactly, as
  * a C pow gives them (the first of itself: exp(0)). */
+/* x^y for x > 0 (finite), whose log is lh + ll (cm_log_dd), and finite y */
+CM_FN double cm_pow_log(double x, double lh, double ll, double y)
+{
+    const double zh = y * lh;
+    const double zl = fma(y, lh, -zh) + y * ll;
+    const double res = cm_exp_dd(zh, zl);
+    return y == 1.0 ? x : res;
+}
+
 CM_FN double cm_pow_tab(double x, double y, const double *tab)
 {
     if (__builtin_expect(!(x > 0.0 && x < HUGE_VAL) || !(fabs(y) < HUGE_VAL), 0)) return cm_pow_special(x, y, tab);
     double lh, ll;
     cm_log_dd(x, tab, &lh, &ll);
-    const double zh = y * lh;
-    const double zl = fma(y, lh, -zh) + y * ll;
-    const double res = cm_exp_dd(zh, zl);
-    return y == 1.0 ? x : res;
+    return cm_pow_log(x, lh, ll, y);
 }
 
 CM_FN double cm_pow(double x, double y) { return cm_pow_tab(x, y, cm_log_table()); }

@@ -60,7 +60,7 @@ __global__ void k_thermprop(View V, Params P, ctsm_col_state S, int n, const int
     const int nbedrock = S.nbedrock[V.c1(c)];
     const double frac_sno = S.frac_sno_eff[V.c1(c)];
     const double h2osno_no_layers = S.h2osno_no_layers[V.c1(c)];
-    for (int j = snl + 1; j <= NG; ++j) S.thk[V.sno(c, j)] = level_thk(V, P, S, c, j, nbedrock, frac_sno);
+    for (int j = snl + 1; j <= NG; ++j) S.thk[V.sno(c, j)] = level_thk(V, P, S, c, j, nbedrock, frac_sno, cm_log_table());
     for (int j = snl + 1; j <= NG; ++j) {
         double tk;
         if (j <= NG - 1) {

@@ -74,7 +74,8 @@ struct GfWave {
 // Every lane of the wave calls it (valid: the lane has a column in range);
 // the sums of a lane whose column soiltemp_column rejects are not used.  The
 // snow levels' sums go to wk.Sab(i, .).
-__device__ void ground_flux_of_wave(const View &V, const ctsm_col_state &S, const ctsm_patch_state &Pt, int c,
+template <class CS, class CP>
+__device__ __forceinline__ void ground_flux_of_wave(const View &V, const CS &S, const CP &Pt, int c,
                                     bool valid, GfWave &L, const TempWork &wk, int i, GroundFlux &g)
 {
     const int lane = threadIdx.x & 63;
@@ -249,10 +250,12 @@ __device__ __forceinline__ bool eliminate(Window &w, int km)
 }
 
 // Full column.  `lane` indexes the workspace.  Returns 0 or an error code.
-__device__ int soiltemp_column(const View &V, const Params &P, const ctsm_col_state &S,
-                               const ctsm_patch_state &Pt, int c, double dtime,
-                               const TempWork &wk, int lane, const GroundFlux &gf)
+template <class CS, class CP>
+__device__ __forceinline__ int soiltemp_column(const View &V, const Params &P, const CS &Sk,
+                               const CP &Pt, int c, double dtime,
+                               const TempWork &wk, int lane, const GroundFlux &gf, const double *lt)
 {
+    const CS &S = Sk;
     const int nlevgrnd = V.nlevgrnd;
     const int snl = S.snl[V.c1(c)], nbedrock = S.nbedrock[V.c1(c)];
     if (snl < -V.nlevsno || snl > 0) return 1;
@@ -325,15 +328,20 @@ __device__ int soiltemp_column(const View &V, const Params &P, const ctsm_col_st
 
     double tkh2osfc = 0.0, fn_h2osfc = 0.0;
     // lookahead state for level j: thk(j), t(j), z(j)
-    double thk_j = level_thk(V, P, S, c, ltop, nbedrock, frac_sno);
+    double thk_j = level_thk(V, P, S, c, ltop, nbedrock, frac_sno, lt);
     double tk_prev = 0.0, fn_prev = 0.0;
     for (int j = ltop; j <= nlevgrnd; ++j) {
+        // the arrays' addresses are read anew in each pass: all of them held over the
+        // loop would not fit the scalar registers
+        const CS *Sp = &Sk;
+        asm volatile("" : "+s"(Sp));
+        const CS &S = *Sp;
         const double tj = S.t_soisno[V.sno(c, j)];
         const double zj = S.z[V.sno(c, j)];
         double thk_n = 0.0, tn = 0.0, zn = 0.0, tk_j, fn_j, fact_j;
         S.thk[V.sno(c, j)] = thk_j;
         if (j < nlevgrnd) {
-            thk_n = level_thk(V, P, S, c, j + 1, nbedrock, frac_sno);
+            thk_n = level_thk(V, P, S, c, j + 1, nbedrock, frac_sno, lt);
             tn = S.t_soisno[V.sno(c, j + 1)];
             zn = S.z[V.sno(c, j + 1)];
             const double zij = S.zi[V.zi(c, j)];
@@ -459,6 +467,9 @@ __device__ int soiltemp_column(const View &V, const Params &P, const ctsm_col_st
     // ---- sweep 2: dtbsv back substitution, rows n-1 .. 0
     double x1 = 0.0, x2 = 0.0, x3 = 0.0, x4 = 0.0;   // x(i+1..i+4)
     for (int i = n - 1; i >= 0; --i) {
+        const CS *Sp = &Sk;
+        asm volatile("" : "+s"(Sp));
+        const CS &S = *Sp;
         double x = wk.U(lane, i, 5);
         const double u1 = wk.U(lane, i, 1), u2 = wk.U(lane, i, 2), u3 = wk.U(lane, i, 3), u4 = wk.U(lane, i, 4);
         // contributions in dtbsv's order: column i+4 first, then i+3, i+2, i+1
@@ -481,6 +492,9 @@ __device__ int soiltemp_column(const View &V, const Params &P, const ctsm_col_st
     {
         double tcur = S.t_soisno[V.sno(c, ltop)];
         for (int j = ltop; j <= nlevgrnd; ++j) {
+            const CS *Sp = &Sk;
+            asm volatile("" : "+s"(Sp));
+            const CS &S = *Sp;
             double fn1;
             double tnext = 0.0;
             if (j <= nlevgrnd - 1) {
@@ -575,6 +589,9 @@ __device__ int soiltemp_column(const View &V, const Params &P, const ctsm_col_st
     if (S.qflx_snomelt_lyr)
         for (int j = -V.nlevsno + 1; j <= 0; ++j) { S.qflx_snomelt_lyr[V.sno(c, j)] = 0.0; S.qflx_snofrz_lyr[V.sno(c, j)] = 0.0; }
     for (int j = ltop; j <= nlevgrnd; ++j) {
+        const CS *Sp = &Sk;
+        asm volatile("" : "+s"(Sp));
+        const CS &S = *Sp;
         double t = S.t_soisno[V.sno(c, j)];
         double liq = S.h2osoi_liq[V.sno(c, j)], ice = S.h2osoi_ice[V.sno(c, j)];
         const double wice0 = ice, wmass0 = ice + liq + 0.0;
@@ -588,7 +605,7 @@ __device__ int soiltemp_column(const View &V, const Params &P, const ctsm_col_st
             if (ice > 0.0 && t > TFRZ) { imelt = 1; tinc = TFRZ - t; t = TFRZ; }
             if (t < TFRZ) {
                 const double smp = HFUS * (TFRZ - t) / (GRAV * t) * 1000.0;
-                supercool = S.watsat[V.soi(c, j)] * cm_pow(smp / S.sucsat[V.soi(c, j)], -1.0 / S.bsw[V.soi(c, j)]);
+                supercool = S.watsat[V.soi(c, j)] * cm_pow_tab(smp / S.sucsat[V.soi(c, j)], -1.0 / S.bsw[V.soi(c, j)], lt);
                 supercool = supercool * S.dz[V.sno(c, j)] * 1000.0;
             }
             if (liq > supercool && t < TFRZ) { imelt = 2; tinc = TFRZ - t; t = TFRZ; }
@@ -704,31 +721,61 @@ __device__ int soiltemp_column(const View &V, const Params &P, const ctsm_col_st
 // lane of the block takes part (the sums are the wave's work).  Returns false
 // for a lane with nothing to solve (past the filter, or a column out of range:
 // reported).
-template <int BLOCK>
-__device__ __forceinline__ bool column_and_ground_flux(const View &V, const ctsm_col_state &S,
-                                                       const ctsm_patch_state &Pt, int n,
+template <int BLOCK, class CS, class CP>
+__device__ __forceinline__ bool column_and_ground_flux(const View &V, const CS &S,
+                                                       const CP &Pt, int n,
                                                        const int32_t *__restrict__ filter, const TempWork &wk,
-                                                       ErrWord *err, int i, int &c, GroundFlux &gf)
+                                                       ErrWord *err, int i, int &c, GroundFlux &gf, const double *&logt)
 {
     __shared__ GfWave gfl[BLOCK / 64];
     const bool active = i < n;
     c = active ? (filter ? filter[i] : V.begc + i) : V.begc;
     const bool in_range = active && col_in_range(V, c);
-    ground_flux_of_wave(V, S, Pt, c, in_range, gfl[threadIdx.x >> 6], wk, i, gf);
+    GfWave &L = gfl[threadIdx.x >> 6];
+    ground_flux_of_wave(V, S, Pt, c, in_range, L, wk, i, gf);
+    // log's table takes the place of the patches' terms, which are summed
+    static_assert(sizeof(L.y) >= CM_LOGT_N * 3 * sizeof(double), "room for the table");
+    double *tab = &L.y[0][0];
+    for (int k = threadIdx.x & 63; k < CM_LOGT_N * 3; k += 64) tab[k] = cm_log_table()[k];
+    wave_sync();
+    logt = tab;
     if (active && !in_range) report_error(err, c, CTSM_E_ARG);
     return in_range;
 }
 
+// The kernels' argument, read in place from the kernel-argument segment, each member
+// where it is used.
+struct SoilTempArgs {
+    View V;
+    Params P;
+    ctsm_col_state S;
+    ctsm_patch_state Pt;
+    int n;
+    const int32_t *filter;
+    double dtime;
+    TempWork wk;
+    ErrWord *err;
+};
+#define KARG __attribute__((address_space(4)))
+#define SOILTEMP_ARGS                                                                                              \
+    const KARG SoilTempArgs *A = (const KARG SoilTempArgs *)__builtin_amdgcn_kernarg_segment_ptr();                \
+    const View V{A->V.begc, A->V.ldc, A->V.begp, A->V.ldp, A->V.nlevsno, A->V.nlevsoi, A->V.nlevgrnd};             \
+    const Params P{A->P.dtmin, A->P.verySmall, A->P.xTolerUpper, A->P.xTolerLower, A->P.e_ice, A->P.lower_bc,      \
+                   A->P.flux_calculation, A->P.snow_thermal_cond, {A->P.log_tkwat[0], A->P.log_tkwat[1]},          \
+                   {A->P.log_tkice[0], A->P.log_tkice[1]}};                                                        \
+    const TempWork wk{A->wk.ws, A->wk.ld};                                                                         \
+    const double *logt
+
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3)))
-k_soiltemp(View V, Params P, ctsm_col_state S, ctsm_patch_state Pt, int n,
-           const int32_t *__restrict__ filter, double dtime, TempWork wk, ErrWord *err)
+k_soiltemp(SoilTempArgs)
 {
+    SOILTEMP_ARGS;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int c;
     GroundFlux gf;
-    if (!column_and_ground_flux<64>(V, S, Pt, n, filter, wk, err, i, c, gf)) return;
-    const int rc = soiltemp_column(V, P, S, Pt, c, dtime, wk, i, gf);
-    if (rc) report_error(err, c, CTSM_E_SOLVER);
+    if (!column_and_ground_flux<64>(V, A->S, A->Pt, A->n, A->filter, wk, A->err, i, c, gf, logt)) return;
+    const int rc = soiltemp_column(V, P, A->S, A->Pt, c, A->dtime, wk, i, gf, logt);
+    if (rc) report_error(A->err, c, CTSM_E_SOLVER);
 }
 
 
@@ -736,37 +783,40 @@ k_soiltemp(View V, Params P, ctsm_col_state S, ctsm_patch_state Pt, int n,
 // first kernel of the two-kernel soil step (the Richards solve follows with G
 // lanes per column).
 // BLOCK: 64 or 128 threads (the LDS of the ground heat flux is per wave).
-// Built for three waves per SIMD (168 VGPRs, 60 B/lane of scratch): on
-// 1,048,576 binned columns 3.48 ms against 4.22 ms at two waves (190 VGPRs);
-// 64-thread blocks, 4.22 against 6.37 ms for 128.
+// Built for three waves per SIMD (168 VGPRs, 32 B/lane of scratch; the LDS of the
+// ground heat flux leaves room for eleven waves a CU).  Bound by FP64 issue and the
+// waits of its loads, whose addresses hang on the level.  With the arrays' addresses
+// held in scalar registers 1,216 of the kernel's 5,300 instructions moved spilled ones
+// to vector lanes and back; read in place 20 do.  With log's table in LDS too, 262,144
+// columns 975 and 916 us, the step of 1,048,576 columns 42.7 and 41.5 ms.
 template <int BLOCK>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3)))
-k_soiltemp_fractions(View V, Params P, ctsm_col_state S, ctsm_patch_state Pt, int n,
-                     const int32_t *__restrict__ filter, double dtime, TempWork wk, ErrWord *err)
+k_soiltemp_fractions(SoilTempArgs)
 {
+    SOILTEMP_ARGS;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int c;
     GroundFlux gf;
-    if (!column_and_ground_flux<BLOCK>(V, S, Pt, n, filter, wk, err, i, c, gf)) return;
-    int rc = soiltemp_column(V, P, S, Pt, c, dtime, wk, i, gf);
-    if (rc == 0) rc = soilwater_fractions_column(V, S, c);
-    if (rc) report_error(err, c, CTSM_E_SOLVER);
+    if (!column_and_ground_flux<BLOCK>(V, A->S, A->Pt, A->n, A->filter, wk, A->err, i, c, gf, logt)) return;
+    int rc = soiltemp_column(V, P, A->S, A->Pt, c, A->dtime, wk, i, gf, logt);
+    if (rc == 0) rc = soilwater_fractions_column(V, A->S, c);
+    if (rc) report_error(A->err, c, CTSM_E_SOLVER);
 }
 
 // The fused soil step in one kernel: SoilTemperature -> SetSoilWaterFractions -> SoilWater.
 template <bool WT>
 __global__ void __launch_bounds__(64)
-k_soil_step(View V, Params P, ctsm_col_state S, ctsm_patch_state Pt, int n,
-            const int32_t *__restrict__ filter, double dtime, TempWork wk, ErrWord *err)
+k_soil_step(SoilTempArgs)
 {
+    SOILTEMP_ARGS;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int c;
     GroundFlux gf;
-    if (!column_and_ground_flux<64>(V, S, Pt, n, filter, wk, err, i, c, gf)) return;
-    int rc = soiltemp_column(V, P, S, Pt, c, dtime, wk, i, gf);
-    if (rc == 0) rc = soilwater_fractions_column(V, S, c);
-    if (rc == 0) rc = richards_column<MAX_NLEVSOI, WT>(V, P, S, c, dtime);
-    if (rc) report_error(err, c, richards_error_code(rc));
+    if (!column_and_ground_flux<64>(V, A->S, A->Pt, A->n, A->filter, wk, A->err, i, c, gf, logt)) return;
+    int rc = soiltemp_column(V, P, A->S, A->Pt, c, A->dtime, wk, i, gf, logt);
+    if (rc == 0) rc = soilwater_fractions_column(V, A->S, c);
+    if (rc == 0) rc = richards_column<MAX_NLEVSOI, WT>(V, P, A->S, c, A->dtime);
+    if (rc) report_error(A->err, c, richards_error_code(rc));
 }
 
 size_t soiltemp_workspace_doubles(int n) { return (size_t)WS_DOUBLES_PER_COL * (size_t)n; }
@@ -779,7 +829,7 @@ void launch_soiltemp(hipStream_t st, const View &V, const Params &P, const ctsm_
     const GptlRange range("soiltemperature");
     const int bs = 64;
     TempWork wk{ws, ld};
-    hipLaunchKernelGGL(k_soiltemp, dim3((n + bs - 1) / bs), dim3(bs), 0, st, V, P, S, Pt, n, filter, dtime, wk, err);
+    hipLaunchKernelGGL(k_soiltemp, dim3((n + bs - 1) / bs), dim3(bs), 0, st, SoilTempArgs{V, P, S, Pt, n, filter, dtime, wk, err});
 }
 
 void launch_soil_step(hipStream_t st, const View &V, const Params &P, const ctsm_col_state &S,
@@ -791,11 +841,9 @@ void launch_soil_step(hipStream_t st, const View &V, const Params &P, const ctsm
     const int bs = 64;
     TempWork wk{ws, ld};
     if (P.lower_bc == CTSM_BC_WATERTABLE)
-        hipLaunchKernelGGL(k_soil_step<true>, dim3((n + bs - 1) / bs), dim3(bs), 0, st, V, P, S, Pt, n, filter, dtime, wk,
-                           err);
+        hipLaunchKernelGGL(k_soil_step<true>, dim3((n + bs - 1) / bs), dim3(bs), 0, st, SoilTempArgs{V, P, S, Pt, n, filter, dtime, wk, err});
     else
-        hipLaunchKernelGGL(k_soil_step<false>, dim3((n + bs - 1) / bs), dim3(bs), 0, st, V, P, S, Pt, n, filter, dtime,
-                           wk, err);
+        hipLaunchKernelGGL(k_soil_step<false>, dim3((n + bs - 1) / bs), dim3(bs), 0, st, SoilTempArgs{V, P, S, Pt, n, filter, dtime, wk, err});
 }
 
 void launch_soiltemp_fractions(hipStream_t st, const View &V, const Params &P, const ctsm_col_state &S,
@@ -806,11 +854,11 @@ void launch_soiltemp_fractions(hipStream_t st, const View &V, const Params &P, c
     const GptlRange range("soiltemperature");
     TempWork wk{ws, ld};
     if (block == 64)
-        hipLaunchKernelGGL(k_soiltemp_fractions<64>, dim3((n + 63) / 64), dim3(64), 0, st, V, P, S, Pt, n, filter,
-                           dtime, wk, err);
+        hipLaunchKernelGGL(k_soiltemp_fractions<64>, dim3((n + 63) / 64), dim3(64), 0, st,
+                           SoilTempArgs{V, P, S, Pt, n, filter, dtime, wk, err});
     else
-        hipLaunchKernelGGL(k_soiltemp_fractions<128>, dim3((n + 127) / 128), dim3(128), 0, st, V, P, S, Pt, n,
-                           filter, dtime, wk, err);
+        hipLaunchKernelGGL(k_soiltemp_fractions<128>, dim3((n + 127) / 128), dim3(128), 0, st,
+                           SoilTempArgs{V, P, S, Pt, n, filter, dtime, wk, err});
 }
 
 }  // namespace ctsm

@@ -1,13 +1,21 @@
 // soiltemp_dev.h -- per-level thermal properties shared by the fused and the
 // plain soil-temperature kernels (SoilThermProp, SoilTemperatureMod.F90:602-901).
+// lt: log's table.
 #pragma once
 #include "common.h"
 
 namespace ctsm {
 
+// x**y of a conductivity whose log the host has formed
+__device__ __forceinline__ double conductivity_power(double x, const double (&log_x)[2], double y, const double *lt)
+{
+    return fabs(y) < HUGE_VAL ? cm_pow_log(x, log_x[0], log_x[1], y) : cm_pow_tab(x, y, lt);
+}
+
 // Thermal conductivity of level j (SoilThermProp :674-760), non-urban soil.
-__device__ __forceinline__ double level_thk(const View &V, const Params &P, const ctsm_col_state &S,
-                                            int c, int j, int nbedrock, double frac_sno)
+template <class CS>
+__device__ __forceinline__ double level_thk(const View &V, const Params &P, const CS &S,
+                                            int c, int j, int nbedrock, double frac_sno, const double *lt)
 {
     const double liq = S.h2osoi_liq[V.sno(c, j)], ice = S.h2osoi_ice[V.sno(c, j)];
     const double dz = S.dz[V.sno(c, j)];
@@ -18,11 +26,12 @@ __device__ __forceinline__ double level_thk(const View &V, const Params &P, cons
         satw = fmin90(1.0, satw);
         if (satw > .1e-6) {
             double dke;
-            if (S.t_soisno[V.sno(c, j)] >= TFRZ) dke = fmax90(0.0, cm_log10(satw) + 1.0);
+            if (S.t_soisno[V.sno(c, j)] >= TFRZ) dke = fmax90(0.0, cm_log10_tab(satw, lt) + 1.0);
             else dke = satw;
             const double fl = (liq / (DENH2O * dz)) /
                               (liq / (DENH2O * dz) + ice / (DENICE * dz) + 0.0 / (DENICE * dz));
-            const double dksat = S.tkmg[V.soi(c, j)] * cm_pow(TKWAT, fl * ws) * cm_pow(TKICE, (1.0 - fl) * ws);
+            const double dksat = S.tkmg[V.soi(c, j)] * conductivity_power(TKWAT, P.log_tkwat, fl * ws, lt) *
+                                 conductivity_power(TKICE, P.log_tkice, (1.0 - fl) * ws, lt);
             th = dke * dksat + (1.0 - dke) * S.tkdry[V.soi(c, j)];
         } else {
             th = S.tkdry[V.soi(c, j)];
@@ -41,7 +50,8 @@ __device__ __forceinline__ double level_thk(const View &V, const Params &P, cons
 }
 
 // Heat capacity of level j (:826-880).
-__device__ __forceinline__ double level_cv(const View &V, const ctsm_col_state &S, int c, int j,
+template <class CS>
+__device__ __forceinline__ double level_cv(const View &V, const CS &S, int c, int j,
                                            int nbedrock, double frac_sno, double h2osno_no_layers)
 {
     const double liq = S.h2osoi_liq[V.sno(c, j)], ice = S.h2osoi_ice[V.sno(c, j)];

@@ -19,8 +19,8 @@ struct RichardsStatic {
 
 // WT: the water-table bottom boundary (watertable_bc.h), a separate
 // instantiation so the flux / zero-flux kernels keep their registers.
-template <int ML, bool WT = false>
-__device__ __forceinline__ int richards_column(const View &V, const Params &P, const ctsm_col_state &S,
+template <int ML, bool WT = false, class CS>
+__device__ __forceinline__ int richards_column(const View &V, const Params &P, const CS &S,
                                                int c, double dtime)
 {
     const int nl = S.nbedrock[V.c1(c)];
@@ -272,7 +272,8 @@ __device__ __forceinline__ int richards_column(const View &V, const Params &P, c
 }
 
 // Device entry used by the fused soil step.
-__device__ __forceinline__ int soilwater_fractions_column(const View &V, const ctsm_col_state &S, int c)
+template <class CS>
+__device__ __forceinline__ int soilwater_fractions_column(const View &V, const CS &S, int c)
 {
     for (int j = 1; j <= V.nlevsoi; ++j) {
         const double ws = S.watsat[V.soi(c, j)];

@@ -27,7 +27,8 @@ __device__ __forceinline__ int richards_error_code(int rc)
 
 // jwt, the layer above the water table: the first j in 1..nlevsoi with
 // zwt <= zi(j) gives j - 1; nlevsoi when the table is below the column.
-__device__ __forceinline__ int watertable_layer(const View &V, const ctsm_col_state &S, int c)
+template <class CS>
+__device__ __forceinline__ int watertable_layer(const View &V, const CS &S, int c)
 {
     const double zwt = S.zwt[V.c1(c)];
     for (int j = 1; j <= V.nlevsoi; ++j)
@@ -60,7 +61,8 @@ __device__ __forceinline__ double watertable_ka(double vwc, double watsat, doubl
 // qcharge of compute_qcharge for jwt < nlevsoi; smp_w is the last trial's
 // smp of layer max(1, jwt).  The 1.e-3 of the jwt = 0 case is a default-real
 // literal in the reference, so it enters as the binary32 value.
-__device__ __forceinline__ double watertable_qcharge(const View &V, const ctsm_col_state &S, int c, int jwt,
+template <class CS>
+__device__ __forceinline__ double watertable_qcharge(const View &V, const CS &S, int c, int jwt,
                                                      double ka, double smp_w, double dtime)
 {
     const double zwt = S.zwt[V.c1(c)];
