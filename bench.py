@@ -42,26 +42,7 @@ HBM_PEAK_GBS = 8000.0
 # (kernel, workload, columns), with the launch shape they were measured at.
 # The bench reports them only for a run of that workload, size and launch
 # shape; any other run reports null.
-PROFILED = {
-    # profiles/canopy_rounds_canopy_uneven1048576.md: FETCH 8,222,014 KiB x 2.0 + WRITE 17,863,759 KiB
-    # x 1.0 per call; 470.3 GFLOP FP64 in 43.50 ms
-    ("k_canopy_round", "canopy_uneven", 1048576): {
-        "traffic": (8222014 * 2.0 + 17863759 * 1.0) * 1024,
-        "fp64_valu_frac": 470.3e9 / 43.50e-3 / 78.6e12,
-        "tuning": {"canopy_first_iterations": 6, "canopy_round_iterations": 6, "canopy_waves": 1},
-    },
-    # profiles/richards_heat_solve_canopy_uneven1048576.md: the three isolated calls after the steps,
-    # FETCH 3,121,768 KiB x 2.0 + WRITE 2,415,621 KiB x 1.0 (Richards), 4,832,447 x 2.0 + 4,272,971
-    # (heat solve) per call
-    ("k_soilwater_g", "canopy_uneven", 1048576): {
-        "traffic": (3121768 * 2.0 + 2415621 * 1.0) * 1024,
-        "tuning": {"richards_lanes": 8},          # measured in 128-lane blocks; the block size moves no bytes
-    },
-    ("k_soiltemp", "canopy_uneven", 1048576): {
-        "traffic": (4832447 * 2.0 + 4272971 * 1.0) * 1024,
-        "tuning": {},
-    },
-}
+PROFILED = {}       # none for the kernels as they are
 
 
 def richards_bytes(st):

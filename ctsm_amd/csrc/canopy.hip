@@ -812,7 +812,8 @@ static_assert(sizeof(CanopyWork) == N_WORK_FIELDS * sizeof(double *), "one point
 // All three are bound by the issue of FP64 and scalar instructions and by the waits
 // of one or two waves per SIMD; HBM is at a sixth of its rate.  On 1,048,576 columns
 // (8.9 million patches) the one kernel took 31.4 ms for its first round and 43.6 ms
-// in all; the set-up 4.1, the rounds 24.7 and the finish 2.1 ms now.
+// in all; the set-up takes 4.1, the rounds 25.5 (the first 16.4) and the finish
+// 2.0 ms now.
 
 // The column-level half of calc_effective_soilporosity, calc_volumetric_h2oliq
 // and calc_root_moist_stress (SoilMoistStressMod.F90:70-126, 190-240,
