@@ -788,13 +788,16 @@ __device__ __forceinline__ void temp_factors(const PRM &P, const DRV &D, const P
 
 // What a patch keeps between the kernels of a call, indexed by its position in
 // the filter (structure of arrays).  Between rounds: the iteration state.  Once it
-// has finished: what the outputs are formed from and no output array holds --
-// FrictionVelocity's last um, obu and fm, temp1 in qsatl, temp2 in el, the leaf
-// temperature before the last step in t_veg and the step in del, rpp in efeb, wtgq
-// in qsatldT.  itlef: the iterations done, -1 for a patch whose set-up failed.
+// has finished: what the outputs are formed from -- FrictionVelocity's last um, obu
+// and fm, its ustar in nmozsgn, temp1 in qsatl and temp2 in el, the leaf temperature
+// before the last step in t_veg and the step in del, rpp in efeb, wtgq in qsatldT,
+// rah2 in taf, eflx_sh_veg in qaf, qflx_evap_veg in delq, qflx_tran_veg in gs_mol.
+// itlef: the iterations done, -1 for a patch whose set-up failed.  No kernel reads
+// an output array of CanopyFluxes back: a caller may point those it does not want
+// at one array.
 struct CanopyWork {
     double *t_veg, *del, *efeb, *nmozsgn, *um, *obu, *fm, *qsatl, *el, *qsatldT, *taf, *qaf, *delq, *itlef, *gs_mol,
-        *unused;
+        *btran;
 };
 constexpr int N_WORK_FIELDS = 16;
 static_assert(sizeof(CanopyWork) == N_WORK_FIELDS * sizeof(double *), "one pointer per saved value");
@@ -812,8 +815,9 @@ static_assert(sizeof(CanopyWork) == N_WORK_FIELDS * sizeof(double *), "one point
 // All three are bound by the issue of FP64 and scalar instructions and by the waits
 // of one or two waves per SIMD; HBM is at a sixth of its rate.  On 1,048,576 columns
 // (8.9 million patches) the one kernel took 31.4 ms for its first round and 43.6 ms
-// in all; the set-up takes 4.1, the rounds 25.5 (the first 16.4) and the finish
-// 2.0 ms now.
+// in all; the set-up takes 4.1, the rounds 26.6 (the first 17.0) and the finish
+// 2.0 ms now.  (With the finish reading the outputs back, 0.3 ms less; the totals
+// would then depend on the caller's arrays being distinct.)
 
 // The column-level half of calc_effective_soilporosity, calc_volumetric_h2oliq
 // and calc_root_moist_stress (SoilMoistStressMod.F90:70-126, 190-240,
@@ -892,8 +896,8 @@ __device__ void soil_terms_of_runs(const CView &V, const COL &col, const CAN &S,
 // Root moisture stress of one patch from its column's terms (SoilMoistStressMod.
 // F90:420-514): rresis, rootr normalised by btran (:480-500), btran.
 template <class CAN>
-__device__ __forceinline__ void root_stress(const CView &V, const CAN &S, const double *__restrict__ pft, int p, int ivt,
-                                            const SoilTerms *soil)
+__device__ __forceinline__ double root_stress(const CView &V, const CAN &S, const double *__restrict__ pft, int p,
+                                              int ivt, const SoilTerms *soil)
 {
     const double smpsc = PF(F_SMPSC), smpso = PF(F_SMPSO);
     double btran = 0.0;
@@ -919,6 +923,7 @@ __device__ __forceinline__ void root_stress(const CView &V, const CAN &S, const 
     for (int j = 0; j < MAX_NLEVGRND; ++j)
         if (j < V.nlevgrnd) S.rootr[V.soip(p, j + 1)] = (btran > 0.0) ? rr[j] / btran : 0.0;
     S.btran[V.p1(p)] = btran;
+    return btran;
 }
 
 // The set-up of one patch after its root stress: roughness, leaf humidity,
@@ -1163,6 +1168,37 @@ __device__ __forceinline__ void store_shared(const CAN &S, uint32_t po, const CS
     if (medlyn && (lit_sun || lit_sha)) at(S.vpd_can, po) = sh.vpd_can;
 }
 
+// A phase's photosynthesis and conductance as the canopy's totals need them: the rate
+// that limits it (0: none, 1: Rubisco, 2: light, 3: product) says which of psn_wc,
+// psn_wj and psn_wp is psn, the others being zero.
+struct PhaseSums {
+    double psn = 0.0, gs = 0.0;
+    int limit = 0;
+    PhaseSums() = default;
+    __device__ explicit PhaseSums(const Phase &ph)
+        : psn(ph.psn), gs(ph.gs_ph), limit(ph.psn_wc != 0.0 ? 1 : ph.psn_wj != 0.0 ? 2 : ph.psn_wp != 0.0 ? 3 : 0)
+    {
+    }
+    __device__ double of(int rate) const { return limit == rate ? psn : 0.0; }
+};
+// PhotosynthesisTotal and the noon water-use efficiency, in a pass that can be the last.
+template <class CAN>
+__device__ __forceinline__ void store_totals(const CAN &S, uint32_t po, bool noon, double laisun, double laisha,
+                                             const PhaseSums &sun, const PhaseSums &sha)
+{
+    const double fpsn = sun.psn * laisun + sha.psn * laisha;
+    at(S.fpsn, po) = fpsn;
+    at(S.fpsn_wc, po) = sun.of(1) * laisun + sha.of(1) * laisha;
+    at(S.fpsn_wj, po) = sun.of(2) * laisun + sha.of(2) * laisha;
+    at(S.fpsn_wp, po) = sun.of(3) * laisun + sha.of(3) * laisha;
+    double iwue = SPVAL;
+    if (noon && fpsn > 0.0) {
+        const double gs = 1.e-6 * (laisun * sun.gs + laisha * sha.gs);
+        iwue = (gs > 0.0) ? fpsn / gs : SPVAL;
+    }
+    at(S.iwue_ln, po) = iwue;
+}
+
 // Step constants of the iteration that wait in LDS ([KC_N][64], the lane's column)
 // instead of in registers: with log's table 20,104 bytes a wave, room for two waves
 // per SIMD.  Values formed from them in a few operations are formed anew.
@@ -1185,7 +1221,8 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
                              int budget, const WRK &W, const PHA &H, const DRV &D, const double *lt, double *kc,
                              double *phs_lane)
 {
-    const double it_done = W.itlef[i0];
+    uint32_t wo = (uint32_t)i0 * 8u;
+    const double it_done = at(W.itlef, wo);
     if (it_done < 0.0) return false;
     const long pp = V.p1(p);
     const int c = S.column[pp];
@@ -1203,7 +1240,7 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
     const bool noon = S.near_local_noon[gg] != 0;
     const bool anyday = nrad >= 1 && (parsun > 0.0 || parsha > 0.0);
     const bool medlyn = sw.stomatal == CTSM_STOMATA_MEDLYN2011;
-    double btran = S.btran[pp], sa_lw;
+    double btran = at(W.btran, wo), sa_lw;
     bool c3;
     {
         const double elai = S.elai[pp], esai = S.esai[pp], emv = S.emv[pp], emg = col.emg[cc];
@@ -1267,31 +1304,32 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
         kc[KC_UR * 64] = fmax90(P.wind_min, sqrt(fu * fu + fvv * fvv));
     }
     // ---- the iteration's state
-    double t_veg = W.t_veg[i0], qsatl = W.qsatl[i0], el = W.el[i0], qsatldT = W.qsatldT[i0], taf = W.taf[i0],
-           qaf = W.qaf[i0], delq = W.delq[i0], um = W.um[i0], obu = W.obu[i0];
-    int nmozsgn = (int)W.nmozsgn[i0];
-    double gs_mol_c = W.gs_mol[i0];
-    double del = W.del[i0], efeb = W.efeb[i0], fm_c = W.fm[i0];
+    double t_veg = at(W.t_veg, wo), qsatl = at(W.qsatl, wo), el = at(W.el, wo), qsatldT = at(W.qsatldT, wo),
+           taf = at(W.taf, wo), qaf = at(W.qaf, wo), delq = at(W.delq, wo), um = at(W.um, wo), obu = at(W.obu, wo);
+    int nmozsgn = (int)at(W.nmozsgn, wo);
+    double gs_mol_c = at(W.gs_mol, wo);
+    double del = at(W.del, wo), efeb = at(W.efeb, wo), fm_c = at(W.fm, wo);
     int itlef = (int)it_done;
     const uint32_t po0 = (uint32_t)pp * 8u, co0 = (uint32_t)cc * 8u, go0 = (uint32_t)gg * 8u;
     for (int it = 0;; ++it) {
         if (it >= budget) {
             // still iterating: keep the state for the next round
-            W.t_veg[i0] = t_veg;
-            W.del[i0] = del;
-            W.efeb[i0] = efeb;
-            W.nmozsgn[i0] = (double)nmozsgn;
-            W.um[i0] = um;
-            W.obu[i0] = obu;
-            W.fm[i0] = fm_c;
-            W.qsatl[i0] = qsatl;
-            W.el[i0] = el;
-            W.qsatldT[i0] = qsatldT;
-            W.taf[i0] = taf;
-            W.qaf[i0] = qaf;
-            W.delq[i0] = delq;
-            W.itlef[i0] = (double)itlef;
-            W.gs_mol[i0] = gs_mol_c;
+            at(W.t_veg, wo) = t_veg;
+            at(W.del, wo) = del;
+            at(W.efeb, wo) = efeb;
+            at(W.nmozsgn, wo) = (double)nmozsgn;
+            at(W.um, wo) = um;
+            at(W.obu, wo) = obu;
+            at(W.fm, wo) = fm_c;
+            at(W.qsatl, wo) = qsatl;
+            at(W.el, wo) = el;
+            at(W.qsatldT, wo) = qsatldT;
+            at(W.taf, wo) = taf;
+            at(W.qaf, wo) = qaf;
+            at(W.delq, wo) = delq;
+            at(W.itlef, wo) = (double)itlef;
+            at(W.gs_mol, wo) = gs_mol_c;
+            if (PHS) at(W.btran, wo) = btran;
             if (bad) report_error(err, p, ENDRUN);
             return true;
         }
@@ -1302,7 +1340,7 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
         // constants are read where they are used, not held in registers across the
         // loop or the pass)
 #define KC(name) kc[KC_##name * 64 + k_]
-#define OPAQUE asm volatile("" : "+v"(k_), "+v"(po), "+v"(co), "+v"(go))
+#define OPAQUE asm volatile("" : "+v"(k_), "+v"(po), "+v"(co), "+v"(go), "+v"(wo))
         uint32_t po = po0, co = co0, go = go0;
         int k_ = 0;
         OPAQUE;
@@ -1340,19 +1378,13 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
         const double svpts = el;
         const double eah = at(S.forc_pbot, co) * qaf / 0.622;
         if (last) {
-            W.obu[i0] = obu;        // the inputs of this FrictionVelocity call
-            W.um[i0] = um;
-            W.fm[i0] = fv.fm;
-            W.qsatl[i0] = temp1;
-            W.el[i0] = temp2;
-            at(S.ustar, po) = ustar;
-            at(S.ram1, po) = ram1;
-            at(S.rah1, po) = rah1;
-            at(S.raw1, po) = raw1;
-            at(S.rah2, po) = rah2;
-            at(S.raw2, po) = raw2;
-            at(S.uaf, po) = uaf;
-            at(S.rb1, po) = rb;
+            at(W.obu, wo) = obu;        // the inputs of this FrictionVelocity call
+            at(W.um, wo) = um;
+            at(W.fm, wo) = fv.fm;
+            at(W.qsatl, wo) = temp1;
+            at(W.el, wo) = temp2;
+            at(W.nmozsgn, wo) = ustar;
+            at(W.taf, wo) = rah2;
             at(S.rh_af, po) = eah / svpts;
             at(S.vpd, po) = fmax90((svpts - eah), 50.0) * 0.001;
         }
@@ -1389,16 +1421,18 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
                 Phase sun = Phase{}, sha = Phase{};
                 btran = photosynthesis_phs(V, sw, P, K, T, H, S, p, c, ivt, nrad, noon, forc_pbot, thm, svpts, eah, o2,
                                            co2, rb, qsatl, qaf, sun, sha, sh, bad, phs_lane, lt);
-                at(S.btran, po) = btran;
                 qflx_tran_veg = at(S.qflx_tran_veg, po);
                 rs_sun = sun.rs;
                 rs_sha = sha.rs;
                 if (last) {
+                    at(W.btran, wo) = btran;
                     store_phase<PHS>(S, po, true, sun, nrad, false);
                     store_phase<PHS>(S, po, false, sha, nrad, false);
+                    store_totals(S, po, noon, KC(LAISUN), KC(LAISHA), PhaseSums(sun), PhaseSums(sha));
                 }
             } else {
                 rs_sun = rs_sha = 0.0;
+                PhaseSums sun{};
                 // one call site for both phases: sun (k = 0), then shade
 #pragma nounroll
                 for (int k = 0; k < 2; ++k) {
@@ -1409,9 +1443,16 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
                                    ks ? S.vcmaxcintsun : S.vcmaxcintsha, ks ? S.o3coefvsun : S.o3coefvsha,
                                    ks ? S.o3coefgsun : S.o3coefgsha, po,
                                    noon, forc_pbot, thm, svpts, eah, o2, co2, rb, btran, ph, sh, bad);
-                    if (ks) rs_sun = ph.rs;
-                    else rs_sha = ph.rs;
-                    if (last) store_phase<PHS>(S, po, ks, ph, nrad, nrad >= 1 && par > 0.0);
+                    if (last) {
+                        store_phase<PHS>(S, po, ks, ph, nrad, nrad >= 1 && par > 0.0);
+                        if (!ks) store_totals(S, po, noon, KC(LAISUN), KC(LAISHA), sun, PhaseSums(ph));
+                    }
+                    if (ks) {
+                        rs_sun = ph.rs;
+                        sun = PhaseSums(ph);
+                    } else {
+                        rs_sha = ph.rs;
+                    }
                 }
             }
             if (last) store_shared<PHS>(S, po, sw, sh, nrad, parsun, parsha);
@@ -1467,9 +1508,6 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
         const double dc1 = forc_rho * CPAIR * hw.wtl;
         const double dc2 = HVAP * forc_rho * mw.wtlq;
         const double efsh = dc1 * (hw.wtga * t_veg - hw.wtg0 * t_grnd - hw.wta0 * thm - hw.wtstem0 * t_stem);
-        double eflx_sh_stem = forc_rho * CPAIR * hw.wtstem
-                              * ((hw.wta0 + hw.wtg0 + hw.wtl0) * t_stem - hw.wtg0 * t_grnd - hw.wta0 * thm
-                                 - hw.wtl0 * t_veg);
         double efe = dc2 * (mw.wtgaq * qsatl - mw.wtgq0 * qg - mw.wtaq0 * forc_q);
         double erre = 0.0;
         if (efe * efeb < 0.0) {
@@ -1504,7 +1542,6 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
         const double ecidif = fmax90(0.0, qflx_evap_veg - qflx_tran_veg - h2ocan_dt);
         qflx_evap_veg = fmin90(qflx_evap_veg, qflx_tran_veg + h2ocan_dt);
         const double eflx_sh_veg = efsh + dc1 * hw.wtga * dt_veg + errp + erre + HVAP * ecidif;
-        eflx_sh_stem = eflx_sh_stem + forc_rho * CPAIR * hw.wtstem * (-hw.wtl0 * dt_veg);
         qsat(t_veg, at(S.forc_pbot, co), qsatl, el, qsatldT);
         taf = hw.wtg0 * t_grnd + hw.wta0 * thm + hw.wtl0 * t_veg + hw.wtstem0 * t_stem;
         qaf = mw.wtlq0 * qsatl + mw.wtgq0 * qg + forc_q * mw.wtaq0;
@@ -1545,18 +1582,15 @@ __device__ __forceinline__ bool canopy_iterate_patch(const CView &V, const CSwit
             converged = det < dtmin && dele < dlemin;
         }
         if (last) {
-            W.t_veg[i0] = tlbef;
-            W.del[i0] = dt_veg;
-            W.efeb[i0] = rpp;
-            W.qsatldT[i0] = wtgq;
-            at(S.eflx_sh_stem, po) = eflx_sh_stem;
-            at(S.eflx_sh_veg, po) = eflx_sh_veg;
-            at(S.qflx_tran_veg, po) = qflx_tran_veg;
-            at(S.qflx_evap_veg, po) = qflx_evap_veg;
+            at(W.t_veg, wo) = tlbef;
+            at(W.del, wo) = dt_veg;
+            at(W.efeb, wo) = rpp;
+            at(W.qsatldT, wo) = wtgq;
+            at(W.qaf, wo) = eflx_sh_veg;
+            at(W.delq, wo) = qflx_evap_veg;
+            at(W.gs_mol, wo) = qflx_tran_veg;
             at(S.um, po) = um;
             at(S.obu, po) = obu;
-            at(S.taf, po) = taf;
-            at(S.qaf, po) = qaf;
             at(S.zeta, po) = zeta;
             at(S.num_iter, po) = num_iter;
         }
@@ -1585,10 +1619,8 @@ __device__ __forceinline__ void canopy_finish_patch(const CView &V, const CSwitc
     const double forc_pbot = S.forc_pbot[cc], forc_q = S.forc_q[cc], forc_rho = S.forc_rho[cc];
     const double qg = S.qg[cc], t_grnd = col.t_grnd[cc];
     const double fu = S.forc_u[gg], fvv = S.forc_v[gg];
-    const double laisun = S.laisun[pp], laisha = S.laisha[pp];
     const double sabv = S.sabv[pp], dleaf = PF(F_DLEAF);
     const double liqcan0 = S.liqcan[pp], snocan0 = S.snocan[pp];
-    const bool noon = S.near_local_noon[gg] != 0;
     Biomass B;
     biomass(sw, P, pft, ivt, elai, esai, htop, B);
     if (sw.biomass) {
@@ -1604,27 +1636,38 @@ __device__ __forceinline__ void canopy_finish_patch(const CView &V, const CSwitc
     const double displa = S.displa[pp], z0mv = S.z0mv[pp];
     const double hu = S.forc_hgt_u[gg] + z0mv + displa;
     const double ur = fmax90(P.wind_min, sqrt(fu * fu + fvv * fvv));
+    const double um = W.um[i0];
     FV fv;
-    fv.ustar = S.ustar[pp];
+    fv.ustar = W.nmozsgn[i0];
     fv.fm = W.fm[i0];
-    friction_velocity_diag(hu, displa, z0mv, z0mv, z0mv, W.obu[i0], ur, W.um[i0], fv, lt);
+    friction_velocity_diag(hu, displa, z0mv, z0mv, z0mv, W.obu[i0], ur, um, fv, lt);
 
     // ---- the last pass again, from what it left
     const double temp1 = W.qsatl[i0], temp2 = W.el[i0];
     const double tlbef = W.t_veg[i0], dt_veg = W.del[i0];
     const double t_veg = tlbef + dt_veg;
-    const double wtgq = W.qsatldT[i0];
-    const double ram1 = S.ram1[pp], rb = S.rb1[pp];
-    const HeatWeights hw = heat_weights(S.rah1[pp], rb, S.rah2[pp], B.sa_leaf, B.sa_stem, B.rstem);
-    const MoistureWeights mw = moisture_weights((double)S.frac_veg_nosno[pp], elai + esai, S.raw1[pp], rb, W.efeb[i0],
-                                                wtgq);
+    const double wtgq = W.qsatldT[i0], rah2 = W.taf[i0], btran = W.btran[i0];
+    const double ram1 = 1.0 / (fv.ustar * fv.ustar / um);
+    const double rah1 = 1.0 / (temp1 * fv.ustar);
+    const double raw1 = 1.0 / (temp2 * fv.ustar);
+    const double uaf = um * sqrt(1.0 / (ram1 * um));
+    const double cf = P.cv / (sqrt(uaf) * sqrt(dleaf));
+    const double rb = 1.0 / (cf * uaf);
+    const HeatWeights hw = heat_weights(rah1, rb, rah2, B.sa_leaf, B.sa_stem, B.rstem);
+    const MoistureWeights mw = moisture_weights((double)S.frac_veg_nosno[pp], elai + esai, raw1, rb, W.efeb[i0], wtgq);
     double qsatl, el, qsatldT;
     qsat(t_veg, forc_pbot, qsatl, el, qsatldT);
-    const double dth = thm - S.taf[pp];
-    const double dqh = forc_q - S.qaf[pp];
+    const double taf = hw.wtg0 * t_grnd + hw.wta0 * thm + hw.wtl0 * t_veg + hw.wtstem0 * ts_ini;
+    const double qaf = mw.wtlq0 * qsatl + mw.wtgq0 * qg + forc_q * mw.wtaq0;
+    const double dth = thm - taf;
+    const double dqh = forc_q - qaf;
     const double delq = mw.wtalq * qg - mw.wtlq0 * qsatl - mw.wtaq0 * forc_q;
-    const double eflx_sh_veg = S.eflx_sh_veg[pp], eflx_sh_stem = S.eflx_sh_stem[pp];
-    const double qflx_evap_veg = S.qflx_evap_veg[pp], qflx_tran_veg = S.qflx_tran_veg[pp];
+    const double eflx_sh_veg = W.qaf[i0];
+    double eflx_sh_stem = forc_rho * CPAIR * hw.wtstem
+                          * ((hw.wta0 + hw.wtg0 + hw.wtl0) * ts_ini - hw.wtg0 * t_grnd - hw.wta0 * thm
+                             - hw.wtl0 * tlbef);
+    eflx_sh_stem = eflx_sh_stem + forc_rho * CPAIR * hw.wtstem * (-hw.wtl0 * dt_veg);
+    const double qflx_evap_veg = W.delq[i0], qflx_tran_veg = W.gs_mol[i0];
     const double lw_stem = B.sa_internal * emv * SB * p4(ts_ini);
     const double lw_leaf = B.sa_internal * emv * SB * p3(tlbef) * (tlbef + 4.0 * dt_veg);
 
@@ -1712,21 +1755,22 @@ __device__ __forceinline__ void canopy_finish_patch(const CView &V, const CSwitc
     S.snocan[pp] = snocan;
     S.liqcan[pp] = liqcan;
 
-    // ---- PhotosynthesisTotal and the noon water-use efficiency
-    const double psn_sun = S.psnsun[pp], psn_sha = S.psnsha[pp];
-    const double fpsn = psn_sun * laisun + psn_sha * laisha;
-    S.fpsn[pp] = fpsn;
-    S.fpsn_wc[pp] = S.psnsun_wc[pp] * laisun + S.psnsha_wc[pp] * laisha;
-    S.fpsn_wj[pp] = S.psnsun_wj[pp] * laisun + S.psnsha_wj[pp] * laisha;
-    S.fpsn_wp[pp] = S.psnsun_wp[pp] * laisun + S.psnsha_wp[pp] * laisha;
-    double iwue = SPVAL;
-    if (noon && fpsn > 0.0) {       // fpsn > 0 only where nrad >= 1, whose phases have written gs_mol
-        const double gs = 1.e-6 * (laisun * S.gs_mol_sun[pp] + laisha * S.gs_mol_sha[pp]);
-        iwue = (gs > 0.0) ? fpsn / gs : SPVAL;
-    }
-    S.iwue_ln[pp] = iwue;
-
     // ---- remaining outputs
+    if (PHS) S.btran[pp] = btran;       // (otherwise the set-up's)
+    S.ustar[pp] = fv.ustar;
+    S.ram1[pp] = ram1;
+    S.rah1[pp] = rah1;
+    S.raw1[pp] = raw1;
+    S.rah2[pp] = rah2;
+    S.raw2[pp] = rah2;
+    S.uaf[pp] = uaf;
+    S.rb1[pp] = rb;
+    S.taf[pp] = taf;
+    S.qaf[pp] = qaf;
+    S.eflx_sh_stem[pp] = eflx_sh_stem;
+    S.eflx_sh_veg[pp] = eflx_sh_veg;
+    S.qflx_evap_veg[pp] = qflx_evap_veg;
+    S.qflx_tran_veg[pp] = qflx_tran_veg;
     S.dhsdt_canopy[pp] = dhsdt_canopy;
     S.t_veg[pp] = t_veg;
     S.t_stem[pp] = t_stem;
@@ -1740,7 +1784,7 @@ __device__ __forceinline__ void canopy_finish_patch(const CView &V, const CSwitc
     // photosyns_inst
     PsnConst K;
     bool bad = false;       // the iteration has reported it
-    psn_static(sw, pft, ivt, PHS ? 0.0 : S.btran[pp], K, bad, PHS);
+    psn_static(sw, pft, ivt, PHS ? 0.0 : btran, K, bad, PHS);
     S.c3flag[pp] = K.c3 ? 1 : 0;
     S.qe[pp] = K.qe;
     if (sw.stomatal == CTSM_STOMATA_BB1987) {
@@ -1814,7 +1858,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     for (int r0 = 0; r0 < nruns; r0 += SOIL_RUNS) {
         soil_terms_of_runs(V, A->col, A->S, run_col, r0, nruns, terms, logt);
         if (run >= r0 && run < r0 + SOIL_RUNS)
-            root_stress(V, A->S, A->pft, p, ivt, terms + (run - r0) * MAX_NLEVGRND);
+            A->W.btran[i0] = root_stress(V, A->S, A->pft, p, ivt, terms + (run - r0) * MAX_NLEVGRND);
     }
     if (!active) return;
     if (run < 0) {      // an index that addresses other arrays lies outside their allocations
@@ -1834,7 +1878,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
 // opaque on every pass, so its loads stay inside the pass instead of being
 // hoisted in front of the loop.
 // WAVES: the register budget the kernel is compiled for (waves per SIMD).  One wave
-// needs 310 registers; the two-wave instance (256, and 240 B/lane of scratch) pays
+// needs 310 registers; the two-wave instance (256, and 176 B/lane of scratch) pays
 // once a filter has a second wave for the SIMDs: launch_canopy has the rule.
 // PHS: CanopyFluxes with plant hydraulic stress (argument RoundArgsPhs).
 template <int WAVES, bool STRIDE, bool PHS = false>
