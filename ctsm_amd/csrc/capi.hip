@@ -344,6 +344,7 @@ int nlev_of(Kind k, const ctsm_config &cfg)
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
+    size_t refused = 0;     // the smallest size ensure_up_to has not been given (0: none)
     hipError_t ensure(size_t b)
     {
         if (b <= bytes) return hipSuccess;
@@ -353,6 +354,19 @@ struct DevBuf {
         hipError_t e = hipMalloc(&p, b);
         if (e == hipSuccess) bytes = b;
         return e;
+    }
+    // b bytes or, where the device has not that much, the largest of b / 2, b / 4, ...
+    // that it has, `least` at the end.  What it has refused once is not asked for
+    // again while `least` is there.
+    hipError_t ensure_up_to(size_t b, size_t least)
+    {
+        if (b <= bytes || (refused && b >= refused && bytes >= least)) return hipSuccess;
+        for (;; b = std::max(b / 2, least)) {
+            const hipError_t e = ensure(b);
+            if (e != hipErrorOutOfMemory || b <= least) return e;
+            (void)hipGetLastError();
+            refused = b;
+        }
     }
     void release()
     {
@@ -1084,10 +1098,31 @@ static int check_canopy_layout(const ctsm_ctx *ctx, const ctsm_layout *L)
     return CTSM_OK;
 }
 
+// The rounds of the context's CanopyFluxes: iterations of the first and of the next.
+static void canopy_rounds(const ctsm_ctx *ctx, int &first, int &later)
+{
+    const bool one_pass = ctx->tun.plain_routines != 0;
+    first = one_pass ? 1001 : ctx->tun.canopy_first_iterations;
+    later = one_pass ? 1 : ctx->tun.canopy_round_iterations;
+}
+
+// Grows buf for CanopyFluxes of n patches.  An iteration without rounds takes a
+// shorter buffer too, and goes over the filter in parts.
+static hipError_t ensure_canopy_work(const ctsm_ctx *ctx, DevBuf &buf, int n)
+{
+    int k0, k;
+    canopy_rounds(ctx, k0, k);
+    const int itmax = ctx->cfg.itmax_canopy_fluxes;
+    const size_t wb = canopy_work_bytes(n, itmax, k0, k);
+    if (wb == 0) return hipSuccess;
+    if (canopy_one_pass_patches(wb, itmax, k0, k) == 0) return buf.ensure(wb);
+    return buf.ensure_up_to(wb, canopy_work_bytes(std::min(n, 64), itmax, k0, k));
+}
+
 // Grows the canopy work buffer to n patches and launches CanopyFluxes.
 // With fixed_work, the kernels use that buffer of fixed_bytes instead and
-// nothing is allocated (CTSM_E_SCRATCH when it is too small for the rounds; an
-// iteration without rounds goes over the filter in parts that fit).  With
+// nothing is allocated (CTSM_E_SCRATCH when it is too small for the rounds).  An
+// iteration without rounds goes over the filter in parts that fit its buffer.  With
 // bounds_are_filter the per-step resets of the bounds (rb1, the
 // photosynthesis outputs) cover the filter's patches instead of the whole
 // layout: a caller whose layout holds other, independent runs (the ensemble
@@ -1099,9 +1134,8 @@ static int run_canopy(ctsm_ctx *ctx, const ctsm_layout *lay, const ctsm_col_stat
 {
     // the configuration fixes the form: the PHS one only through the ctsm_canopyfluxes_phs entries
     if ((ctx->cfg.use_hydrstress != 0) != (phs_h != nullptr)) return CTSM_E_CONFIG;
-    const bool one_pass = ctx->tun.plain_routines != 0;
-    const int k0 = one_pass ? 1001 : ctx->tun.canopy_first_iterations;
-    const int k = one_pass ? 1 : ctx->tun.canopy_round_iterations;
+    int k0, k;
+    canopy_rounds(ctx, k0, k);
     const size_t wb = canopy_work_bytes(n, ctx->cfg.itmax_canopy_fluxes, k0, k);
     void *work = nullptr;
     int part = 0;
@@ -1114,9 +1148,11 @@ static int run_canopy(ctsm_ctx *ctx, const ctsm_layout *lay, const ctsm_col_stat
         }
         work = fixed_work;
     } else if (wb) {
-        hipError_t he = ctx->cwork.ensure(wb);
+        hipError_t he = ensure_canopy_work(ctx, ctx->cwork, n);
         if (he != hipSuccess) return hip_fail(ctx, he);
         work = ctx->cwork.p;
+        if (wb > ctx->cwork.bytes)
+            part = canopy_one_pass_patches(ctx->cwork.bytes, ctx->cfg.itmax_canopy_fluxes, k0, k);
     }
     launch_canopy(ctx->stream, *lay, ctx->cfg, ctx->cprm, (const double *)ctx->pft.p, col, can, n, filter_dev, dtime,
                   ctx->err, work, part, k0, k, zero_cgrnd, ctx->tun.canopy_waves, bounds_are_filter, phs_q, phs_h,
@@ -1214,10 +1250,7 @@ static int capture_graph(ctsm_ctx *ctx, int32_t nc, int32_t np, bool canopy, cts
     he = gr->work.ensure(std::max<size_t>(std::max(step_work_doubles(ctx, nc), land_work_doubles(ctx, nc)), 1) *
                          sizeof(double));
     if (he == hipSuccess && step_partf_bytes(ctx, nc)) he = gr->partf.ensure(step_partf_bytes(ctx, nc));
-    const size_t cwb = canopy ? canopy_work_bytes(np, ctx->cfg.itmax_canopy_fluxes, ctx->tun.canopy_first_iterations,
-                                                  ctx->tun.canopy_round_iterations)
-                              : 0;
-    if (he == hipSuccess && cwb) he = gr->cwork.ensure(cwb);
+    if (he == hipSuccess && canopy) he = ensure_canopy_work(ctx, gr->cwork, np);
     if (he != hipSuccess) {
         ctsm_graph_destroy(gr);
         return hip_fail(ctx, he);

@@ -606,7 +606,9 @@ typedef struct ctsm_phs_canopy_state {
  *   canopy_round_iterations more, the following ones for twice as many as the one
  *   before.  A filter of at most 65,536 patches takes a single later round.
  *   canopy_first_iterations > itmax_canopy_fluxes runs the whole iteration in one
- *   pass.  Both >= 1; results do not depend on them.
+ *   pass, over the filter in parts where the device has no memory for the work
+ *   buffer of all its patches (128 B each).  Both >= 1; results do not depend on
+ *   them.
  * step_streams: the fused soil step splits its filter into this many
  *   contiguous parts run on as many streams of the context at once, joined
  *   before the call's later work (1..4).  A batch stored in work-binned
