@@ -376,6 +376,15 @@ struct DevBuf {
     }
 };
 
+// Device mirrors of one struct of host arrays: a buffer per field, or all fields
+// packed in the buffer behind those (mirror()).
+struct Mirrors {
+    std::vector<DevBuf> bufs;
+    bool packed = false;        // where the fields of the last copy to the device lie
+    std::vector<DevBuf>::iterator begin() { return bufs.begin(); }
+    std::vector<DevBuf>::iterator end() { return bufs.end(); }
+};
+
 // Streaming copy: 16 B per lane per iteration, grid-stride.
 __global__ void __launch_bounds__(256) k_copy16(uint4 *__restrict__ dst, const uint4 *__restrict__ src, size_t n16)
 {
@@ -425,23 +434,23 @@ struct ctsm_ctx {
     ErrWord *err = nullptr;            // device
     DevBuf work;                       // heat-solve workspace
     DevBuf filt;                       // filter (drop-in mode)
-    std::vector<DevBuf> colmir, pchmir; // drop-in mirrors
-    std::vector<DevBuf> canp, canc, cang; // canopy drop-in mirrors
+    Mirrors colmir, pchmir; // drop-in mirrors
+    Mirrors canp, canc, cang; // canopy drop-in mirrors
     ctsm_canopy_params cprm{};         // canopy param-file scalars
     DevBuf pft;                        // PFT table (N_PFT_FIELDS x CTSM_MAX_PFT doubles)
     DevBuf cwork;                      // CanopyFluxes round state, patch lists and counters
     DevBuf filt2;                      // second filter (drop-in calls taking column and patch filters)
     DevBuf bal;                        // balance-check reduction word
-    std::vector<DevBuf> sfp, sfc;      // SoilFluxes drop-in mirrors
-    std::vector<DevBuf> swm;           // surface-water drop-in mirrors
-    std::vector<DevBuf> wtm;           // water-table drop-in mirrors
-    std::vector<DevBuf> drm;           // drainage drop-in mirrors
-    std::vector<DevBuf> phsp, phsc;    // plant-hydraulics drop-in mirrors
+    Mirrors sfp, sfc;      // SoilFluxes drop-in mirrors
+    Mirrors swm;           // surface-water drop-in mirrors
+    Mirrors wtm;           // water-table drop-in mirrors
+    Mirrors drm;           // drainage drop-in mirrors
+    Mirrors phsp, phsc;    // plant-hydraulics drop-in mirrors
     DevBuf phs_tab;                    // PHS parameter table (17 x CTSM_MAX_PFT doubles)
     int32_t phs_npft = 0;              // 0 until ctsm_set_phs_params
     bool phs_kmax = false;             // the table holds kmax (calcstress may run)
-    std::vector<DevBuf> stp, stc;      // calcstress drop-in mirrors
-    std::vector<DevBuf> phcm;          // PHS CanopyFluxes drop-in mirrors
+    Mirrors stp, stc;      // calcstress drop-in mirrors
+    Mirrors phcm;          // PHS CanopyFluxes drop-in mirrors
     char *stage = nullptr;             // pinned staging of the drop-in copies
     size_t stage_size = 0, stage_used = 0;
     bool have_canopy = false;
@@ -542,9 +551,11 @@ Range filter_range(int n, const int32_t *f, int def_lo)
 // 35.5 and 2.2, 16,384 (99 MB a call) 50.6 and 27.5, 32,768 66.7 and 53.4 ms.
 constexpr size_t kStageBytes = 128u << 20;
 
-// `bytes` of staging that no copy in flight uses.
+// `bytes` of staging that no copy in flight uses; null where there is no pinned memory
+// for them.
 int stage_room(ctsm_ctx *ctx, size_t bytes, char **p)
 {
+    *p = nullptr;
     if (ctx->stage_used + bytes > ctx->stage_size) {
         hipError_t e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, e);
@@ -554,8 +565,11 @@ int stage_room(ctsm_ctx *ctx, size_t bytes, char **p)
             ctx->stage = nullptr;
             ctx->stage_size = 0;
             const size_t want = std::min(std::max<size_t>(2 * bytes, 1u << 20), kStageBytes);
-            if ((e = hipHostMalloc((void **)&ctx->stage, want, hipHostMallocDefault)) != hipSuccess)
-                return hip_fail(ctx, e);
+            if (hipHostMalloc((void **)&ctx->stage, want, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
+                ctx->stage = nullptr;
+                return CTSM_OK;
+            }
             ctx->stage_size = want;
         }
     }
@@ -565,13 +579,16 @@ int stage_room(ctsm_ctx *ctx, size_t bytes, char **p)
 }
 
 // Copy [lo, hi] of every level of each non-null field between host arrays
-// (layout ld / beg) and dense device mirrors (layout hi-lo+1 / lo).  The mirrors of
-// a staged call lie in one buffer, bufs[nmeta], the writable fields in front.
+// (layout ld / beg) and dense device mirrors (layout hi-lo+1 / lo).  Where the
+// fields are at most kStageBytes and there is memory for it, their mirrors lie in one
+// buffer, the last of mir.bufs, the writable fields in front, and are copied at once
+// through the staging; else each field has a mirror and a copy of its own.
 int mirror(ctsm_ctx *ctx, const FieldMeta *meta, int nmeta, const void *host_struct, void *dev_struct,
-           std::vector<DevBuf> &bufs, int beg_alloc, int ld, Range r, bool to_device)
+           Mirrors &mir, int beg_alloc, int ld, Range r, bool to_device)
 {
     const int w = r.hi - r.lo + 1;
-    if (bufs.size() < (size_t)nmeta + 1) bufs.resize(nmeta + 1);
+    if (mir.bufs.size() < (size_t)nmeta + 1) mir.bufs.resize(nmeta + 1);
+    DevBuf &pack = mir.bufs[nmeta];
     const auto host = [&](int f) { return *(char *const *)((const char *)host_struct + meta[f].offset); };
     const auto row = [&](int f) { return (size_t)w * meta[f].elem; };
     const auto levels = [&](int f) { return nlev_of(meta[f].kind, ctx->cfg); };
@@ -585,23 +602,23 @@ int mirror(ctsm_ctx *ctx, const FieldMeta *meta, int nmeta, const void *host_str
         }
         if (pass == 0) written = total;
     }
-    const bool staged = total <= kStageBytes;
+    char *sp = nullptr;         // the staging, where the copy goes through it
     const size_t moved = to_device ? total : written;
-    char *sp = nullptr, *base = nullptr;
-    if (staged && moved) {
+    if (moved && (to_device ? total <= kStageBytes : mir.packed)) {
         int rc = stage_room(ctx, moved, &sp);
         if (rc) return rc;
-        if (to_device) {
-            hipError_t e = bufs[nmeta].ensure(total);
-            if (e != hipSuccess) return hip_fail(ctx, e);
+    }
+    if (to_device) {
+        if (sp && pack.ensure(total) != hipSuccess) {
+            (void)hipGetLastError();
+            sp = nullptr;
         }
-        base = (char *)bufs[nmeta].p;
-        if (!to_device) {
-            hipError_t e = hipMemcpyAsync(sp, base, moved, hipMemcpyDeviceToHost, ctx->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-            if (e != hipSuccess) return hip_fail(ctx, e);
-            ctx->stage_used = 0;
-        }
+        mir.packed = sp != nullptr;
+    } else if (sp) {
+        hipError_t e = hipMemcpyAsync(sp, pack.p, moved, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) return hip_fail(ctx, e);
+        ctx->stage_used = 0;
     }
     for (int f = 0; f < nmeta; ++f) {
         const FieldMeta &m = meta[f];
@@ -611,30 +628,28 @@ int mirror(ctsm_ctx *ctx, const FieldMeta *meta, int nmeta, const void *host_str
         if (!to_device && !m.writable) continue;
         const int nl = levels(f);
         char *hsrc = hp + (size_t)(r.lo - beg_alloc) * m.elem;
-        if (staged) {
+        hipError_t e;
+        if (to_device) {
+            if (!mir.packed && (e = mir.bufs[f].ensure(row(f) * nl)) != hipSuccess) return hip_fail(ctx, e);
+            *dslot = mir.packed ? (char *)pack.p + at[f] : (char *)mir.bufs[f].p;
+        }
+        if (sp) {
             for (int l = 0; l < nl; ++l) {
                 char *h = hsrc + (size_t)l * ld * m.elem, *t = sp + at[f] + l * row(f);
                 if (to_device) std::memcpy(t, h, row(f));
                 else std::memcpy(h, t, row(f));
             }
-            if (to_device) *dslot = base + at[f];
             continue;
         }
-        if (to_device) {
-            hipError_t e = bufs[f].ensure(row(f) * nl);
-            if (e != hipSuccess) return hip_fail(ctx, e);
-            *dslot = (char *)bufs[f].p;
-        }
-        char *dp = (char *)bufs[f].p;
-        hipError_t e;
+        char *dp = mir.packed ? (char *)pack.p + at[f] : (char *)mir.bufs[f].p;
         if (to_device)
             e = hipMemcpy2DAsync(dp, row(f), hsrc, (size_t)ld * m.elem, row(f), nl, hipMemcpyHostToDevice, ctx->stream);
         else
             e = hipMemcpy2DAsync(hsrc, (size_t)ld * m.elem, dp, row(f), row(f), nl, hipMemcpyDeviceToHost, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, e);
     }
-    if (staged && to_device && moved) {
-        hipError_t e = hipMemcpyAsync(base, sp, moved, hipMemcpyHostToDevice, ctx->stream);
+    if (sp && to_device) {
+        hipError_t e = hipMemcpyAsync(pack.p, sp, moved, hipMemcpyHostToDevice, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, e);
     }
     return CTSM_OK;

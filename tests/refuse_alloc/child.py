@@ -9,8 +9,9 @@ import numpy as np  # noqa: E402
 from ctsm_amd import synthetic as S  # noqa: E402
 from ctsm_amd.lib import Context  # noqa: E402
 from ctsm_amd.state import DeviceState  # noqa: E402
+from oracle import oracle as O  # noqa: E402
 
-shim.refuse_device.argtypes = [C.c_size_t, C.c_size_t]
+shim.refuse_device.argtypes = shim.refuse_pinned.argtypes = [C.c_size_t, C.c_size_t]
 
 
 def same(a, b):
@@ -57,7 +58,35 @@ def one_pass(plain, graph):
     same(results[1], results[0])
 
 
+def host_arrays(what):
+    """SoilWater on host arrays: no pinned memory at all, none on a call that needs more
+    than the one before it, or no device memory for the fields in one piece; every call
+    right, and the copies in one piece again once there is memory."""
+    ctx = Context()
+    print(f"case: SoilWater on host arrays, no memory: {what}", flush=True)
+    for ncol, full in ((300, what != "pinned later"), (2000, True), (700, False)):
+        if full:
+            size = 2000 * ncol      # less than the fields take in one piece, more than one takes
+            if what == "device":
+                shim.refuse_device(size, 1 << 40)
+            else:
+                shim.refuse_pinned(0, 1 << 40)
+        st = S.workload("uneven", ncol=ncol)
+        g = st.copy()
+        ctx.soilwater(g)
+        shim.refuse_device(0, 0)
+        shim.refuse_pinned(0, 0)
+        assert (shim.refusals() > 0) == full, ncol
+        assert O.soilwater(st)[0] == 0
+        for k, v in st.col.items():
+            np.testing.assert_array_equal(g.col[k], v, err_msg=f"{ncol} columns: {k}")
+    ctx.close()
+
+
 CASES = {
+    "host_arrays_pinned": lambda: host_arrays("pinned"),
+    "host_arrays_pinned_later": lambda: host_arrays("pinned later"),
+    "host_arrays_device": lambda: host_arrays("device"),
     "one_pass": lambda: one_pass(False, False),
     "one_pass_plain": lambda: one_pass(True, False),
     "one_pass_graph": lambda: one_pass(False, True),

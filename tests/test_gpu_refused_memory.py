@@ -1,6 +1,6 @@
 """Calls on a device that has less memory than they ask for.  Each case runs in a
-process of its own in front of whose library an allocation function stands that
-answers out-of-memory for a range of sizes (refuse_alloc/refuse.c).
+process of its own in front of whose library allocation functions stand that
+answer out-of-memory for a range of sizes (refuse_alloc/refuse.c).
 
 Each test prints its case before the GPU work starts.
 """
@@ -24,7 +24,8 @@ def shim(tmp_path_factory):
     return so
 
 
-@pytest.mark.parametrize("case", ["one_pass", "one_pass_plain", "one_pass_graph"])
+@pytest.mark.parametrize("case", ["one_pass", "one_pass_plain", "one_pass_graph", "host_arrays_pinned",
+                                  "host_arrays_pinned_later", "host_arrays_device"])
 def test_refused_memory(shim, case):
     print(f"case: {case}", flush=True)
     env = dict(os.environ, PYTHONPATH=ROOT)
