@@ -99,9 +99,12 @@ __device__ __forceinline__ void wave_sync()
 // product, its remainder, one correction): the instructions of the compiler's own
 // division without the scaling that only operands near the ends of the exponent
 // range need, so the quotient is the correctly rounded one, for 4 instructions
-// instead of 11.  For denominators and quotients of magnitudes between 2^-900 and
-// 2^900 (zero, infinite and NaN operands are settled by v_div_fixup as in a
-// division).
+// instead of 11.  For denominators from 2^-1020 to 2^1020, numerators of at least
+// 2^-960 (below that the remainder is not exact) and quotients from 2^-1020 to 2^1020;
+// zero, infinite and NaN operands are settled by v_div_fixup as in a division.
+// The Richards solve holds its operands to that (richards_group.h).  In CanopyFluxes
+// the denominators are heights, pressures, curvatures and conductances, and a
+// numerator below 2^-960 would be a photosynthesis rate of 1e-280.
 struct Recip {
     double b, y;
 };
@@ -117,6 +120,14 @@ __device__ __forceinline__ double operator/(double a, const Recip &r)
     const double q = a * r.y;
     return __builtin_amdgcn_div_fixup(fma(fma(-r.b, q, a), r.y, q), r.b, a);
 }
+// The same interface with a division, for operands of any range.
+struct Plain {
+    double b;
+};
+__device__ __forceinline__ double operator/(double a, const Plain &r) { return a / r.b; }
+template <class D> __device__ __forceinline__ D divisor(double b);
+template <> __device__ __forceinline__ Recip divisor<Recip>(double b) { return recip(b); }
+template <> __device__ __forceinline__ Plain divisor<Plain>(double b) { return Plain{b}; }
 
 // log's table in the LDS of a one-wave block (ctsm_math.h)
 #define LOG_TABLE(name)                                                                                            \

@@ -27,6 +27,8 @@
 // layers each), so one kernel can give each wavefront the group size its
 // columns' depth needs.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 #include "watertable_bc.h"
 
@@ -60,25 +62,59 @@ __device__ __forceinline__ double group_max(double v, int GS)
     return v;
 }
 
+// whether v is 2^lo .. 2^hi
+__device__ __forceinline__ bool within(double v, int lo, int hi)
+{
+    return (unsigned)__double2hiint(v) - ((unsigned)(1023 + lo) << 20) < ((unsigned)(hi - lo) << 20);
+}
+// whether `here` holds on any lane of the group
+__device__ __forceinline__ bool any_of_group(bool here, int GS)
+{
+    const unsigned long long m = __ballot(here);
+    return m && ((m >> (__lane_id() & ~(GS - 1))) & ((1ull << GS) - 1)) != 0;
+}
+
+// The solve with reciprocals (D = Recip) gives up, with the column as it was, where an
+// operand of its divisions might leave the range they are exact in; the solve with
+// divisions (D = Plain) takes any.  Ranges of the layers' constants that hold every
+// operand but the substitution's to it, with s in 0.01 .. 1:
+//   hk   0 or 2^-419 .. 2^20     (hkc s^(2b+3))
+//   dsm  2^-9 .. 2^212           (b suc s^-b / (s ws))
+//   the flux derivatives' numerators 0 or 2^-529 .. 2^232, a row's entries dl 0 or from
+//   2^-682, its diagonal up to 2^290, so dl / d 0 or from 2^-972.
+// Real soils are far inside; a NaN is outside.
+constexpr int RICHARDS_RANGE = 6;
+__device__ __forceinline__ bool ordinary_layer(double dz, double den, double ws, double bsw, double suc, double hkc)
+{
+    return within(dz, -10, 20) && within(den, -10, 20) && within(ws, -10, 1) && within(bsw, -4, 5) && bsw <= 24.0 &&
+           within(suc, -4, 30) && (within(hkc, -80, 20) || hkc == 0.0);
+}
+__device__ __forceinline__ bool ordinary_steps(const Params &P, double dtime)
+{
+    return within(dtime, -20, 30) && P.dtmin >= 0x1.0p-20 && P.verySmall >= 0x1.0p-60;
+}
+
 // WT: the water-table bottom boundary (watertable_bc.h), a separate
 // instantiation so the flux / zero-flux kernels keep their registers.
 // lt: log's table in LDS.
-template <int G, bool WT = false, int K = (MAX_NLEVSOI + (G > 0 ? G : 1) - 1) / (G > 0 ? G : 1)>
-__device__ __forceinline__ int richards_group(const View &V, const Params &P, const ctsm_col_state &S, int c,
-                                              double dtime, int g, const double *lt, int gsz = G)
+template <class D, int G, bool WT, int K>
+__device__ __forceinline__ int richards_group_by(const View &V, const Params &P, const ctsm_col_state &S, int c,
+                                                 double dtime, int g, const double *lt, int gsz)
 {
+    constexpr bool RANGED = std::is_same<D, Recip>::value;
     const int GS = (G > 0) ? G : gsz;       // lanes in the group
     const int nl = S.nbedrock[V.c1(c)];
     if (nl < 2 || nl > MAX_NLEVSOI || nl > GS * K) return 1;
 
     // the layers of the lane; a layer below the column's last holds ordinary values,
     // which run through the trials without effect
-    Recip mdz[K], ws[K], den[K];
+    D mdz[K], ws[K], den[K];
     double bsw[K], hkc[K], suc[K], sink[K], liq[K];
     double Ud[K], Udu[K], Udl[K], Ub[K], f1[K];
     const double infl = S.qflx_infl[V.c1(c)];
     // watsat of the first layer of the next lane (for the interface below our last layer)
-    Recip ws_nl = recip(1.0);
+    D ws_nl = divisor<D>(1.0);
+    bool outside = RANGED && !ordinary_steps(P, dtime);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int j = g * K + k;            // 0-based layer
@@ -104,14 +140,16 @@ __device__ __forceinline__ int richards_group(const View &V, const Params &P, co
             }
             hkc[k] = cm_pow_tab(10.0, -(P.e_ice * icei), lt) * S.hksat[V.soi(c, jj)];
         }
-        mdz[k] = recip(dzk);
-        ws[k] = recip(wsk);
-        den[k] = recip(denk);
+        if (RANGED && !ordinary_layer(dzk, denk, wsk, bsw[k], suc[k], hkc[k])) outside = true;
+        mdz[k] = divisor<D>(dzk);
+        ws[k] = divisor<D>(wsk);
+        den[k] = divisor<D>(denk);
     }
     {
         const int jn = (g + 1) * K;
-        if (jn < nl) ws_nl = recip(S.watsat[V.soi(c, jn + 1)]);
+        if (jn < nl) ws_nl = divisor<D>(S.watsat[V.soi(c, jn + 1)]);
     }
+    if (RANGED && any_of_group(outside, GS)) return RICHARDS_RANGE;
 
     const bool zero_flux_bottom = (P.lower_bc == CTSM_BC_ZERO_FLUX);
     constexpr bool wt_bottom = WT;
@@ -156,7 +194,7 @@ __device__ __forceinline__ int richards_group(const View &V, const Params &P, co
             const double s2n = k + 1 < K ? s2[k + 1 < K ? k + 1 : k] : s2_nx;
             const double smpn = k + 1 < K ? smp[k + 1 < K ? k + 1 : k] : smp_nx;
             const double dsmn = k + 1 < K ? dsm[k + 1 < K ? k + 1 : k] : dsm_nx;
-            const Recip wsn = k + 1 < K ? ws[k + 1 < K ? k + 1 : k] : ws_nl;
+            const D wsn = k + 1 < K ? ws[k + 1 < K ? k + 1 : k] : ws_nl;
             double s1 = bottom ? s2[k] : 0.5 * (s2[k] + s2n);
             s1 = fmin90(s1, 1.0);
             s1 = fmax90(0.01, s1);
@@ -241,7 +279,7 @@ __device__ __forceinline__ int richards_group(const View &V, const Params &P, co
                     const double nd = k + 1 < K ? Ud[k + 1 < K ? k + 1 : k] : b_nx;
                     const double ndu = k + 1 < K ? Udu[k + 1 < K ? k + 1 : k] : c_nx;
                     const double nb = k + 1 < K ? Ub[k + 1 < K ? k + 1 : k] : r_nx;
-                    const double fact = dl / recip(cd);
+                    const double fact = dl / divisor<D>(cd);
                     Ud[k] = cd; Udu[k] = cdu; Udl[k] = 0.0; Ub[k] = cb;
                     double td = nd - fact * cdu, tdu = ndu, tb = nb - fact * cb;
                     if (!(fabs(cd) > fabs(dl))) {
@@ -265,22 +303,19 @@ __device__ __forceinline__ int richards_group(const View &V, const Params &P, co
                 cb = from_prev(cb);
             }
         }
-        // any lane singular -> the whole column fails
-        const unsigned long long sing = __ballot(singular);
-        if (sing && ((sing >> (__lane_id() & ~(GS - 1))) & ((1ull << GS) - 1)) != 0) { status = 2; break; }
 
         // ---- back substitution in reverse stages (the reciprocals of the diagonal
         //      beforehand, outside the chain), then the error estimate
-        double yd[K];
+        D d[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k) yd[k] = recip(Ud[k]).y;
+        for (int k = 0; k < K; ++k) d[k] = divisor<D>(Ud[k]);
         double x1 = 0.0, x2 = 0.0;
 #pragma unroll
         for (int s = GS - 1; s >= 0; --s) {
             if (g == s) {
 #pragma unroll
                 for (int k = K - 1; k >= 0; --k) {
-                    const double x = (Ub[k] - Udu[k] * x1 - Udl[k] * x2) / Recip{Ud[k], yd[k]};
+                    const double x = (Ub[k] - Udu[k] * x1 - Udl[k] * x2) / d[k];
                     Ub[k] = x;
                     x2 = x1;
                     x1 = x;
@@ -290,6 +325,17 @@ __device__ __forceinline__ int richards_group(const View &V, const Params &P, co
                 x1 = from_next(x1);
                 x2 = from_next(x2);
             }
+        }
+        if (RANGED) {
+            // the numerators of the substitution, and what the water content can become
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (!(fabs(Ub[k] * Ud[k]) >= 0x1.0p-900 && fabs(Ub[k]) < 0x1.0p+200) && Ub[k] != 0.0) outside = true;
+        }
+        // any lane singular -> the whole column fails
+        if (any_of_group(singular || outside, GS)) {
+            if (!RANGED || any_of_group(singular, GS)) { status = 2; break; }
+            return RICHARDS_RANGE;
         }
         double emax = 0.0, dwat_bot = 0.0;
         bool have_e = false;
@@ -354,6 +400,15 @@ __device__ __forceinline__ int richards_group(const View &V, const Params &P, co
     for (int k = 0; k < K; ++k)
         if (g * K + k < nl) S.h2osoi_liq[V.sno(c, g * K + k + 1)] = liq[k];
     return 0;
+}
+
+template <int G, bool WT = false, int K = (MAX_NLEVSOI + (G > 0 ? G : 1) - 1) / (G > 0 ? G : 1)>
+__device__ __forceinline__ int richards_group(const View &V, const Params &P, const ctsm_col_state &S, int c,
+                                              double dtime, int g, const double *lt, int gsz = G)
+{
+    int rc = richards_group_by<Recip, G, WT, K>(V, P, S, c, dtime, g, lt, gsz);
+    if (rc == RICHARDS_RANGE) rc = richards_group_by<Plain, G, WT, K>(V, P, S, c, dtime, g, lt, gsz);
+    return rc;
 }
 
 }  // namespace ctsm
