@@ -275,6 +275,13 @@ __device__ __forceinline__ int richards_group_by(const View &V, const Params &P,
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const int j = g * K + k;
+                    if (!RANGED && j >= nl - 1) {
+                        // a NaN or an infinity would pass from the last row to those below
+                        if (j > nl - 1) continue;
+                        Ud[k] = cd; Udu[k] = 0.0; Udl[k] = 0.0; Ub[k] = cb;
+                        if (cd == 0.0) singular = true;
+                        continue;
+                    }
                     const double dl = k + 1 < K ? Udl[k + 1 < K ? k + 1 : k] : a_nx;
                     const double nd = k + 1 < K ? Ud[k + 1 < K ? k + 1 : k] : b_nx;
                     const double ndu = k + 1 < K ? Udu[k + 1 < K ? k + 1 : k] : c_nx;
@@ -315,7 +322,14 @@ __device__ __forceinline__ int richards_group_by(const View &V, const Params &P,
             if (g == s) {
 #pragma unroll
                 for (int k = K - 1; k >= 0; --k) {
-                    const double x = (Ub[k] - Udu[k] * x1 - Udl[k] * x2) / d[k];
+                    double r = Ub[k] - Udu[k] * x1 - Udl[k] * x2;
+                    if (!RANGED) {
+                        // and from the rows below the last to it
+                        const int j = g * K + k;
+                        if (j == nl - 1) r = Ub[k];
+                        if (j == nl - 2) r = Ub[k] - Udu[k] * x1;
+                    }
+                    const double x = r / d[k];
                     Ub[k] = x;
                     x2 = x1;
                     x1 = x;
@@ -338,17 +352,21 @@ __device__ __forceinline__ int richards_group_by(const View &V, const Params &P,
             return RICHARDS_RANGE;
         }
         double emax = 0.0, dwat_bot = 0.0;
-        bool have_e = false;
+        bool top_nan = false;
 #pragma unroll
         for (int k = K - 1; k >= 0; --k) {
             const int j = g * K + k;
             const double x = Ub[k], dtdz = dtsub / mdz[k];
             const double ev = fabs(f1[k] - x / dtdz) * dtsub * 0.5;
             if (j == nl - 1) dwat_bot = x;
-            if (j < nl && (!have_e || ev > emax)) { emax = ev; have_e = true; }
+            if (j < nl && ev > emax) emax = ev;
+            if (j == 0) top_nan = ev != ev;
         }
-        // group max of the error estimate (each owned layer's value; empty lanes hold 0 <= any)
-        const double errorMax = group_max(emax, GS);
+        // group max of the error estimate (each owned layer's value; empty lanes hold 0 <=
+        // any).  As in the reference's maxval from the first layer on, a NaN there stays
+        // and one below it does not count; the solve with reciprocals meets none.
+        double errorMax = group_max(emax, GS);
+        if (!RANGED && any_of_group(top_nan, GS)) errorMax = NAN;
         if (errorMax > P.xTolerUpper && dtsub > P.dtmin) {
             dtsub = fmax90(dtsub / 2.0, P.dtmin);
             continue;

@@ -81,3 +81,26 @@ def test_beyond_the_range_bitwise(ctx, change, lanes):
     change(st)
     print(f"case: SoilWater, {change.__name__}, {lanes} lanes", flush=True)
     check(ctx, st, lanes)
+
+
+def nan_at_the_bottom(st):
+    """A retention exponent that is NaN in the last layer of every fourth column, beside
+    columns beyond the range."""
+    nb = st.col["nbedrock"]
+    nb[::2] = 20
+    st.col["bsw"][:, 1::2] = 30.0
+    st.col["bsw"][nb[::4] - 1, np.arange(0, NCOL, 4)] = np.nan
+
+
+def flood(st):
+    """Infinite infiltration into every third column."""
+    st.col["qflx_infl"][::3] = np.inf
+
+
+@pytest.mark.parametrize("lanes", [0, 4, 8])
+@pytest.mark.parametrize("change", [nan_at_the_bottom, flood])
+def test_nan_and_infinity_bitwise(ctx, change, lanes):
+    st = S.workload("uneven", ncol=NCOL)
+    change(st)
+    print(f"case: SoilWater, {change.__name__}, {lanes} lanes", flush=True)
+    check(ctx, st, lanes)
