@@ -58,10 +58,10 @@ k_soilwater_fractions(View V, ctsm_col_state S, int n, const int32_t *__restrict
 
 // G lanes per column (richards_group.h).  Groups are aligned to G lanes, so a
 // column's lanes retire together.  For G = 8 the register budget is capped at 168
-// VGPRs for three waves per SIMD (192 B/lane of scratch): 262,144 uneven columns
-// 3.61 ms, 4.09 at two waves and 4.77 at four.  G = 4 needs 374 registers: 4.24 ms
-// at one wave per SIMD, 4.52 at two, 5.89 at three.
-template <int G> struct RichardsWaves { static constexpr int value = 1; };
+// VGPRs for three waves per SIMD (176 B/lane of scratch): 262,144 uneven columns
+// 3.42 ms, 3.85 at two waves and 4.22 at four.  G = 4: 3.82 ms at two waves, 3.96 at
+// one and 5.43 at three.
+template <int G> struct RichardsWaves { static constexpr int value = 2; };
 template <> struct RichardsWaves<8> { static constexpr int value = 3; };
 
 template <int G, bool WT>
@@ -86,11 +86,10 @@ k_soilwater_g(View V, Params P, ctsm_col_state S, int n, const int32_t *__restri
 // passes of 64 / lanes.  A batch stored by depth gives most blocks the
 // smallest group its columns allow, so no lane holds only empty layers; the
 // results do not depend on the group size.  Built for three waves per SIMD
-// (168 VGPRs): at four (128 VGPRs, 120 spilled) the solve of 1,048,576
-// uneven columns took 8.3 ms, at three 7.4, at two 8.1.
+// (168 VGPRs): 262,144 uneven columns 3.34 ms, 3.50 at two and 4.14 at four.
 // A deep block runs its 32 columns in four passes of 8, so that 20,000 columns in
-// their own order take 3.53 ms a land step against the 8-lane kernel's 2.80; on
-// 262,144 ordered ones 3.26 and 3.39 ms.
+// their own order take 3.58 ms a land step against the 8-lane kernel's 2.80; on
+// the 262,144 ordered ones 3.34 and 3.42 ms.
 constexpr int ADAPT_SPAN = 32;
 constexpr int ADAPT_K = 3;
 template <bool WT>
@@ -152,7 +151,7 @@ void launch_soilwater_k(hipStream_t st, const View &V, const Params &P, const ct
     }
     if (lanes == 2 || lanes == 4 || lanes == 8) {
         // two lanes run as four: 262,144 columns 6.12 ms at two lanes of 10 layers, which
-        // spill, 3.83 at four and 3.39 at eight
+        // spill, 3.82 at four and 3.42 at eight
         if (block <= 0 || block > 256) block = 128;
         const int G = lanes == 8 ? 8 : 4;
         const dim3 grid((unsigned)(((long)n * G + block - 1) / block));
