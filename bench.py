@@ -13,7 +13,7 @@ HBM, generated in binned column order, for 48 steps (one day); the soil
 launch shape and the CanopyFluxes round split are chosen by the autotuner;
 the 48 timed steps are captured once as one HIP graph and launched once.
 The same 48 steps are also run in the plain form (one launch per reference
-routine, CanopyFluxes iterating every patch to convergence in one launch).
+routine, CanopyFluxes iterating every patch to convergence in one round).
 
 Prints ONE JSON line with the metric, the roofline of the dominant kernel
 (algorithmic bytes per CanopyFluxes call / its measured time vs 8 TB/s) and
@@ -39,10 +39,32 @@ HBM_PEAK_GBS = 8000.0
 # dispatch, scaled by the same counters' readings on a streaming copy of
 # known size) and FP64 VALU share (SQ_INSTS_VALU_*_F64 over the launch time
 # against the 78.6 TFLOP/s vector peak) of a dominant kernel, keyed by
-# (kernel, workload, columns), with the launch shape they were measured at.
+# (routine, workload, columns), with the launch shape they were measured at.
 # The bench reports them only for a run of that workload, size and launch
 # shape; any other run reports null.
-PROFILED = {}       # none for the kernels as they are
+# profiles/counters_canopy_uneven1048576.md: one call of each routine after the steps,
+# FETCH x 2.0 + WRITE x 1.0 KiB (CanopyFluxes: its set-up, rounds and finish together).
+PROFILED = {
+    ("canopy", "canopy_uneven", 1048576): {
+        "traffic": (23472322 * 2.0 + 31329663 * 1.0) * 1024,
+        "fp64_valu_frac": 411.7e9 / 32.1e-3 / 78.6e12,
+        "tuning": {"canopy_first_iterations": 6, "canopy_round_iterations": 3, "canopy_waves": 2},
+    },
+    ("richards", "canopy_uneven", 1048576): {
+        "traffic": (3820157 * 2.0 + 3513411 * 1.0) * 1024,
+        "tuning": {"richards_lanes": 8},          # measured in 128-lane blocks; the block size moves no bytes
+    },
+    ("soiltemp", "canopy_uneven", 1048576): {
+        "traffic": (4802646 * 2.0 + 4223756 * 1.0) * 1024,
+        "tuning": {},
+    },
+}
+
+
+def profiled(routine, args, ncol, tuning):
+    """PROFILED's entry for this run, or None."""
+    p = PROFILED.get((routine, args.workload, ncol))
+    return None if p is None or any(tuning.get(k) != v for k, v in p["tuning"].items()) else p
 
 
 def richards_bytes(st):
@@ -561,10 +583,7 @@ def main():
                                   "frac": step_bytes / (ms_step * 1e-3) / 1e9 / HBM_PEAK_GBS}
     for nm in ("soiltemp", "richards"):
         ms = res["kernel_ms"][nm]
-        kn = "k_soiltemp" if nm == "soiltemp" else "k_soilwater_g"
-        p = PROFILED.get((kn, args.workload, ncol))
-        if p and any(res["tuning"].get(k) != v for k, v in p["tuning"].items()):
-            p = None
+        p = profiled(nm, args, ncol, res["tuning"])
         res.setdefault("roofline_other", {})[nm] = {
             "kernel": "k_soiltemp" if nm == "soiltemp" else "k_soilwater_g (with its sub-step column order)",
             "ms": ms, "alg_bytes_per_launch": bytes_by[nm], "achieved_GBps": bytes_by[nm] / (ms * 1e-3) / 1e9,
@@ -590,10 +609,7 @@ def main():
     if args.serve_requests > 0:
         res["served_ensemble"] = served_ensemble(ctx, args)
         print("[bench] served ensemble done", file=sys.stderr, flush=True)
-    kname = "k_canopy_round"
-    prof = PROFILED.get((kname, args.workload, ncol))
-    if prof and any(res["tuning"].get(k) != v for k, v in prof["tuning"].items()):
-        prof = None
+    prof = profiled("canopy", args, ncol, res["tuning"])
     lanes = res["tuning"]["richards_lanes"]
     out = {
         "metric": "column-steps/sec (FP64, 1 GPU)",
@@ -620,7 +636,8 @@ def main():
                    "richards_lanes": lanes},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": prof["traffic"] if prof else None,
-                     "kernel": kname + " (all rounds of one CanopyFluxes call)", "launch_ms": kms,
+                     "kernel": "k_canopy_setup, k_canopy_round (all rounds), k_canopy_finish: one CanopyFluxes call",
+                     "launch_ms": kms,
                      "alg_bytes_per_launch": kb,
                      "fp64_valu_frac": prof["fp64_valu_frac"] if prof else None},
         "detail": res,

@@ -812,9 +812,11 @@ static_assert(sizeof(CanopyWork) == N_WORK_FIELDS * sizeof(double *), "one point
 // iteration now keeps its state only; what the outputs need of its last pass is
 // written by the passes that can be the last one (the leaf temperature had settled
 // in the pass before, or itmax is reached), each later one over the earlier.
-// All three are bound by the issue of FP64 and scalar instructions and by the waits
-// of one or two waves per SIMD; HBM is at a sixth of its rate.  On 1,048,576 columns
-// (8.9 million patches) the one kernel took 31.4 ms for its first round and 43.6 ms
+// What bounds them, by counters on 1,048,576 columns (8.9 million patches): the set-up
+// moves 19.6 GB in 4.2 ms, as fast as a copy; the first round issues vector
+// instructions in 63 % of the SIMDs' cycles (and moves 28.7 GB in 17.1 ms); the later
+// rounds, in 35 %, wait for their slow patches; the finish moves 6.7 GB in 2.0 ms,
+// three quarters of a copy's rate.  There the one kernel took 31.4 ms for its first round and 43.6 ms
 // in all; the set-up takes 4.1, the rounds 26.6 (the first 17.0) and the finish
 // 2.0 ms now.  (With the finish reading the outputs back, 0.3 ms less; the totals
 // would then depend on the caller's arrays being distinct.)
@@ -1878,7 +1880,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
 // opaque on every pass, so its loads stay inside the pass instead of being
 // hoisted in front of the loop.
 // WAVES: the register budget the kernel is compiled for (waves per SIMD).  One wave
-// needs 310 registers; the two-wave instance (256, and 176 B/lane of scratch) pays
+// needs 296 registers; the two-wave instance (256, and 176 B/lane of scratch) pays
 // once a filter has a second wave for the SIMDs: launch_canopy has the rule.
 // PHS: CanopyFluxes with plant hydraulic stress (argument RoundArgsPhs).
 template <int WAVES, bool STRIDE, bool PHS = false>
@@ -2170,7 +2172,9 @@ void launch_canopy(hipStream_t st, const ctsm_layout &L, const ctsm_config &cfg,
                     0, 0, nullptr, nullptr, nullptr, nullptr, CanopyWork{}};
         // The two-wave instance from the first block that has no SIMD to itself.  65,536
         // columns (8,704 waves): 3380 us with one wave per SIMD, 3150 us with two; 762
-        // waves: 1469 and 1566 us.  About a quarter of the patches goes on to round 1.
+        // waves: 1469 and 1566 us.  The later rounds, with the rest as it is, one wave and
+        // two: 20,000 columns (2,656 blocks) 1688 and 1796 us, 40,000 (5,313) 2273 and
+        // 2316, 65,536 (8,704) 2989 and 3048, 262,144 (34,816) 8903 and 8692.
         const bool two = waves > 1 && blocks > SIMDS, two_later = waves > 1 && blocks > 4 * SIMDS;
         auto first_kernel = two ? k_canopy_round<2, false> : k_canopy_round<1, false>;
         auto later_kernel = two_later ? k_canopy_round<2, true> : k_canopy_round<1, true>;

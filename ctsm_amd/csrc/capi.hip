@@ -545,10 +545,10 @@ Range filter_range(int n, const int32_t *f, int def_lo)
 
 // The drop-in copies go through pinned staging where the fields of a mirror call are
 // at most this much: packed by the host and copied at once.  A pageable copy per field
-// costs some 100 us whatever its size, packing about 0.2 ns a byte, so the gain ends
-// where a field's rows are long; the bound is on the memory a context keeps.  The three
-// soil routines on host arrays, per field and staged: 64 columns 32.3 and 1.1 ms, 1,024
-// 35.5 and 2.2, 16,384 (99 MB a call) 50.6 and 27.5, 32,768 66.7 and 53.4 ms.
+// costs some 100 us whatever its size, packing about 0.2 ns a byte.  The bound is on the
+// pinned memory a context keeps, not where the gain ends.  The three soil routines on
+// host arrays, per field and staged: 64 columns 32.3 and 1.1 ms, 1,024 35.5 and 2.2,
+// 16,384 (99 MB a call) 50.6 and 27.5, 32,768 (with twice the bound) 66.7 and 53.4 ms.
 constexpr size_t kStageBytes = 128u << 20;
 
 // `bytes` of staging that no copy in flight uses; null where there is no pinned memory

@@ -421,8 +421,6 @@ CM_FN double cm_pow_special(double x, double y, const double *tab)
     return odd ? -res : res;
 }
 
-/* x**y; the physics takes it of x > 0 only.  x**0 = 1 and x**1 = x exactly, as
- * a C pow gives them (the first of itself: exp(0)). */
 /* x^y for x > 0 (finite), whose log is lh + ll (cm_log_dd), and finite y */
 CM_FN double cm_pow_log(double x, double lh, double ll, double y)
 {
@@ -432,6 +430,8 @@ CM_FN double cm_pow_log(double x, double lh, double ll, double y)
     return y == 1.0 ? x : res;
 }
 
+/* x**y; the physics takes it of x > 0 only.  x**0 = 1 and x**1 = x exactly, as
+ * a C pow gives them (the first of itself: exp(0)). */
 CM_FN double cm_pow_tab(double x, double y, const double *tab)
 {
     if (__builtin_expect(!(x > 0.0 && x < HUGE_VAL) || !(fabs(y) < HUGE_VAL), 0)) return cm_pow_special(x, y, tab);

@@ -111,12 +111,12 @@ __global__ void __launch_bounds__(256) k_phs_root_sink(PView V, ctsm_phs_state S
     S.qflx_phs_neg[cc] = neg;
 }
 
-// Bound by FP64 issue: up to 50 Newton passes of 8 powers, ~20 divides and the
-// root's 20-layer sum.  A patch per lane, its soil in LDS (stage_soil, 20 KB a
-// wave: two waves per SIMD, 219 VGPRs, no scratch).  262,144 patches: 2.24 ms when
-// every pass read its layers from HBM and took 28 powers, 0.65 ms so and 0.60 with log's
-// table in LDS (0.69 ms with
-// the scheduler told of the two waves instead of asked for three).
+// Bound by the chain of up to 50 Newton passes, each of 8 powers, ~20 divides and the
+// root's 20-layer sum: vector instructions take 43 % of the SIMDs' cycles, with one wave
+// a SIMD on the average because a block's slowest patch keeps its place.  A patch per
+// lane, its soil and log's table in LDS (stage_soil; 22.7 KB a wave, seven waves a CU;
+// 220 VGPRs, no scratch).  262,144 patches: 2.24 ms when every pass read its layers
+// from HBM and took 28 powers, 0.60 ms so (0.65 with log's table in global memory).
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8)))
 k_phs_calcstress(PView V, ctsm_phs_stress_state S, const double *__restrict__ T, int npft, int n,
                  const int32_t *__restrict__ filter, ErrWord *err)

@@ -15,13 +15,13 @@
 //     group takes the same accept / halve / double decision.
 // A lane keeps ~K*13 doubles instead of 20*13, and several waves share a SIMD.
 // Values are bit-identical to the one-lane form.
-// Bound by FP64 issue: vector instructions take 72 % of the SIMDs' cycles (1,048,576
-// columns, three waves per SIMD), the HBM traffic, two thirds of it spilled registers
-// and the trials' diagnostics, 3.0 TB/s.  The serial stages run with one lane of a group, so what can leave them has: the error
-// estimate's two divisions a row, the diagonal's reciprocals, the row interchange's
-// selects (a branch that few rows take).  The properties are straight-line over the
-// lane's layers, divisors used several times are inverted once, log's table is in
-// LDS.  262,144 uneven columns: 5.31 ms before, 3.42 ms so with 8 lanes; 7.12 and
+// Bound by FP64 issue: vector instructions take 63 % of the SIMDs' cycles (1,048,576
+// columns, three waves per SIMD); the HBM traffic, seven times the columns' own through
+// spilled registers and the trials' diagnostics, runs at 3.0 TB/s.  The serial stages
+// run with one lane of a group, so what can leave them has: the error estimate's two
+// divisions a row, the diagonal's reciprocals, the row interchange's selects (a branch
+// that few rows take).  The properties are straight-line over the lane's layers,
+// divisors used several times are inverted once, log's table is in LDS.  262,144 uneven columns: 5.31 ms before, 3.42 ms so with 8 lanes; 7.12 and
 // 3.82 ms with 4.
 // G = 0 takes the group size at run time (argument gsz: 2, 4 or 8 lanes of K
 // layers each), so one kernel can give each wavefront the group size its

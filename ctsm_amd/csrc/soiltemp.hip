@@ -784,10 +784,12 @@ k_soiltemp(SoilTempArgs)
 // lanes per column).
 // BLOCK: 64 or 128 threads (the LDS of the ground heat flux is per wave).
 // Built for three waves per SIMD (168 VGPRs, 32 B/lane of scratch; the LDS of the
-// ground heat flux leaves room for eleven waves a CU).  Bound by FP64 issue and the
-// waits of its loads, whose addresses hang on the level.  With the arrays' addresses
-// held in scalar registers 1,216 of the kernel's 5,300 instructions moved spilled ones
-// to vector lanes and back; read in place 20 do.  With log's table in LDS too, 262,144
+// ground heat flux leaves room for eleven waves a CU).  Bound by HBM: k_soiltemp moves
+// 14.2 GB for 1,048,576 columns in 3.58 ms, 91 % of what a large copy reaches and twice
+// the arrays' own bytes (the elimination's rows are stored and read back); vector
+// instructions take 25 % of the SIMDs' cycles.  With the arrays' addresses held in
+// scalar registers 1,216 of the kernel's 5,300 instructions moved spilled ones to
+// vector lanes and back; read in place 20 do.  With log's table in LDS too, 262,144
 // columns 975 and 916 us, the step of 1,048,576 columns 42.7 and 41.5 ms.
 template <int BLOCK>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3)))

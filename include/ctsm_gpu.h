@@ -616,9 +616,10 @@ typedef struct ctsm_phs_canopy_state {
  * plain_routines: 1 = the land steps (ctsm_land_step_full_dev and its
  *   captures) run the plain form: SoilTemperature and SoilWater as one launch
  *   per reference routine with intermediates through HBM (the plain kernels of
- *   the *_dev entries' `plain` argument), CanopyFluxes as one launch that
- *   iterates every patch to convergence (no compacted rounds).  The comparison
- *   baseline of the batched step; results are the same.
+ *   the *_dev entries' `plain` argument), CanopyFluxes with one iteration launch
+ *   that takes every patch to convergence (no compacted rounds) between its
+ *   set-up and its outputs.  The comparison baseline of the batched step; results
+ *   are the same.
  * canopy_waves: the waves per SIMD the CanopyFluxes iteration is built for, at
  *   most: 1, or 2 and 3 for the two-wave kernel on filters that have a second
  *   wave for the SIMDs (more than 65,536 patches).  Results do not depend on
