@@ -21,8 +21,8 @@
 // run with one lane of a group, so what can leave them has: the error estimate's two
 // divisions a row, the diagonal's reciprocals, the row interchange's selects (a branch
 // that few rows take).  The properties are straight-line over the lane's layers,
-// divisors used several times are inverted once, log's table is in LDS.  262,144 uneven columns: 5.31 ms before, 3.42 ms so with 8 lanes; 7.12 and
-// 3.82 ms with 4.
+// divisors used several times are inverted once, log's table is in LDS.  262,144
+// uneven columns: 5.31 ms before, 3.42 ms so with 8 lanes; 7.12 and 3.82 ms with 4.
 // G = 0 takes the group size at run time (argument gsz: 2, 4 or 8 lanes of K
 // layers each), so one kernel can give each wavefront the group size its
 // columns' depth needs.
